@@ -308,3 +308,22 @@ def test_nest_without_buffers_reports_division_by_zero(dev):
     status = k({})
     torch.cuda.synchronize()
     assert int(status.item()) == ln.STATUS_DIV0
+
+
+@pytest.mark.parametrize("K", [1, 3, 4, 8, 33])
+def test_int8_products_summed_into_int64_keep_the_high_half(dev, K):
+    M, N = 5, 7
+    rng = np.random.default_rng(K)
+    A = rng.integers(-128, 128, (M, K), dtype=np.int8)
+    B = rng.integers(-128, 128, (K, N), dtype=np.int8)
+    D = rng.integers(-2**62, 2**62, (M, N), dtype=np.int64)
+    k = ln.LoopNestKernel(ln.matmul_stmt(M, K, N), {"A": {"dtype": "int8", "shape": (M, K)},
+                                                    "B": {"dtype": "int8", "shape": (K, N)},
+                                                    "C": {"dtype": "int64", "shape": (M, N)}})
+    t = {"A": torch.from_numpy(A.reshape(-1)).to(dev), "B": torch.from_numpy(B.reshape(-1)).to(dev),
+         "C": torch.from_numpy(D.reshape(-1).copy()).to(dev)}
+    st = k(t)
+    torch.cuda.synchronize()
+    assert int(st.item()) == 0
+    want = D + A.astype(np.int64) @ B.astype(np.int64)
+    assert np.array_equal(t["C"].cpu().numpy().reshape(M, N), want)

@@ -487,6 +487,7 @@ def _walk_notes(stmt, mapped_vars, notes):
 
 class _Emitter:
     guard = None   # cap on each thread's sequential iterations, when counted at run time
+    wide = False   # the store being emitted is 64-bit (vt_rd8)
 
     def __init__(self, buffers, layout):
         self.buffers = buffers
@@ -544,7 +545,8 @@ class _Emitter:
         if kind == "read":
             # a read converts to the context's type; a floating value read
             # in integer context truncates toward zero, as a C cast does
-            return "((%s)vt_rd(%s, %s))" % (ty, e[1], self.guarded(e[1], e[2]))
+            rd = "vt_rd8" if self.wide and self.buf_dtype(e[1]) == "int8" else "vt_rd"
+            return "((%s)%s(%s, %s))" % (ty, rd, e[1], self.guarded(e[1], e[2]))
         left, right = self.expr(e[1], ty), self.expr(e[2], ty)
         if kind in ("div", "mod") and ty == "long long":
             return "vt_%s(%s, %s, vt_status)" % (kind, left, right)
@@ -581,7 +583,9 @@ class _Emitter:
             buf, idx, val = s[1], s[2], s[3]
             ty = self.value_type(buf, val)
             ctype = DTYPES[self.buf_dtype(buf)]
+            self.wide = self.buf_dtype(buf) == "int64"
             value = self.expr(val, ty)
+            self.wide = False
             if self.buf_dtype(buf) == "int32" and ty == "long long":
                 # int32 accumulator: keep the low 32 bits (two's complement wrap)
                 value = "(int)(unsigned int)(unsigned long long)%s" % value
@@ -623,6 +627,9 @@ class _Emitter:
 
 # Device helpers of every emitted kernel: guarded index, guarded read, and
 # integer division / modulo that cannot trap or invoke undefined behaviour.
+# vt_rd8 reads an int8 cell for a 64-bit store without showing the compiler
+# that it has 8 bits: it turns unrolled sums of int8 products into
+# v_dot4_i32_i8, and loses the high half of a 64-bit sum (ROCm 7.2).
 _PRELUDE = r"""__device__ __forceinline__ long long vt_idx(long long i, long long n, int *st) {
   if (i >= 0 && i < n) return i;
   atomicOr(st, 1);
@@ -630,6 +637,11 @@ _PRELUDE = r"""__device__ __forceinline__ long long vt_idx(long long i, long lon
 }
 template <typename T> __device__ __forceinline__ T vt_rd(const T *p, long long i) {
   return i >= 0 ? p[i] : T(0);
+}
+__device__ __forceinline__ int vt_rd8(const signed char *p, long long i) {
+  int v = i >= 0 ? p[i] : 0;
+  asm("" : "+v"(v));
+  return v;
 }
 __device__ __forceinline__ long long vt_div(long long a, long long b, int *st) {
   if (b == 0 || (b == -1 && a == (-9223372036854775807LL - 1))) { atomicOr(st, 2); return 0; }
