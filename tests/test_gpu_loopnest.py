@@ -327,3 +327,63 @@ def test_int8_products_summed_into_int64_keep_the_high_half(dev, K):
     assert int(st.item()) == 0
     want = D + A.astype(np.int64) @ B.astype(np.int64)
     assert np.array_equal(t["C"].cpu().numpy().reshape(M, N), want)
+
+
+# ---------------------------------------------------------------------------
+# Tiled reductions against one thread per cell
+# ---------------------------------------------------------------------------
+
+TYPES = {"int8": ("int8", "int8", "int32"), "int8_wide": ("int8", "int8", "int64"),
+         "int32": ("int32", "int32", "int32"), "float32": ("float32", "float32", "float32"),
+         "float64": ("float64", "float64", "float64")}
+
+
+def _weighted(M, K, N):
+    """C[i,j] = B[k,j] * A[i,k] + C[i,j] + k: the sum on the other side, a loop variable."""
+    return loop("i", M, loop("j", N, loop("k", K, wr("C", [var("i"), var("j")], {
+        "tag": "add", "left": {"tag": "mul", "left": rd("B", var("k"), var("j")),
+                               "right": rd("A", var("i"), var("k"))},
+        "right": {"tag": "add", "left": rd("C", var("i"), var("j")), "right": var("k")}}))))
+
+
+TILED_NESTS = dict(NESTS, weighted=_weighted,
+                   # two sequential loops, flattened in order
+                   split_k=lambda M, K, N: tile(ln.matmul_stmt(M, K, N), "i2", K // 3),
+                   # an outer mapped loop besides the rows and the lanes
+                   row_tiles=lambda M, K, N: tile(ln.matmul_stmt(M, K, N), "i0", M // 2))
+
+
+@pytest.mark.parametrize("types", sorted(TYPES))
+@pytest.mark.parametrize("nest,shape,layout", [
+    ("naive", (64, 3, 64), "dense"), ("k_outer", (130, 33, 33), "reference"),
+    ("weighted", (70, 96, 127), "dense"), ("split_k", (68, 129, 64), "reference"),
+    ("row_tiles", (66, 71, 65), "dense"), ("naive", (260, 64, 100), "reference")])
+def test_tiled_reductions_equal_one_thread_per_cell(dev, monkeypatch, shape, nest, types, layout):
+    """The same nest lowered both ways: every cell bit for bit the same (each
+    cell's steps run in the same order, so floating sums round alike), padding
+    cells untouched, no status bit."""
+    M, K, N = shape
+    say("tiled", shape, nest, types, layout)
+    stmt = TILED_NESTS[nest](M, K, N)
+    decl = {b: {"dtype": t, "shape": s}
+            for b, t, s in zip("ABC", TYPES[types], ((M, K), (K, N), (M, N)))}
+    rng = np.random.default_rng(M * K + N)
+    data = {}
+    for b, d in decl.items():
+        n = ln._max_index(d["shape"], layout) + 1
+        if d["dtype"].startswith("float"):
+            data[b] = rng.standard_normal(n).astype(d["dtype"])
+        else:
+            info = np.iinfo(d["dtype"])
+            data[b] = rng.integers(info.min, info.max, n, dtype=d["dtype"], endpoint=True)
+    got = {}
+    for cells in (1, 1 << 62):
+        monkeypatch.setattr(ln, "TILED_MIN_CELLS", cells)
+        k = ln.LoopNestKernel(stmt, decl, layout=layout)
+        assert ("vt_tile" in k.source) == (cells == 1)
+        t = {b: torch.from_numpy(v.copy()).to(dev) for b, v in data.items()}
+        status = k(t)
+        torch.cuda.synchronize()
+        assert int(status.item()) == 0
+        got[cells] = t["C"].cpu().numpy()
+    assert np.array_equal(got[1], got[1 << 62])

@@ -37,6 +37,10 @@ Lowering, MI355X first
     reported as suppressed (the reference writes the same "suppressed"
     comment instead of a pragma); `unrolled` adds `#pragma unroll` to a
     sequential loop.
+  * Reductions. A nest that sums products over its sequential loops, with
+    constant bounds and indices proven in range, runs on LDS tiles
+    (plan_tiled): a workgroup reads each operand once for a block of cells
+    and keeps the cells in registers, each summed in program order.
   * Layouts. "reference": every buffer is flat with the reference's
     stride-1000 index, i0*1000^(d-1) + ... + i_{d-1} (emit_c.py:29-44), so
     buffers laid out for the reference's emitted C work unchanged. "dense":
@@ -51,10 +55,10 @@ Lowering, MI355X first
     throughout, which is layout "reference" with float64 buffers.
 
 Memory safety. An emitted kernel never touches memory outside the declared
-buffers, whatever the nest computes: every access checks its flat index
-against the buffer's declared size (the host checks each tensor holds at
-least that many elements) and integer division or modulo by zero yields 0;
-either event sets a bit in a status word (STATUS_RANGE, STATUS_DIV0) that
+buffers, whatever the nest computes: every access not proven in range when
+the kernel is emitted checks its flat index against the buffer's declared
+size (the host checks each tensor holds at least that many elements) and
+integer division or modulo by zero yields 0; either event sets a bit in a status word (STATUS_RANGE, STATUS_DIV0) that
 the call returns, and the offending store is skipped or read is 0.
 
 Bounded work. Each GPU thread runs at most MAX_THREAD_ITERATIONS iterations
@@ -706,6 +710,445 @@ def _used(stmt):
     return {buf for buf, _, _ in _accesses(stmt, frozenset(), [])}
 
 
+# ---------------------------------------------------------------------------
+# Tiled lowering of reductions
+# ---------------------------------------------------------------------------
+
+# Rows per wave: the first of TILE_ROWS that gives TILE_WORKGROUPS workgroups
+# (165 x 452 x 94 float64: 88 workgroups of 4 rows a wave 7.9 us, 336 of 1 row
+# 10.2; 129 x 84 x 143: 66 of 1 row 7.1, 18 of 4 rows 10.3). Smaller nests than
+# TILED_MIN_CELLS cells keep one thread per cell.
+WAVE = 64
+TILE_ROWS = (4, 2, 1)
+TILE_WORKGROUPS = 64
+TILED_MIN_CELLS = 4096
+TILE_LDS = 60 * 1024       # most LDS of a workgroup (both buffers)
+GROUP = 4                  # steps whose operands leave LDS together
+_SIZES = {"int8": 1, "int32": 4, "int64": 8, "float32": 4, "float64": 8}
+
+
+def _reads(e, out):
+    """The read nodes of a value (those inside indices excluded)."""
+    if e[0] == "read":
+        out.append(e)
+    elif e[0] in _BINOPS:
+        _reads(e[1], out)
+        _reads(e[2], out)
+    return out
+
+
+def plan_tiled(stmt, mapped, buffers, layout):
+    """How a reduction nest runs on LDS tiles, or None when it keeps the
+    general lowering.
+
+    Taken: a perfect nest of constant bounds around one store W[x] = value
+    where every read of W is W[x], x is free of the sequential loops (so a
+    cell's running value stays in a register), every index is affine and
+    proven inside its buffer over the whole nest (so no access needs its
+    guard), there is no integer division or modulo, and of the mapped loops
+    the innermost, whose points become the lanes of a wave, has a read that
+    changes with it and the steps but not with another one, the rows, so that
+    a workgroup reads it once for all its rows.
+
+    Mapped iterations touch disjoint cells (threads_disjoint), so several may
+    run in one thread, step by step; each cell meets its own steps in program
+    order, so floating sums round as in the sequential nest.
+    """
+    ranges = _var_ranges(stmt, {})
+    node, loops = stmt, []
+    while node[0] == "loop":
+        lo, hi = _const(node[2]), _const(node[3])
+        if lo is None or hi is None or hi <= lo:
+            return None
+        loops.append((node[1], lo, hi - lo))
+        node = node[5]
+    if node[0] != "write" or len(mapped) < 2:
+        return None
+    buf, idx, value = node[1], node[2], node[3]
+    names = {m[0] for m in mapped}
+    seq = [v for v in loops if v[0] not in names]
+    cells, steps = _prod(m[2] for m in mapped), _prod(v[2] for v in seq)
+    if not seq or not TILED_MIN_CELLS <= cells < 2**31 or steps >= 2**30:
+        return None
+    if max(abs(lo) + ext for _, lo, ext in loops) >= 2**30:
+        return None
+    floating = any(buffers[b]["dtype"] in FLOAT_DTYPES
+                   for b in {buf} | {r[1] for r in _reads(value, [])})
+
+    def plain(e):
+        if e[0] in ("lit", "var", "read"):
+            return True
+        return (floating or e[0] in ("add", "mul")) and plain(e[1]) and plain(e[2])
+
+    if not plain(value):
+        return None
+    out, forms = (buf, idx), {}
+    for b, ix in [out] + [(r[1], r[2]) for r in _reads(value, [])]:
+        if b == buf and ix != idx:
+            return None
+        form = _flat_form(b, ix, buffers, layout)
+        span = None if form is None else _interval(form, ranges)
+        if (span is None or span[0] < 0
+                or span[1] > _max_index(tuple(buffers[b]["shape"]), layout)):
+            return None
+        # every partial sum of the index stays in 32 bits
+        if sum(abs(c) * (1 if v is None else max(map(abs, ranges[v])))
+               for v, c in form.items()) >= 2**31:
+            return None
+        forms[(b, ix)] = form
+    if any(forms[out].get(v[0], 0) for v in seq):
+        return None
+    lane = mapped[-1]
+    chunks = -(-lane[2] // WAVE)
+    if 2 * lane[2] < chunks * WAVE:      # more than half of the lanes idle
+        return None
+
+    def uses(key, loops):
+        return any(forms[key].get(v[0], 0) for v in loops)
+
+    reads = [key for key in forms if key != out]
+    stepped = [key for key in reads if uses(key, seq)]
+    rows = [m for m in mapped[:-1] if m[2] >= 4
+            and any(uses(key, [lane]) and not uses(key, [m]) for key in stepped)]
+    if not rows:
+        return None
+    row = max(rows, key=lambda m: m[2])
+    others = [m for m in mapped[:-1] if m is not row]
+    # Staged in LDS: per lane (shared by the rows), or per row (shared by the
+    # lanes). The rest is read where it is used.
+    by_lane = [k for k in stepped if uses(k, [lane]) and not uses(k, [row])]
+    by_row = [k for k in stepped if uses(k, [row]) and not uses(k, [lane])]
+
+    bytes_read = [k for k in reads if buffers[k[0]]["dtype"] == "int8"]
+    if any(k not in by_lane + by_row for k in bytes_read):
+        return None      # see size
+    # An int8 product into an int32 sum runs on four-element dot products.
+    dot = None
+    if (not floating and buffers[buf]["dtype"] == "int32" and value[0] == "add"
+            and len(by_lane) == len(by_row) == 1 and len(bytes_read) == len(reads) == 2):
+        for acc, prod in ((value[1], value[2]), (value[2], value[1])):
+            if (acc == ("read",) + out and prod[0] == "mul"
+                    and {prod[1], prod[2]} == {("read",) + k for k in reads}):
+                dot = (by_lane[0], by_row[0])
+
+    def size(key):
+        """Bytes of a staged cell. int8 outside the dot products is staged as
+        int32: the compiler turns unrolled sums of int8 products into
+        v_dot4_i32_i8 by itself, also into 64-bit sums, whose high half it
+        then loses (ROCm 7.2)."""
+        return max(_SIZES[buffers[key[0]]["dtype"]], 1 if dot else 4)
+
+    for per_wave in TILE_ROWS:
+        groups = -(-row[2] // (per_wave * (BLOCK // WAVE)))
+        workgroups = groups * chunks * _prod(m[2] for m in others)
+        if workgroups >= TILE_WORKGROUPS:
+            break
+    span = per_wave * (BLOCK // WAVE)
+    batch = 64 if dot else 32
+    while batch > 8 and 2 * (sum(size(k) * WAVE * (batch + 4) for k in by_lane)
+                             + sum(size(k) * span * batch for k in by_row)) > TILE_LDS:
+        batch //= 2
+    if workgroups >= 2**31 or 2 * (sum(size(k) * WAVE * (batch + 4) for k in by_lane)
+                                   + sum(size(k) * span * batch for k in by_row)) > TILE_LDS:
+        return None
+    return {"out": out, "value": value, "forms": forms, "seq": seq, "steps": steps, "lane": lane,
+            "row": row, "others": others, "per_wave": per_wave, "groups": groups,
+            "chunks": chunks, "workgroups": workgroups, "batch": batch, "by_lane": by_lane,
+            "by_row": by_row, "dot": dot, "floating": floating,
+            "staged_type": {k: "int" if not dot and k in bytes_read
+                            else DTYPES[buffers[k[0]]["dtype"]] for k in by_lane + by_row}}
+
+
+class _Tiled:
+    """Emission of a tiled reduction: one workgroup owns per_wave * 4 rows by
+    64 lanes of cells, one lane a column, each wave per_wave rows. The
+    sequential loops run flattened, in order, `batch` steps at a time: the
+    workgroup loads the next batch of each staged read into registers, runs
+    this batch from LDS, and stores the loaded one into the other buffer.
+
+    One thread per cell, with its guards, was bound by its memory accesses: a
+    guarded load of each operand and a load and a store of the cell per step.
+    Here a float64 step is 2 * per_wave multiplies and adds, and what bounds a
+    500^3 nest is their issue (8.9 cycles each with one wave per SIMD, 5 with
+    four) plus about a quarter of the cycles in waits. MI355X, HIP graph per
+    launch with the status word's clear, one thread per cell against this
+    lowering: float64 500^3 120 -> 30 us, 640^3 267 -> 53, 129 x 84 x 143 31 ->
+    7.1; int8 into int32 (dot products) 500^3 84 -> 10, 640^3 140 -> 17, 299 x
+    177 x 184 31 -> 5.2. Unrolling a whole batch gave 26 us at 500^3 for 40 ms more of
+    compilation.
+    """
+
+    def __init__(self, plan, buffers, lines):
+        self.p, self.buffers, self.w = plan, buffers, lines.append
+        self.rows = plan["per_wave"]
+        self.span = self.rows * (BLOCK // WAVE)      # rows of the workgroup
+        self.ty = "double" if plan["floating"] else "long long"
+
+    def ctype(self, key):
+        return DTYPES[self.buffers[key[0]]["dtype"]]
+
+    def staged(self, key):
+        return self.p["staged_type"][key]
+
+    def pitch(self, key):
+        """Cells per lane of a per-lane tile: an odd number of its LDS words,
+        so the lanes' reads of one step fall on distinct banks."""
+        return self.p["batch"] + (4 if self.staged(key) == "signed char" else 1)
+
+    def flat(self, key, names, env):
+        """Text of the key's index terms over `names`, variables as in env."""
+        form = self.p["forms"][key]
+        terms = ["%d * (%s)" % (form[v], env.get(v, v)) for v in names if form.get(v, 0)]
+        return " + ".join(terms) or "0"
+
+    def step_env(self, step):
+        """Values of the sequential loop variables at flattened step `step`."""
+        env, inner = {}, 1
+        for n, (v, lo, ext) in enumerate(reversed(self.p["seq"])):
+            digit = "(%s)" % step if inner == 1 else "(%s) / %d" % (step, inner)
+            if n + 1 < len(self.p["seq"]):
+                digit = "(%s) %% %d" % (digit, ext)
+            env[v], inner = "%d + %s" % (lo, digit), inner * ext
+        return env
+
+    def seq_names(self):
+        return [v[0] for v in self.p["seq"]]
+
+    def load(self, pad, key, n, first):
+        """Registers vt_g<n>[..] = the batch of `key` from step `first` on;
+        steps past the last one repeat it (they are never used)."""
+        p, batch = self.p, self.p["batch"]
+        lanes = key in p["by_lane"]
+        count = batch * (WAVE if lanes else self.span)
+        last = p["steps"] - 1
+        for i in range(-(-count // BLOCK)):
+            at = "(vt_t + %d)" % (i * BLOCK)
+            step = "%s + %s %s %d" % ((first, at) + (("/", WAVE) if lanes else ("%", batch)))
+            self.w("%s{ const int vt_s = %s < %d ? %s : %d;" % (pad, step, last, step, last))
+            if lanes:
+                self.w("%s  vt_g%d[%d] = vt_src%d[%s]; }"
+                       % (pad, n, i, n, self.flat(key, self.seq_names(), self.step_env("vt_s"))))
+            else:
+                row = p["row"]
+                at_row = "vt_row0 + %s / %d" % (at, batch)
+                env = self.step_env("vt_s")
+                env[row[0]] = "%d + (%s < %d ? %s : %d)" % (row[1], at_row, row[2], at_row, row[2] - 1)
+                self.w("%s  vt_g%d[%d] = vt_src%d[%s]; }"
+                       % (pad, n, i, n, self.flat(key, self.seq_names() + [row[0]], env)))
+
+    def store(self, pad, key, n, to):
+        p, batch = self.p, self.p["batch"]
+        lanes = key in p["by_lane"]
+        count = batch * (WAVE if lanes else self.span)
+        for i in range(-(-count // BLOCK)):
+            at = "(vt_t + %d)" % (i * BLOCK)
+            cell = ("%s %% %d * %d + %s / %d" % (at, WAVE, self.pitch(key), at, WAVE) if lanes else at)
+            guard = "" if (i + 1) * BLOCK <= count else "if (%s < %d) " % (at, count)
+            self.w("%s%svt_tile%d[%s][%s] = vt_g%d[%d];" % (pad, guard, n, to, cell, n, i))
+
+    def value(self, e, r, u, step):
+        """Text of value `e` for the wave's row r; u: where the staged reads'
+        registers hold the step."""
+        p, kind = self.p, e[0]
+        if kind == "lit":
+            return ("%d.0" % e[1]) if p["floating"] else ("%dLL" % e[1])
+        if kind == "var":
+            env = self.step_env(step)
+            env[p["row"][0]] = "vt_r%d" % r
+            return "((%s)(%s))" % (self.ty, env.get(e[1], e[1]))
+        if kind == "read":
+            key = (e[1], e[2])
+            if key == p["out"]:
+                return "((%s)vt_acc%d)" % (self.ty, r)
+            if key in self.index:
+                return "((%s)vt_x%d_%d_%d[%d])" % ((self.ty, self.index[key],
+                                                    0 if key in p["by_lane"] else r) + u)
+            env = self.step_env(step)
+            env[p["row"][0]] = "vt_r%d" % r
+            form = p["forms"][key]
+            names = self.seq_names() + self.points()
+            return "((%s)%s[%d + %s])" % (self.ty, key[0], form.get(None, 0),
+                                          self.flat(key, names, env))
+        left, right = self.value(e[1], r, u, step), self.value(e[2], r, u, step)
+        if kind == "mod":
+            return "fmod(%s, %s)" % (left, right)
+        return "(%s %s %s)" % (left, _BINOPS[kind], right)
+
+    def points(self):
+        return [self.p["row"][0], self.p["lane"][0]] + [m[0] for m in self.p["others"]]
+
+    def term(self):
+        """The X of a value W + X or X + W that does not read W, else None."""
+        value, acc = self.p["value"], ("read",) + self.p["out"]
+        if value[0] != "add" or acc not in value[1:]:
+            return None
+        term = value[2] if value[1] == acc else value[1]
+        return None if acc in _reads(term, []) else term
+
+    def compute(self, pad, count, first):
+        """Run `count` steps of the buffer vt_b, whose first one is `first`."""
+        p = self.p
+        if p["dot"]:
+            # four steps per instruction; steps past the last one multiply the
+            # zeros of zero_tail
+            a, b = (self.index[k] for k in p["dot"])
+            self.w("%s#pragma unroll" % pad)
+            self.w("%sfor (int vt_u = 0; vt_u < %d; vt_u += 4) {" % (pad, -(-count // 4) * 4))
+            self.w("%s  const int vt_x = *(const int *)&vt_tile%d[vt_b][vt_lane * %d + vt_u];"
+                   % (pad, a, self.pitch(p["dot"][0])))
+            for r in range(self.rows):
+                self.w("%s  vt_acc%d = __builtin_amdgcn_sdot4(vt_x, *(const int *)&vt_tile%d[vt_b]"
+                       "[(vt_wave * %d + %d) * %d + vt_u], vt_acc%d, false);"
+                       % (pad, r, b, self.rows, r, p["batch"], r))
+            self.w(pad + "}")
+            return
+        # Operands come out of LDS a group of steps ahead of their use: left to
+        # itself the compiler waits for each step's reads right before it (one
+        # or two waves a SIMD do not hide that). Two groups an iteration, one
+        # per register set.
+        pair = 2 * GROUP
+        main = count // pair * pair
+        self.w(pad + "{")
+        pad += "  "
+        for key, n in self.index.items():
+            for r in range(1 if key in p["by_lane"] else self.rows):
+                for side in (0, 1):
+                    self.w("%s%s vt_x%d_%d_%d[%d];" % (pad, self.staged(key), n, r, side, GROUP))
+        if main:
+            self.fetch(pad, "0", GROUP, 0)
+            self.w(pad + "#pragma unroll 1")
+            self.w("%sfor (int vt_u = 0; vt_u < %d; vt_u += %d) {" % (pad, main, pair))
+            self.fetch(pad + "  ", "vt_u + %d" % GROUP, GROUP, 1)
+            self.steps(pad + "  ", first + " + vt_u", GROUP, 0)
+            self.w("%s  const int vt_v = vt_u + %d < %d ? vt_u + %d : 0;" % (pad, pair, main, pair))
+            self.fetch(pad + "  ", "vt_v", GROUP, 0)
+            self.steps(pad + "  ", "%s + vt_u + %d" % (first, GROUP), GROUP, 1)
+            self.w(pad + "}")
+        for at in range(main, count, GROUP):
+            size = min(GROUP, count - at)
+            self.fetch(pad, "%d" % at, size, 0)
+            self.steps(pad, "%s + %d" % (first, at), size, 0)
+        self.w(pad[:-2] + "}")
+
+    def fetch(self, pad, at, size, side):
+        """Registers of one side = the staged operands of `size` steps from
+        step `at` of the buffer vt_b."""
+        for key, n in self.index.items():
+            lanes = key in self.p["by_lane"]
+            for r in range(1 if lanes else self.rows):
+                base = ("vt_lane * %d" % self.pitch(key) if lanes else
+                        "(vt_wave * %d + %d) * %d" % (self.rows, r, self.p["batch"]))
+                for u in range(size):
+                    self.w("%svt_x%d_%d_%d[%d] = vt_tile%d[vt_b][%s + %s + %d];"
+                           % (pad, n, r, side, u, n, base, at, u))
+        self.w(pad + "__builtin_amdgcn_sched_barrier(0);")
+
+    def steps(self, pad, first, size, side):
+        """`size` steps from flattened step `first` on, out of one side's registers."""
+        p, out = self.p, self.ctype(self.p["out"])
+        here = [(u, r) for u in range(size) for r in range(self.rows)]
+        term = self.term()
+        if term is not None:
+            # every term of the group before the first sum: a sum right behind
+            # its own term waits for it
+            self.w(pad + "{")
+            for u, r in here:
+                self.w("%s%s vt_m%d_%d = %s;" % (pad, self.ty, u, r, self.value(
+                    term, r, (side, u), "%s + %d" % (first, u))))
+            self.w(pad + "__builtin_amdgcn_sched_barrier(0);")
+        for u, r in here:
+            if term is not None:
+                acc, new = "((%s)vt_acc%d)" % (self.ty, r), "vt_m%d_%d" % (u, r)
+                v = "(%s + %s)" % ((new, acc) if p["value"][1] == term else (acc, new))
+            else:
+                v = self.value(p["value"], r, (side, u), "%s + %d" % (first, u))
+            if out == "int" and not p["floating"]:
+                v = "(int)(unsigned int)(unsigned long long)%s" % v
+            else:
+                v = "(%s)%s" % (out, v)
+            self.w("%svt_acc%d = %s;" % (pad, r, v))
+        if term is not None:
+            self.w(pad + "}")
+        self.w(pad + "__builtin_amdgcn_sched_barrier(0);")
+
+    def emit(self):
+        p, w = self.p, self.w
+        lane, row, batch = p["lane"], p["row"], p["batch"]
+        staged = p["by_lane"] + p["by_row"]
+        self.index = {key: n for n, key in enumerate(staged)}
+        for key, n in self.index.items():
+            cells = WAVE * self.pitch(key) if key in p["by_lane"] else self.span * batch
+            w("  __shared__ __attribute__((aligned(16))) %s vt_tile%d[2][%d];"
+              % (self.staged(key), n, cells))
+        w("  const int vt_t = (int)threadIdx.x, vt_lane = vt_t %% %d;" % WAVE)
+        w("  const int vt_wave = __builtin_amdgcn_readfirstlane(vt_t / %d);" % WAVE)
+        w("  int vt_rest = (int)blockIdx.x;")
+        w("  const int vt_row0 = vt_rest %% %d * %d;" % (p["groups"], self.span))
+        w("  vt_rest /= %d;" % p["groups"])
+        w("  const int vt_at = vt_rest %% %d * %d + vt_lane;" % (p["chunks"], WAVE))
+        w("  const bool vt_live = vt_at < %d;" % lane[2])
+        # lanes and rows past the end repeat the last one and store nothing
+        w("  const int %s = %d + (vt_live ? vt_at : %d);" % (lane[0], lane[1], lane[2] - 1))
+        w("  vt_rest /= %d;" % p["chunks"])
+        for v, lo, ext in reversed(p["others"]):
+            w("  const int %s = %d + vt_rest %% %d;" % (v, lo, ext))
+            w("  vt_rest /= %d;" % ext)
+        for r in range(self.rows):
+            w("  const int vt_at%d = vt_row0 + vt_wave * %d + %d;" % (r, self.rows, r))
+            w("  const int vt_r%d = %d + (vt_at%d < %d ? vt_at%d : %d);"
+              % (r, row[1], r, row[2], r, row[2] - 1))
+        out = p["out"]
+        for r in range(self.rows):
+            w("  %s *const vt_out%d = %s + (%d + %s);"
+              % (self.ctype(out), r, out[0], p["forms"][out].get(None, 0),
+                 self.flat(out, self.points(), {row[0]: "vt_r%d" % r})))
+            w("  %s vt_acc%d = *vt_out%d;" % (self.ctype(out), r, r))
+        for key, n in self.index.items():
+            names = [v for v in self.points() if v != row[0]]
+            w("  const %s *const vt_src%d = %s + (%d + %s);"
+              % (self.ctype(key), n, key[0], p["forms"][key].get(None, 0),
+                 self.flat(key, names, {})))
+            count = batch * (WAVE if key in p["by_lane"] else self.span)
+            w("  %s vt_g%d[%d];" % (self.staged(key), n, -(-count // BLOCK)))
+        steps, main = p["steps"], p["steps"] // batch
+        left = steps - main * batch
+        for key, n in self.index.items():
+            self.load("  ", key, n, "0")
+        for key, n in self.index.items():
+            if p["dot"] and not main:
+                self.zero_tail("  ", key, n, "0")
+            self.store("  ", key, n, "0")
+        w("  __syncthreads();")
+        w("  int vt_b = 0;")
+        if main:
+            w("  for (int vt_first = 0; vt_first < %d; vt_first += %d) {" % (main * batch, batch))
+            # (after the last whole batch the loads repeat the last step)
+            for key, n in self.index.items():
+                self.load("    ", key, n, "vt_first + %d" % batch)
+            w("    __builtin_amdgcn_sched_barrier(0);")
+            self.compute("    ", batch, "vt_first")
+            for key, n in self.index.items():
+                if p["dot"] and left:
+                    self.zero_tail("    ", key, n, "vt_first + %d" % batch)
+                self.store("    ", key, n, "vt_b ^ 1")
+            w("    __syncthreads();")
+            w("    vt_b ^= 1;")
+            w("  }")
+        if left:
+            self.compute("  ", left, "%d" % (main * batch))
+        for r in range(self.rows):
+            w("  if (vt_live && vt_at%d < %d) *vt_out%d = vt_acc%d;" % (r, row[2], r, r))
+
+    def zero_tail(self, pad, key, n, first):
+        """Steps past the last one of a per-row tile read as zero."""
+        p, batch = self.p, self.p["batch"]
+        if key not in p["by_row"]:
+            return
+        for i in range(-(-batch * self.span // BLOCK)):
+            self.w("%sif (%s + (vt_t + %d) %% %d >= %d) vt_g%d[%d] = 0;"
+                   % (pad, first, i * BLOCK, batch, p["steps"], n, i))
+
+
 def emit_kernel(stmt, buffers, name="loopnest", layout="dense",
                 max_iterations=MAX_THREAD_ITERATIONS):
     """Lower a parsed (or JSON) loop nest to a HIP kernel.
@@ -759,36 +1202,42 @@ def emit_kernel(stmt, buffers, name="loopnest", layout="dense",
                                                DTYPES[buffers[b]["dtype"]], b) for b in params]
                     + ["int *__restrict__ vt_status"])
     em.lines.append('extern "C" __global__ __launch_bounds__(%d) void %s(%s) {' % (BLOCK, name, sig))
-    em.lines.append("  const long long vt_t = (long long)blockIdx.x * %d + threadIdx.x;" % BLOCK)
-    em.lines.append("  if (vt_t >= %dLL) return;" % total)
-    if em.guard is not None:
-        em.lines.append("  unsigned long long vt_iters = 0;")
-    if mapped:
-        em.lines.append("  long long vt_rest = vt_t;")
-        for var, lo, ext in reversed(mapped):
-            # an empty mapped loop makes total 0 and this unreachable; the
-            # divisor stays nonzero all the same
-            em.lines.append("  const long long %s = %dLL + vt_rest %% %dLL;" % (var, lo, max(ext, 1)))
-            em.lines.append("  vt_rest /= %dLL;" % max(ext, 1))
-    # sequential loops of the chain, then the innermost body
-    depth = 1
-    for loop in seq_chain:
-        var, lo, hi, ann = loop[1], loop[2], loop[3], loop[4]
-        pad = "  " * depth
-        if ann == "unrolled":
-            em.lines.append(pad + "#pragma unroll")
-        em.lines.append("%sfor (long long %s = %s; %s < %s; ++%s) {"
-                        % (pad, var, em.expr_int(lo), var, em.expr_int(hi), var))
-        depth += 1
-        em.count_iteration(depth)
-    em.stmt(inner, depth)
-    for d in range(depth - 1, 0, -1):
-        em.lines.append("  " * d + "}")
-    em.lines.append("}")
+    tiled = plan_tiled(stmt, mapped, buffers, layout)
+    if tiled is not None:
+        _Tiled(tiled, buffers, em.lines).emit()
+        em.lines.append("}")
+        blocks = tiled["workgroups"]
+    else:
+        em.lines.append("  const long long vt_t = (long long)blockIdx.x * %d + threadIdx.x;" % BLOCK)
+        em.lines.append("  if (vt_t >= %dLL) return;" % total)
+        if em.guard is not None:
+            em.lines.append("  unsigned long long vt_iters = 0;")
+        if mapped:
+            em.lines.append("  long long vt_rest = vt_t;")
+            for var, lo, ext in reversed(mapped):
+                # an empty mapped loop makes total 0 and this unreachable; the
+                # divisor stays nonzero all the same
+                em.lines.append("  const long long %s = %dLL + vt_rest %% %dLL;" % (var, lo, max(ext, 1)))
+                em.lines.append("  vt_rest /= %dLL;" % max(ext, 1))
+        # sequential loops of the chain, then the innermost body
+        depth = 1
+        for loop in seq_chain:
+            var, lo, hi, ann = loop[1], loop[2], loop[3], loop[4]
+            pad = "  " * depth
+            if ann == "unrolled":
+                em.lines.append(pad + "#pragma unroll")
+            em.lines.append("%sfor (long long %s = %s; %s < %s; ++%s) {"
+                            % (pad, var, em.expr_int(lo), var, em.expr_int(hi), var))
+            depth += 1
+            em.count_iteration(depth)
+        em.stmt(inner, depth)
+        for d in range(depth - 1, 0, -1):
+            em.lines.append("  " * d + "}")
+        em.lines.append("}")
+        blocks = max(1, -(-total // BLOCK))
     header = ["// Emitted by veritac_amd.specializations.hip_gemm.loopnest (layout %s)." % layout]
     header += ["// %s" % n for n in notes]
     header += [_PRELUDE]
-    blocks = max(1, -(-total // BLOCK))
     if blocks > 2**31 - 1:
         raise LoopNestError("%d mapped iterations exceed the launch limit" % total)
     return {"source": "\n".join(header + em.lines) + "\n", "kernel": name, "params": params,
