@@ -78,7 +78,8 @@ def test_reference_side_descriptor_passes_the_reference_path_rule(tmp_path):
                            for p in shipped)
 
 
-@pytest.mark.skipif(not os.path.isdir(REFERENCE), reason="no reference checkout here")
+@pytest.mark.skipif(not (os.path.isdir(REFERENCE) and os.listdir(REFERENCE)),
+                    reason="no reference checkout here")
 def test_reference_side_paths_exist_in_the_reference_checkout():
     """The descriptor's paths outside specializations/hip_gemm/ are the
     reference's own files (Lean contract, recorded results)."""
