@@ -393,9 +393,12 @@ int vt_pack_b_i8(const int8_t *B, int8_t *Bp, int64_t K, int64_t N, int64_t ldb,
  *     groups of four 16-column blocks when N gives 192 or more of them, else
  *     smaller groups, about one per CU.
  * k_split: workgroups along K for the groups of up to 64 rows (0 =
- * automatic: 1 unless even half-block groups are too few, else a split whose
- * partial sums are finished in the kernel up to 16 rows, through the
- * finishing words described under Workspace, or added by a second kernel);
+ * automatic: a split when even half-block groups are too few, or when narrow
+ * groups over a long K would read A for longer than a split of two or four
+ * over wider groups takes to sum (not needed: such a call runs unsplit when
+ * its stream is captured before it has a workspace). The partial sums are
+ * finished in the kernel up to 16 rows, through the finishing words described
+ * under Workspace, or added by a second kernel);
  * the tile kernels choose their own.
  */
 int vt_gemm_i8_packed(const int8_t *A, const int8_t *Bp, const int32_t *D, int32_t *C,

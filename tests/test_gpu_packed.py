@@ -511,3 +511,52 @@ def test_packed_b_on_the_256x128_form_batches(dev, shared):
     C = hg.run(plan, to_dev(dev, A), hg.pack_b(to_dev(dev, B)), to_dev(dev, D)).cpu().numpy()
     for b in range(batch):
         assert np.array_equal(C[b], go.gemm_i8(A[b], B if shared else B[b], D[b])), b
+
+
+# m, n, k -> (half blocks per group, K slices): one to four column blocks per
+# wave, one to four row blocks, row counts off the blocks, per-wave steps below,
+# at and past the stages loaded ahead, K tails; K split to read less of A.
+PACKED_STAGES = [
+    (1, 3120, 64, 2, 1), (7, 3200, 1616, 2, 1), (33, 4096, 4144, 2, 1),       # one block, 4 stages
+    (16, 8192, 1536, 4, 1), (49, 8192, 3648, 4, 1),                          # two blocks, 3 stages
+    (30, 10000, 1040, 5, 1), (64, 12224, 2064, 6, 1),                        # three blocks
+    (48, 14336, 1552, 8, 1),                                                 # four blocks
+    (16, 4096, 12288, 8, 4), (15, 4096, 12304, 8, 4), (40, 4096, 12352, 8, 4), (64, 2048, 8192, 4, 4),
+]
+
+
+@pytest.mark.parametrize("m,n,k,hpw,ks", PACKED_STAGES)
+def test_packed_stages_and_splits(dev, m, n, k, hpw, ks):
+    plan = hg.make_plan(m, n, k, variant=hg.PACKED_VARIANT)
+    assert (hg.packed_columns(plan)[0], hg.packed_split(plan)[0]) == (hpw, ks)
+    say("packed stages", m, n, k)
+    rng = np.random.default_rng(m + n + k)
+    A = rng.integers(-128, 128, (m, k), dtype=np.int8)
+    B = rng.integers(-128, 128, (k, n), dtype=np.int8)
+    D = rng.integers(-2**31, 2**31, (m, n), dtype=np.int32)
+    assert np.array_equal(gpu_gemm_packed(dev, A, B), go.gemm_i8(A, B, None))
+    assert np.array_equal(gpu_gemm_packed(dev, A, B, D, in_place=True), go.gemm_i8(A, B, D))
+
+
+def test_packed_split_needs_no_workspace_under_capture(dev):
+    """A split that only saves reads of A runs unsplit on a stream that is
+    captured before it ever had a workspace, as such calls did before."""
+    m, n, k = 16, 4096, 14336
+    plan = hg.make_plan(m, n, k, variant=hg.PACKED_VARIANT)
+    assert hg.packed_split(plan)[0] == 4
+    rng = np.random.default_rng(5)
+    A = rng.integers(-128, 128, (m, k), dtype=np.int8)
+    B = rng.integers(-128, 128, (k, n), dtype=np.int8)
+    At, Bp = to_dev(dev, A), hg.pack_b(to_dev(dev, B))
+    out = torch.full((m, n), INT32_MIN, dtype=torch.int32, device=dev)
+    torch.cuda.synchronize()
+    say("packed split under a cold capture")
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(graph, stream=stream):
+        hg.run(plan, At, Bp, out=out)
+    want = go.gemm_i8(A, B)
+    for _ in range(3):
+        out.fill_(INT32_MIN)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(out.cpu().numpy(), want)

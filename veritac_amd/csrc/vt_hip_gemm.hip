@@ -1771,20 +1771,25 @@ struct PackedArgs {
 // feeds MB MFMAs, so B is streamed once for all of them.
 // One workgroup = WAVES waves over one column group and one K slice.
 // A column group is hpw consecutive 8-column half blocks, so it touches at
-// most NBW 16-column blocks; tiles past its last block are dead and store
-// nothing. Whole groups (hpw = 2 * NBW, MASKED false) load every tile, a dead
-// tile of the last group re-reading the last block. Smaller groups (MASKED)
-// load only live columns: dead tiles load nothing, and with hpw odd the first
-// or last block may be live in one half only, whose other half's lanes
-// neither load B (a packed tile's half is whole 128-byte lines) nor store C.
-// Small groups let a small N spread over every CU without splitting K.
+// most NBW = ceil(hpw / 2) 16-column blocks; with hpw odd the first or last
+// block may be live in one half only. Small groups let a small N spread over
+// every CU without splitting K. Lanes of a dead half read the live half's
+// bytes, and tiles past the group's last block re-read it (lines the wave
+// fetches anyway); their columns are not stored.
 // Wave w takes the 64-row blocks kb_beg + w, kb_beg + w + WAVES, ...;
-// per block it loads its MB A fragments (16 bytes per lane, rows past M and k
-// past K zero) and the NBW packed B tiles, S blocks ahead of the MFMAs
-// (non-temporal loads: B is streamed once). The WAVES partial sums of each
-// column block are added through LDS, one row block at a time, and written
-// once (plus D), or go to the workspace when K is split across workgroups.
-template <int NBW, int WAVES, int S, int MB, bool HAS_D, bool MASKED, bool FIN = false>
+// per block it loads its MB A fragments (16 bytes per lane) and the NBW packed
+// B tiles, S blocks ahead of the MFMAs (non-temporal loads: B is streamed
+// once). Every load is unconditional: rows past M read row M - 1 (their
+// outputs are not stored), k past K reads the row's last 16 bytes (packed B is
+// zero there), and blocks past the wave's last one repeat it. A branch around
+// the loads made the compiler wait for all of them at every step.
+// S: what bounds the kernel is the bytes in flight, NBW * S KB per wave. With
+// the two stages that four tiles need, one tile per wave left 16 KB in flight
+// per CU: M = 1, N = 4096, K = 14336 17.0 us, with four stages 10.4.
+// The WAVES partial sums of each column block are added through LDS, one row
+// block at a time, and written once (plus D), or go to the workspace when K
+// is split across workgroups.
+template <int NBW, int WAVES, int S, int MB, bool HAS_D, bool FIN = false>
 __global__ __launch_bounds__(64 * WAVES) void packed_skinny_kernel(PackedArgs p) {
   static_assert(!FIN || MB == 1, "finishing in the kernel is instantiated for M <= 16");
   __shared__ v4i red[WAVES * NBW * 64];
@@ -1802,27 +1807,22 @@ __global__ __launch_bounds__(64 * WAVES) void packed_skinny_kernel(PackedArgs p)
   const int kb_beg = split * p.kb_per_split;
   const int kb_end = min(kb_beg + p.kb_per_split, p.kbt);
   const int acol = (lane >> 4) * 16;
-  bool arow_ok[MB];
   const int8_t *a_src[MB];
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb) {
-    const int arow = mb * 16 + (lane & 15);
-    arow_ok[mb] = arow < p.M;
-    a_src[mb] = p.A + bidx * p.sa + (int64_t)(arow_ok[mb] ? arow : 0) * p.lda + acol;
-  }
+  for (int mb = 0; mb < MB; ++mb)
+    a_src[mb] = p.A + bidx * p.sa + (int64_t)min(mb * 16 + (lane & 15), p.M - 1) * p.lda;
   const int8_t *Bb = p.Bp + bidx * p.sbp;
   // Tiles 0 .. live-1 are blocks nb0 .. nb_last. Live columns of tile n within
-  // its block: [col_lo(n), col_hi(n)); with MASKED a lane loads B only for a
-  // live column (l % 16).
+  // its block: [col_lo(n), col_hi(n)).
   const int live = nb_last - nb0 + 1;
-  auto col_lo = [&](int n) { return (MASKED && n == 0 && (h0 & 1)) ? 8 : 0; };
-  auto col_hi = [&](int n) { return n >= live ? 0 : (MASKED && n == live - 1 && (h1 & 1)) ? 8 : 16; };
-  bool b_live[NBW];
+  auto col_lo = [&](int n) { return (n == 0 && (h0 & 1)) ? 8 : 0; };
+  auto col_hi = [&](int n) { return n >= live ? 0 : (n == live - 1 && (h1 & 1)) ? 8 : 16; };
   int64_t b_off[NBW];
 #pragma unroll
   for (int n = 0; n < NBW; ++n) {
-    b_live[n] = (lane & 15) >= col_lo(n) && (lane & 15) < col_hi(n);
-    b_off[n] = (int64_t)min(nb0 + n, nbt - 1) * p.kbt * 1024 + lane * 16;
+    const int t = min(n, live - 1), c = lane & 15;
+    const bool dead = c < col_lo(t) || c >= col_hi(t);
+    b_off[n] = (int64_t)(nb0 + t) * p.kbt * 1024 + (dead ? lane ^ 8 : lane) * 16;
   }
   v4i acc[MB][NBW];
 #pragma unroll
@@ -1834,36 +1834,42 @@ __global__ __launch_bounds__(64 * WAVES) void packed_skinny_kernel(PackedArgs p)
   const int steps = first < kb_end ? (kb_end - first + WAVES - 1) / WAVES : 0;
   v4i a[S][MB], b[S][NBW];
   auto load = [&](int s, v4i (&av)[MB], v4i (&bv)[NBW]) {
-    if (s < steps) {
-      const int kb = first + s * WAVES;
+    const int kb = first + s * WAVES;
+#pragma unroll
+    for (int n = 0; n < NBW; ++n)
+      bv[n] = __builtin_nontemporal_load((const v4i *)(Bb + b_off[n] + (int64_t)kb * 1024));
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) av[mb] = *(const v4i *)(a_src[mb] + min(kb * 64 + acol, p.K - 16));
+  };
+  auto multiply = [&](const v4i (&av)[MB], const v4i (&bv)[NBW]) {
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
       for (int n = 0; n < NBW; ++n)
-        bv[n] = (!MASKED || b_live[n])
-                    ? __builtin_nontemporal_load((const v4i *)(Bb + b_off[n] + (int64_t)kb * 1024))
-                    : v4i{0, 0, 0, 0};
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb)
-        av[mb] = (arow_ok[mb] && kb * 64 + acol < p.K) ? *(const v4i *)(a_src[mb] + kb * 64)
-                                                       : v4i{0, 0, 0, 0};
-    } else {
-#pragma unroll
-      for (int n = 0; n < NBW; ++n) bv[n] = v4i{0, 0, 0, 0};
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) av[mb] = v4i{0, 0, 0, 0};
-    }
+        acc[mb][n] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[mb], bv[n], acc[mb][n], 0, 0, 0);
   };
+  // Whole rounds of S blocks have no branch around a load (it makes the
+  // compiler wait for every load in flight); the last round loads only the
+  // blocks that are left.
+  if (steps > 0) {
 #pragma unroll
-  for (int s = 0; s < S; ++s) load(s, a[s], b[s]);
-  for (int s0 = 0; s0 < steps; s0 += S) {
+    for (int s = 0; s < S; ++s) load(min(s, steps - 1), a[s], b[s]);
+    int s0 = 0;
+    for (; s0 + 2 * S <= steps; s0 += S) {
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        multiply(a[s], b[s]);
+        load(s0 + s + S, a[s], b[s]);
+      }
+    }
 #pragma unroll
     for (int s = 0; s < S; ++s) {
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-        for (int n = 0; n < NBW; ++n)
-          acc[mb][n] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[s][mb], b[s][n], acc[mb][n], 0, 0, 0);
-      load(s0 + s + S, a[s], b[s]);
+      if (s0 + s < steps) multiply(a[s], b[s]);
+      if (s0 + s + S < steps) load(s0 + s + S, a[s], b[s]);
     }
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+      if (s0 + s + S < steps) multiply(a[s], b[s]);
   }
 
   // 16x16 accumulator layout: element e of lane l is row 4*(l/16) + e,
@@ -1894,11 +1900,11 @@ __global__ __launch_bounds__(64 * WAVES) void packed_skinny_kernel(PackedArgs p)
         s0 = add_wrap(s0, v[e]);
         s1 = add_wrap(s1, v[e + 1]);
       }
-      if (MASKED ? (c < col_lo(n) || c >= col_hi(n)) : n >= live) continue;
+      if (c < col_lo(n) || c >= col_hi(n)) continue;
       if (row >= p.M) continue;
       const int col = (nb0 + n) * 16 + c;
-      // Rows past M hold zero sums (zero A rows): a lone last row's
-      // neighbour field adds the bias alone.
+      // A lone last row's neighbour field adds row M - 1's sum again: in
+      // range like any other, and never stored.
       const uint64_t lo = (uint64_t)((int64_t)s0 + bias), hi = (uint64_t)((int64_t)s1 + bias);
       uint64_t *word = fb + (int64_t)pr * p.N + col;
       const uint64_t old = __hip_atomic_fetch_add(word, (1ull << (2 * fw)) | (hi << fw) | lo,
@@ -1932,7 +1938,7 @@ __global__ __launch_bounds__(64 * WAVES) void packed_skinny_kernel(PackedArgs p)
       for (int wv = 0; wv < WAVES; ++wv)
         s = add_wrap(s, ((const int32_t *)&red[(wv * NBW + n) * 64 + src])[e]);
       const int row = mb * 16 + r16;
-      if (MASKED ? (c < col_lo(n) || c >= col_hi(n)) : n >= live) continue;
+      if (c < col_lo(n) || c >= col_hi(n)) continue;
       if (row >= p.M) continue;
       const int col = (nb0 + n) * 16 + c;
       if (p.k_split == 1) {
@@ -2908,36 +2914,74 @@ int launch_skinny(const Problem &q, int k_split, Scratch &scr) {
 // Packed-B decode configuration: 4 column blocks (64 columns) per workgroup,
 // 8 waves, 2 row blocks of loads ahead. For N = 14336 that is 224 workgroups
 // streaming 256 KiB each.
-constexpr int kPackedNBW = 4, kPackedWaves = 8, kPackedS = 2;
+constexpr int kPackedNBW = 4, kPackedWaves = 8;
 
 int64_t packed_kbt(int64_t K) { return (K + 63) / 64; }
 
-// Half blocks per column group. Whole groups of NBW blocks when they alone
-// give 192 or more workgroups (N = 14336: 224 groups). Below that, groups as
-// small as needed for one per CU, at half-block granularity, instead of a K
-// split and a second kernel: measured at K = 4096, N = 1024 .. 8192 run 16-22 %
-// faster that way. At N = 14336, 256 groups of 3.5 blocks ran 3 % slower than
-// 224 groups of 4, so larger N keeps whole groups.
-int packed_hpw(int64_t N, int64_t batch, int num_cus) {
+// Half blocks per column group with K in `ks` slices. Whole groups of NBW
+// blocks when they alone give 192 or more workgroups (N = 14336: 224 groups).
+// Below that, groups as small as needed for one workgroup per CU, at
+// half-block granularity. At N = 14336, 256 groups of 3.5 blocks ran 3 %
+// slower than 224 groups of 4, so larger N keeps whole groups.
+int packed_hpw(int64_t N, int64_t batch, int ks, int num_cus) {
   const int64_t nbt = N / 16;
-  if ((nbt + kPackedNBW - 1) / kPackedNBW * batch >= 192) return 2 * kPackedNBW;
-  int64_t h = (2 * nbt * batch + num_cus - 1) / num_cus;
+  if ((nbt + kPackedNBW - 1) / kPackedNBW * batch * ks >= 192) return 2 * kPackedNBW;
+  int64_t h = (2 * nbt * batch * ks + num_cus - 1) / num_cus;
   if (h < 1) h = 1;
   if (h > 2 * kPackedNBW) h = 2 * kPackedNBW;
   return (int)h;
 }
 
-// Workgroups along K for the packed kernel, given the column groups of all
-// batches: 1 when those alone give most CUs a workgroup, else enough K slices
-// for ~224 workgroups, each slice at least one row block per wave.
-int packed_k_split(int64_t groups, int64_t K) {
-  if (groups >= 192) return 1;
-  int64_t ks = (224 + groups - 1) / groups;
-  const int64_t max_by_k = (packed_kbt(K) + kPackedWaves - 1) / kPackedWaves;
-  if (ks > max_by_k) ks = max_by_k;
-  if (ks < 1) ks = 1;
-  if (ks > 64) ks = 64;
-  return (int)ks;
+// Slices of K for M (<= 64) rows over so few columns that one workgroup per
+// CU takes narrow groups: every workgroup then reads its whole slice of A,
+// which costs 27 ns per KB (N = 4096, K = 14336, narrow groups unsplit: M = 1
+// 10.4 us, 16 16.8, 32 22.3, 48 29.3). Slices with wider groups read A/ks but
+// have to be summed: about 2 us through the finishing words, or 4 us and the
+// partial sums' traffic at 3 TB/s in a second kernel. The least of the three
+// estimates, in ns: at that N and K four slices for M = 16 (12.8 us), 32
+// (16.6) and 48 (20.0) and none for M = 1 (two slices 11.1); N = 2048,
+// K = 8192 four for M = 48 (16.4 -> 10.6); N = 8192, K = 4096 none (M = 48
+// 12.5 us, two slices 14.4).
+int packed_a_split(int64_t M, int64_t N, int64_t K) {
+  int best = 1;
+  int64_t least = 0;
+  for (int ks = 1; ks <= 4; ks *= 2) {
+    if (ks > 1 && packed_kbt(K) < (int64_t)ks * kPackedWaves) break;
+    const int64_t chunk = (packed_kbt(K) + ks - 1) / ks * 64;
+    int64_t ns = 27 * M * K / ks / 1000;
+    if (ks > 1)
+      ns += M <= kSkinnyFinMaxM && skinny_fin_bits(ks, chunk) > 0 ? 2000 : 4000 + 8 * M * N * ks / 3000;
+    if (ks == 1 || ns < least) {
+      least = ns;
+      best = ks;
+    }
+  }
+  return best;
+}
+
+// Workgroups along K for the packed kernel and the columns of their groups.
+// Few columns in all (fewer than 192 groups of half blocks): enough K slices
+// for ~224 workgroups, each slice at least one row block per wave; else
+// packed_a_split's, when `a_split` is allowed and groups are narrow.
+struct PackedGeom {
+  int hpw, ks;
+};
+
+PackedGeom packed_geometry(int64_t M, int64_t N, int64_t K, int64_t batch, bool a_split, int num_cus) {
+  PackedGeom g = {packed_hpw(N, batch, 1, num_cus), 1};
+  const int64_t groups = (2 * (N / 16) + g.hpw - 1) / g.hpw * batch;
+  if (groups < 192) {
+    int64_t ks = (224 + groups - 1) / groups;
+    const int64_t max_by_k = (packed_kbt(K) + kPackedWaves - 1) / kPackedWaves;
+    if (ks > max_by_k) ks = max_by_k;
+    if (ks < 1) ks = 1;
+    if (ks > 64) ks = 64;
+    g.ks = (int)ks;
+  } else if (a_split && g.hpw < 2 * kPackedNBW) {
+    g.ks = packed_a_split(M, N, K);
+    g.hpw = packed_hpw(N, batch, g.ks, num_cus);
+  }
+  return g;
 }
 
 // Whether the rows of a packed-B GEMM in whole 256-row tiles can run on the
@@ -3048,32 +3092,45 @@ int launch_packed_dma128(const Problem &q, hipStream_t stream, int num_cus) {
   return VT_OK;
 }
 
+// Blocks of 64 rows each wave loads ahead, by the column blocks it holds. More
+// were no faster (M = 1, N = 4096, K = 14336, one column block: 4 stages 10.4
+// us, 6 10.7, 8 10.9; 2048 x 8192, M = 8: 7.0, 7.3, 7.2).
+constexpr int packed_stages(int nbw) { return nbw == 1 ? 4 : nbw == 2 ? 3 : 2; }
+
+template <int NBW, int MB, bool FIN>
+void launch_packed_blocks(bool d_in, dim3 grid, dim3 block, hipStream_t s, const PackedArgs &a) {
+  constexpr int S = packed_stages(NBW);
+  if (d_in) hipLaunchKernelGGL((packed_skinny_kernel<NBW, kPackedWaves, S, MB, true, FIN>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((packed_skinny_kernel<NBW, kPackedWaves, S, MB, false, FIN>), grid, block, 0, s, a);
+}
+
 template <int MB, bool FIN = false>
-void launch_packed_kernel(bool d_in, bool masked, dim3 grid, dim3 block, hipStream_t s,
-                          const PackedArgs &a) {
-  if (d_in && masked)
-    hipLaunchKernelGGL((packed_skinny_kernel<kPackedNBW, kPackedWaves, kPackedS, MB, true, true, FIN>), grid, block, 0, s, a);
-  else if (d_in)
-    hipLaunchKernelGGL((packed_skinny_kernel<kPackedNBW, kPackedWaves, kPackedS, MB, true, false, FIN>), grid, block, 0, s, a);
-  else if (masked)
-    hipLaunchKernelGGL((packed_skinny_kernel<kPackedNBW, kPackedWaves, kPackedS, MB, false, true, FIN>), grid, block, 0, s, a);
-  else
-    hipLaunchKernelGGL((packed_skinny_kernel<kPackedNBW, kPackedWaves, kPackedS, MB, false, false, FIN>), grid, block, 0, s, a);
+void launch_packed_kernel(bool d_in, dim3 grid, dim3 block, hipStream_t s, const PackedArgs &a) {
+  switch ((a.hpw + 1) / 2) {
+    case 1: launch_packed_blocks<1, MB, FIN>(d_in, grid, block, s, a); break;
+    case 2: launch_packed_blocks<2, MB, FIN>(d_in, grid, block, s, a); break;
+    case 3: launch_packed_blocks<3, MB, FIN>(d_in, grid, block, s, a); break;
+    default: launch_packed_blocks<kPackedNBW, MB, FIN>(d_in, grid, block, s, a); break;
+  }
 }
 
 // One launch (plus the partial-sum reduction when K is split) over at most
-// kSkinnyMaxM (64) rows of A / C / D: 1, 2 or 4 row blocks of 16.
-int launch_packed_rows(const Problem &q, int k_split, Scratch &scr) {
+// kSkinnyMaxM (64) rows of A / C / D: 1 to 4 row blocks of 16. a_split: K may
+// be split to read less of A (packed_a_split).
+int launch_packed_rows(const Problem &q, int k_split, Scratch &scr, bool a_split = true) {
   PackedArgs a;
   a.A = q.A; a.Bp = q.B; a.D = q.D; a.C = q.C;
   a.lda = q.lda; a.ldd = q.ldd; a.ldc = q.ldc;
   a.sa = q.sa; a.sbp = q.sb; a.sd = q.sd; a.sc = q.sc;
   a.M = (int)q.M; a.N = (int)q.N; a.K = (int)q.K;
   a.kbt = (int)packed_kbt(q.K);
-  a.hpw = packed_hpw(q.N, q.batch, scr.st->num_cus);
+  const int cus = scr.st->num_cus;
+  const PackedGeom base = packed_geometry(q.M, q.N, q.K, q.batch, false, cus);
+  const PackedGeom geo = k_split > 0 ? PackedGeom{base.hpw, k_split}
+                                     : packed_geometry(q.M, q.N, q.K, q.batch, a_split, cus);
+  a.hpw = geo.hpw;
   a.groups = (int)((2 * (q.N / 16) + a.hpw - 1) / a.hpw);
-  const int ks0 = k_split > 0 ? k_split : packed_k_split((int64_t)a.groups * q.batch, q.K);
-  a.kb_per_split = (a.kbt + ks0 - 1) / ks0;
+  a.kb_per_split = (a.kbt + geo.ks - 1) / geo.ks;
   a.k_split = (a.kbt + a.kb_per_split - 1) / a.kb_per_split;
   a.ws = nullptr;
   a.fin = nullptr;
@@ -3083,31 +3140,38 @@ int launch_packed_rows(const Problem &q, int k_split, Scratch &scr) {
   // The K slices finish in the kernel on the skinny kernel's terms (few
   // rows, a count that fits beside the fields, a per-stream workspace).
   const bool fin = skinny_finishes(q.M, a.k_split, (int64_t)a.kb_per_split * 64, scr);
-  if (fin) {
+  if (a.k_split > 1) {
     void *w = nullptr;
-    int rc = scr.take(kFinWords, (size_t)q.batch * ((q.M + 1) / 2) * q.N * sizeof(uint64_t), &w);
-    if (rc) return rc;
-    a.fin = (uint64_t *)w;
-    a.fin_bits = skinny_fin_bits(a.k_split, (int64_t)a.kb_per_split * 64);
-  } else if (a.k_split > 1) {
-    void *w = nullptr;
-    const size_t pbytes = (size_t)q.batch * a.k_split * q.M * q.N * sizeof(int32_t);
-    int rc = scr.take(kPartials, pbytes, &w);
-    if (rc) return rc;
-    a.ws = (int32_t *)w;
+    const size_t bytes = fin ? (size_t)q.batch * ((q.M + 1) / 2) * q.N * sizeof(uint64_t)
+                             : (size_t)q.batch * a.k_split * q.M * q.N * sizeof(int32_t);
+    if (int rc = scr.take(fin ? kFinWords : kPartials, bytes, &w)) {
+      // A split only to read less of A is not needed: without a workspace
+      // (none yet on a stream being captured, or no memory) run unsplit.
+      if (k_split > 0 || base.ks == geo.ks) return rc;
+      (void)hipGetLastError();
+      g_err.clear();
+      return launch_packed_rows(q, 0, scr, false);
+    }
+    if (fin) {
+      a.fin = (uint64_t *)w;
+      a.fin_bits = skinny_fin_bits(a.k_split, (int64_t)a.kb_per_split * 64);
+    } else {
+      a.ws = (int32_t *)w;
+    }
   }
   hipStream_t s = (hipStream_t)scr.stream;
   dim3 grid((unsigned)(a.groups * a.k_split), (unsigned)q.batch), block(64 * kPackedWaves);
-  const bool d_in = q.D && (a.k_split == 1 || fin), masked = a.hpw != 2 * kPackedNBW;
+  const bool d_in = q.D && (a.k_split == 1 || fin);
   if (fin) {
-    launch_packed_kernel<1, true>(d_in, masked, grid, block, s, a);
+    launch_packed_kernel<1, true>(d_in, grid, block, s, a);
     VT_HIP_CHECK(hipGetLastError());
     return VT_OK;
   }
-  switch (skinny_row_blocks(q.M)) {
-    case 1: launch_packed_kernel<1>(d_in, masked, grid, block, s, a); break;
-    case 2: launch_packed_kernel<2>(d_in, masked, grid, block, s, a); break;
-    default: launch_packed_kernel<4>(d_in, masked, grid, block, s, a); break;
+  switch ((q.M + 15) / 16) {
+    case 1: launch_packed_kernel<1>(d_in, grid, block, s, a); break;
+    case 2: launch_packed_kernel<2>(d_in, grid, block, s, a); break;
+    case 3: launch_packed_kernel<3>(d_in, grid, block, s, a); break;
+    default: launch_packed_kernel<4>(d_in, grid, block, s, a); break;
   }
   VT_HIP_CHECK(hipGetLastError());
   if (a.k_split > 1) {

@@ -180,34 +180,67 @@ def _auto_k_split(n, k, batch):
 PACKED_NBW = 4   # 16-column blocks one packed workgroup holds
 
 
+def _packed_hpw(n, batch, ks, num_cus):
+    """packed_hpw in csrc/vt_hip_gemm.hip."""
+    nbt = n // 16
+    if -(-nbt // PACKED_NBW) * batch * ks >= 192:
+        return 2 * PACKED_NBW
+    return max(1, min(-(-2 * nbt * batch * ks // num_cus), 2 * PACKED_NBW))
+
+
+def _packed_a_split(m, n, k):
+    """packed_a_split in csrc/vt_hip_gemm.hip: K slices for m rows over narrow
+    column groups, by the least estimated cost of reading A and summing."""
+    kbt, best, least = -(-k // 64), 1, None
+    for ks in (1, 2, 4):
+        if ks > 1 and kbt < ks * PACKED_WAVES:
+            break
+        ns = 27 * m * k // ks // 1000
+        if ks > 1:
+            fin = m <= SKINNY_FIN_MAX_M and skinny_fin_bits(ks, -(-kbt // ks) * 64) > 0
+            ns += 2000 if fin else 4000 + 8 * m * n * ks // 3000
+        if least is None or ns < least:
+            best, least = ks, ns
+    return best
+
+
+def _packed_geometry(plan, num_cus=NUM_CUS):
+    """(8-column half blocks per column group, K slices) of the packed kernel
+    (packed_geometry / launch_packed_rows in csrc/vt_hip_gemm.hip) for at most
+    SKINNY_MAX_M rows; a plan of more rows runs groups of that many."""
+    n, k, batch = plan["n"], plan["k"], plan["batch"]
+    m = min(plan["m"], SKINNY_MAX_M)
+    hpw = _packed_hpw(n, batch, 1, num_cus)
+    if plan["k_split"] > 0:
+        return hpw, plan["k_split"]
+    groups = -(-2 * (n // 16) // hpw) * batch
+    if groups < 192:
+        return hpw, max(1, min(-(-224 // groups), -(-(-(-k // 64)) // PACKED_WAVES), 64))
+    if hpw == 2 * PACKED_NBW:
+        return hpw, 1
+    ks = _packed_a_split(m, n, k)
+    return _packed_hpw(n, batch, ks, num_cus), ks
+
+
 def packed_columns(plan, num_cus=NUM_CUS):
     """(8-column half blocks per column group, column groups per batch) of the
-    packed kernel: whole groups of PACKED_NBW blocks when they give 192 or
-    more workgroups, else groups as small as one per CU needs (down to half a
-    block) instead of a K split. Mirrors packed_hpw / launch_packed_rows in
-    csrc/vt_hip_gemm.hip, which use the device's CU count (256 on an MI355X)."""
-    nbt, batch = plan["n"] // 16, plan["batch"]
-    if -(-nbt // PACKED_NBW) * batch >= 192:
-        hpw = 2 * PACKED_NBW
-    else:
-        hpw = max(1, min(-(-2 * nbt * batch // num_cus), 2 * PACKED_NBW))
-    return hpw, -(-2 * nbt // hpw)
+    packed kernel: whole groups of PACKED_NBW blocks when they (times the K
+    slices) give 192 or more workgroups, else groups as small as one per CU
+    needs (down to half a block). Mirrors csrc/vt_hip_gemm.hip, which uses the
+    device's CU count (256 on an MI355X)."""
+    hpw = _packed_geometry(plan, num_cus)[0]
+    return hpw, -(-2 * (plan["n"] // 16) // hpw)
 
 
 def packed_split(plan):
     """(k_split, 64-row blocks per slice) the packed kernel launches.
 
-    Mirrors packed_k_split / launch_packed_rows in csrc/vt_hip_gemm.hip.
+    Mirrors launch_packed_rows in csrc/vt_hip_gemm.hip (which runs unsplit
+    where a split that only saves reads of A finds no workspace, as on a
+    stream captured before its first such call).
     """
-    k, batch, ks = plan["k"], plan["batch"], plan["k_split"]
-    kbt = -(-k // 64)
-    if ks <= 0:
-        groups = packed_columns(plan)[1] * batch
-        if groups >= 192:
-            ks = 1
-        else:
-            ks = max(1, min(-(-224 // groups), -(-kbt // PACKED_WAVES), 64))
-    per = -(-kbt // ks)
+    kbt = -(-plan["k"] // 64)
+    per = -(-kbt // _packed_geometry(plan)[1])
     return -(-kbt // per), per
 
 
