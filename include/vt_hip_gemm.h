@@ -69,14 +69,16 @@ extern "C" {
                                       when those do as well                   */
 #define VT_VARIANT_SKINNY 3        /* M <= 64 decode shapes: B streamed once,
                                       v_mfma_i32_16x16x64_i8, K split         */
-#define VT_VARIANT_GENERIC 4       /* any shape/stride/alignment, VALU        */
+#define VT_VARIANT_GENERIC 4       /* any shape/stride/alignment: VALU for tiny
+                                      products and N or K below 16, else the
+                                      MFMA / skinny kernels reading A and B
+                                      in place                                */
 #define VT_VARIANT_MFMA_256x128 5  /* 256x128 tile, 4 waves; M >= 256, N >= 128,
                                       K % 256 == 0 with 16-byte aligned C, D
                                       run persistently (one workgroup per CU) */
-#define VT_VARIANT_PADDED 6        /* any shape: A and B copied with K and N
-                                      zero-padded to multiples of 16, run on
-                                      the MFMA / skinny kernels, C copied out
-                                      (plus D)                                */
+#define VT_VARIANT_PADDED 6        /* any shape: as above, or A and B copied with
+                                      K and N zero-padded and run on the MFMA /
+                                      skinny kernels                          */
 #define VT_VARIANT_COUNT 7
 
 /*
@@ -102,10 +104,12 @@ extern "C" {
  * multiples of 16 and 16-byte-aligned A and B; an explicit one returns
  * VT_EUNSUPPORTED otherwise. For such shapes VT_VARIANT_AUTO picks
  * VT_VARIANT_PADDED from 3 * 2^24 multiply-adds on (M, N + 15, K + 15 < 2^30,
- * batch <= 65535) and VT_VARIANT_GENERIC below. VT_VARIANT_PADDED copies
- * the operands the vector variants cannot read as they are, zero padded, to
- * a workspace the library allocates once per (device, stream) and grows as
- * needed; when N % 16 == 0 the product writes C directly. For aligned
+ * batch <= 65535) and VT_VARIANT_GENERIC below. Both read such operands in
+ * place (N, K >= 16 and rows the MFMA variants can address); for large
+ * products VT_VARIANT_PADDED copies the operands the vector variants cannot
+ * read, zero padded, to a workspace the library allocates once per (device,
+ * stream) and grows as needed. vt_gemm_check reports the most it takes. For
+ * aligned
  * shapes VT_VARIANT_AUTO picks VT_VARIANT_SKINNY for M <= 16, and for
  * M <= 64 when K >= 512 and ceil(N / 128) * batch < 256 (the skinny kernel
  * runs 1, 2 or 4 row blocks of 16 over one stream of B), VT_VARIANT_GENERIC when K <= 64 and

@@ -50,7 +50,9 @@
 //       next on the same stream, adds them (and D); up to 16 rows the kernel
 //       finishes them itself through one 64-bit word per two output elements.
 //   generic_kernel  any shape, stride or alignment; one thread per output,
-//       int32 VALU. Used where the vector kernels' alignment rules fail.
+//       int32 VALU. Used for tiny products, and where N or K is below 16.
+//   Operands off the 16-byte grid (odd N, K, pitches or addresses) are read in
+//       place by gemm_mfma_kernel<.., EDGE 3> and skinny_kernel<.., ANY>.
 //
 // Tails: rows of A past M and columns of B past N are read from clamped (valid)
 // addresses and their outputs are never stored; k past K reads A as zero, so
@@ -112,6 +114,41 @@ __device__ __forceinline__ void st_lds_b128(int8_t *base, int off, v4i v) {
 __device__ __forceinline__ v2i ld_lds_tr8(const int8_t *base, int off) {
   return __builtin_amdgcn_ds_read_tr8_b64_v2i32(
       (LDS_AS v2i *)((LDS_AS int8_t *)base + off));
+}
+
+// 16 bytes of global memory at any address (the target's global loads need no
+// alignment), cached or streamed.
+typedef v4i v4i_any __attribute__((aligned(1)));
+__device__ __forceinline__ v4i ld_any(const int8_t *p) { return *(const v4i_any *)p; }
+__device__ __forceinline__ v4i ld_any_nt(const int8_t *p) {
+  return __builtin_nontemporal_load((const v4i_any *)p);
+}
+
+// v moved down by `bytes` bytes (byte i takes byte i + bytes), zeros from the
+// top; all zeros from 16 on.
+__device__ __forceinline__ v4i drop_bytes(v4i v, int bytes) {
+  uint64_t lo = (uint32_t)v.x | (uint64_t)(uint32_t)v.y << 32;
+  uint64_t hi = (uint32_t)v.z | (uint64_t)(uint32_t)v.w << 32;
+  if (bytes >= 8) {
+    lo = hi;
+    hi = 0;
+  }
+  const int sh = (bytes & 7) * 8;
+  if (sh) {
+    lo = lo >> sh | hi << (64 - sh);
+    hi >>= sh;
+  }
+  if (bytes >= 16) lo = hi = 0;
+  return v4i{(int)(uint32_t)lo, (int)(lo >> 32), (int)(uint32_t)hi, (int)(hi >> 32)};
+}
+
+// Bytes pos .. pos + 15 of a row of `len` >= 16 bytes at any address, zero
+// past its end: nothing past the row is read.
+__device__ __forceinline__ v4i ld_row(const int8_t *row, int pos, int len) {
+  const int at = min(pos, len - 16);
+  v4i v = ld_any(row + at);
+  if (at != pos) v = drop_bytes(v, pos - at);
+  return v;
 }
 
 __device__ __forceinline__ int32_t add_wrap(int32_t a, int32_t b) {
@@ -234,12 +271,15 @@ struct GemmArgs {
   int M, N, K;
   int tiles_m, tiles_n, group_m;
   int batch_count;   // batches (the persistent kernel walks all their tiles)
+  int k_last;        // EDGE 3: K of the last batch (K slices run as batches)
 };
 
 // EDGE: 0 full tiles; 1 M or N not a multiple of the tile (clamped source
 // rows and columns, masked stores); 2 also K not a multiple of 128 (each load
 // checks the K tail). The K checks sit in the k loop, so a ragged M or N
-// alone does not pay for them.
+// alone does not pay for them; 3 any M, any N and K of at least 16, operands at
+// any address and pitch (16-byte loads need no alignment): a row's last bytes
+// are read from its last 16, moved into place, and zero past it.
 //
 // PACKED_B: B is in the packed layout of vt_pack_b_i8 (p.B = Bp, p.ldb = kbt,
 // the 64-row blocks per 16-column block; p.sb = the packed batch stride). A
@@ -287,7 +327,8 @@ __global__ __launch_bounds__(256, 1) void gemm_mfma_kernel(GemmArgs p) {
   const int m0 = (first_m + within % gm) * BM;
   const int n0 = (within / gm) * BN;
 
-  const int M = p.M, N = p.N, K = p.K;
+  const int M = p.M, N = p.N;
+  const int K = EDGE == 3 && bidx == p.batch_count - 1 ? p.k_last : p.K;
   // 64-bit bases at the tile's origin (row m0 of A, column n0 of B), so only
   // offsets within one tile need 32 bits (the host checks BM*lda and
   // BK*ldb), whatever the size of the whole matrix.
@@ -296,19 +337,29 @@ __global__ __launch_bounds__(256, 1) void gemm_mfma_kernel(GemmArgs p) {
 
   // Per-thread global source offsets for one 64-deep k slice, relative to a
   // wave-uniform base that advances by one slice per step.
-  uint32_t a_goff[CA];
+  // EDGE >= 2: the offsets in the last slice, where chunks past K move back to
+  // end there and rows of B past K re-read row K - 1. Offsets are from 16 bytes
+  // before the base with EDGE 3, whose moved chunks may start left of it.
+  constexpr int LEFT = EDGE == 3 ? 16 : 0;
+  const int k_tail = ((K + BK - 1) / BK - 1) * BK;   // first k of the last slice
+  uint32_t a_goff[CA], a_tail[EDGE >= 2 ? CA : 1];
   int a_lds[CA], a_k[CA];
 #pragma unroll
   for (int i = 0; i < CA; ++i) {
     const int row = (tid >> 2) + 64 * i, c = tid & 3;
     int trow = row;
     if (EDGE) trow = min(m0 + row, M - 1) - m0;
-    a_goff[i] = (uint32_t)((int64_t)trow * p.lda + c * 16);
+    a_goff[i] = (uint32_t)((int64_t)trow * p.lda + c * 16 + LEFT);
+    if constexpr (EDGE >= 2)
+      a_tail[i] = a_goff[i] - (uint32_t)max(c * 16 - (K - 16 - k_tail), 0);
     a_lds[i] = a_off(row, c);
     a_k[i] = c * 16;
   }
-  int b_row[CB], b_lds[CB];
-  uint32_t b_goff[CB];
+  // EDGE 3: a last tile's chunk moves back to end at column N; its columns
+  // below N drop into place on the way to LDS.
+  const bool b_moved = EDGE == 3 && n0 + BN > N;
+  int b_lds[CB], b_drop[EDGE == 3 ? CB : 1];
+  uint32_t b_goff[CB], b_tail[EDGE >= 2 ? CB : 1];
 #pragma unroll
   for (int i = 0; i < CB; ++i) {
     if constexpr (PACKED_B) {
@@ -316,47 +367,61 @@ __global__ __launch_bounds__(256, 1) void gemm_mfma_kernel(GemmArgs p) {
       const int ch = tid + 256 * i, t = ch >> 6, l = ch & 63;
       int tb = t;
       if (EDGE) tb = min(n0 / 16 + t, N / 16 - 1) - n0 / 16;
-      b_row[i] = 0;
       b_goff[i] = (uint32_t)((int64_t)tb * p.ldb * 1024 + l * 16);
+      if constexpr (EDGE >= 2) b_tail[i] = b_goff[i];   // rows past K are zero in the layout
       b_lds[i] = t * 1024 + l * 16;
     } else {
       const int row = tid / BCH + (256 / BCH) * i, c = tid % BCH;
       int tcol = c * 16;
       if (EDGE) tcol = min(n0 + tcol, N - 16) - n0;
-      b_row[i] = row;
-      b_goff[i] = (uint32_t)((int64_t)row * p.ldb + tcol);
+      b_goff[i] = (uint32_t)((int64_t)row * p.ldb + tcol + LEFT);
+      if constexpr (EDGE >= 2)
+        b_tail[i] = b_goff[i] - (uint32_t)max(row - (K - 1 - k_tail), 0) * (uint32_t)p.ldb;
+      if constexpr (EDGE == 3) b_drop[i] = min(c * 16 - tcol, 16);
       b_lds[i] = row * BN + ((c ^ b_swz<BCH>(row)) << 4);
     }
   }
 
   const int KT = (K + BK - 1) / BK;
   // Global -> VGPR staging of k slice kt into (ra, rb). Slices past the last
-  // one re-read the last slice (L2-resident); on the edge path their A part
-  // is zero, so a padding step computes nothing, and elsewhere they are never
-  // computed. The main loop thus has no data-dependent branches.
+  // one re-read the last slice (L2-resident); with EDGE >= 2 their A part is
+  // zeroed on the way to LDS, so a padding step computes nothing, and elsewhere
+  // they are never computed. No load has a branch around it and no loaded
+  // value is used before store_slice, two steps later: the K tail's check at
+  // the load made the compiler wait for it there (64x64 tiles, 1000 x 1008 x
+  // 1008 + D: 9.5 -> 7.3 us).
   auto load_slice = [&](int kt, v4i *ra, v4i *rb) {
     const int k0 = min(kt, KT - 1) * BK;
-    const int8_t *abase = Ab + k0;
-    const int8_t *bbase = Bb + (PACKED_B ? (int64_t)(k0 / BK) * 1024 : (int64_t)k0 * p.ldb);
+    const int8_t *abase = Ab + k0 - LEFT;
+    const int8_t *bbase = Bb + (PACKED_B ? (int64_t)(k0 / BK) * 1024 : (int64_t)k0 * p.ldb) - LEFT;
+    const bool tail = EDGE >= 2 && kt >= KT - 1;
 #pragma unroll
     for (int i = 0; i < CA; ++i) {
-      if (EDGE == 2 && kt * BK + a_k[i] >= K) {
-        ra[i] = v4i{0, 0, 0, 0};
-      } else {
-        ra[i] = *(const v4i *)(abase + a_goff[i]);
-      }
+      if constexpr (EDGE == 3) ra[i] = ld_any(abase + (tail ? a_tail[i] : a_goff[i]));
+      else if constexpr (EDGE == 2) ra[i] = *(const v4i *)(abase + (tail ? a_tail[i] : a_goff[i]));
+      else ra[i] = *(const v4i *)(abase + a_goff[i]);
     }
 #pragma unroll
     for (int i = 0; i < CB; ++i) {
-      if (!PACKED_B && EDGE == 2 && k0 + b_row[i] >= K) {
-        // rows past K: re-read row K-1 (A is zero there)
-        rb[i] = *(const v4i *)(Bb + (int64_t)(K - 1 - b_row[i]) * p.ldb + b_goff[i]);
-      } else {
-        rb[i] = *(const v4i *)(bbase + b_goff[i]);
-      }
+      if constexpr (EDGE == 3) rb[i] = ld_any(bbase + (tail ? b_tail[i] : b_goff[i]));
+      else if constexpr (EDGE == 2) rb[i] = *(const v4i *)(bbase + (tail ? b_tail[i] : b_goff[i]));
+      else rb[i] = *(const v4i *)(bbase + b_goff[i]);
     }
   };
-  auto store_slice = [&](int buf, const v4i *ra, const v4i *rb) {
+  // Slice kt's registers -> LDS buffer buf.
+  auto store_slice = [&](int buf, int kt, v4i *ra, v4i *rb) {
+    if (EDGE >= 2 && (kt + 1) * BK > K) {
+#pragma unroll
+      for (int i = 0; i < CA; ++i) {
+        const int past = kt * BK + a_k[i] - (K - 16);   // bytes of the chunk past K
+        if constexpr (EDGE == 3) ra[i] = drop_bytes(ra[i], max(past, 0));
+        else ra[i] = past > 0 ? v4i{0, 0, 0, 0} : ra[i];
+      }
+    }
+    if (EDGE == 3 && b_moved) {
+#pragma unroll
+      for (int i = 0; i < CB; ++i) rb[i] = drop_bytes(rb[i], b_drop[i]);
+    }
 #pragma unroll
     for (int i = 0; i < CA; ++i) st_lds_b128(As0 + buf * A_BYTES, a_lds[i], ra[i]);
 #pragma unroll
@@ -455,13 +520,13 @@ __global__ __launch_bounds__(256, 1) void gemm_mfma_kernel(GemmArgs p) {
   if constexpr (SHORT) {
     load_slice(0, ra0, rb0);
     load_slice(1, ra1, rb1);
-    store_slice(0, ra0, rb0);
-    store_slice(1, ra1, rb1);
+    store_slice(0, 0, ra0, rb0);
+    store_slice(1, 1, ra1, rb1);
   } else {
     load_slice(0, ra0, rb0);
-    store_slice(0, ra0, rb0);
     load_slice(1, ra1, rb1);
-    store_slice(1, ra1, rb1);
+    store_slice(0, 0, ra0, rb0);
+    store_slice(1, 1, ra1, rb1);
     load_slice(2, ra0, rb0);
     load_slice(3, ra1, rb1);
   }
@@ -469,7 +534,11 @@ __global__ __launch_bounds__(256, 1) void gemm_mfma_kernel(GemmArgs p) {
   read_frags(0, 0, fa0, fb0);
   int b0 = 0, b1 = 1, b2 = 2;   // buffers of slices kt, kt+1, kt+2
   constexpr int NMFMA = MI * NI, NREAD = MI + (PACKED_B ? 1 : 2) * NI, NSTORE = CA + CB;
-  auto step = [&](int kt, v4i *ra, v4i *rb) {
+  // fill: how much of the pipeline behind slice kt the step still feeds
+  // (compile time): 2 slice kt + 2 to LDS and slice kt + 4 from memory, 1 only
+  // the former, 0 neither.
+  auto step = [&](auto fill, int kt, v4i *ra, v4i *rb) {
+    constexpr int FILL = decltype(fill)::value;
     // First half step: fragments of k 32..63 load under the MFMAs of k 0..31.
     read_frags(b0, 1, fa1, fb1);
     mfma_block(fa0, fb0);
@@ -479,22 +548,19 @@ __global__ __launch_bounds__(256, 1) void gemm_mfma_kernel(GemmArgs p) {
       if (2 * i < NREAD) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // DS read
     }
     __builtin_amdgcn_sched_barrier(0);
-    // Second half step: slice kt+2 to LDS, slice kt+4 from memory (neither
-    // exists with SHORT) and the next step's first fragments, interleaved
-    // with the MFMAs of k 32..63.
-    if constexpr (!SHORT) {
-      store_slice(b2, ra, rb);
-      load_slice(kt + 4, ra, rb);
-    }
+    // Second half step: slice kt+2 to LDS, slice kt+4 from memory and the
+    // next step's first fragments, interleaved with the MFMAs of k 32..63.
+    if constexpr (FILL > 0) store_slice(b2, kt + 2, ra, rb);
+    if constexpr (FILL > 1) load_slice(kt + 4, ra, rb);
     read_frags(b1, 0, fa0, fb0);
     mfma_block(fa1, fb1);
 #pragma unroll
     for (int i = 0; i < NMFMA; ++i) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 1);                   // MFMA
-      if (i < NSTORE) {
+      if (FILL > 0 && i < NSTORE) {
         __builtin_amdgcn_sched_group_barrier(0x200, 1, 1);                 // DS write
-        __builtin_amdgcn_sched_group_barrier(0x020, 1, 1);                 // VMEM read
-      } else if (2 * (i - NSTORE) < NREAD) {
+        if (FILL > 1) __builtin_amdgcn_sched_group_barrier(0x020, 1, 1);   // VMEM read
+      } else if (2 * (FILL > 0 ? i - NSTORE : i) < NREAD) {
         __builtin_amdgcn_sched_group_barrier(0x100, 2, 1);                 // DS read
       }
     }
@@ -506,16 +572,26 @@ __global__ __launch_bounds__(256, 1) void gemm_mfma_kernel(GemmArgs p) {
     b2 = bt;
   };
   // Two steps per iteration (one per staging set). An odd step count only
-  // occurs with EDGE == 2 (the host routes K % 128 != 0 there), where the
-  // padding step multiplies zero A columns.
+  // occurs with EDGE >= 2 (the host routes K % 128 != 0 there), where the
+  // padding step multiplies zero A columns. The last four steps are peeled:
+  // loading on to the end of the loop fetched four slices nobody multiplies
+  // (K = 1024: a quarter of the tile's traffic).
+  using Full = std::integral_constant<int, 2>;
+  using Drain = std::integral_constant<int, 1>;
+  using Last = std::integral_constant<int, 0>;
   if constexpr (SHORT) {
-    step(0, ra0, rb0);
-    step(1, ra1, rb1);
+    step(Last(), 0, ra0, rb0);
+    step(Last(), 1, ra1, rb1);
   } else {
-    for (int kt = 0; kt < KT; kt += 2) {
-      step(kt, ra0, rb0);
-      step(kt + 1, ra1, rb1);
+    int kt = 0;
+    for (; kt + 4 < KT; kt += 2) {
+      step(Full(), kt, ra0, rb0);
+      step(Full(), kt + 1, ra1, rb1);
     }
+    step(Drain(), kt, ra0, rb0);
+    step(Drain(), kt + 1, ra1, rb1);
+    step(Last(), kt + 2, ra0, rb0);
+    step(Last(), kt + 3, ra1, rb1);
   }
 
   if constexpr (D_TILE) {
@@ -1396,6 +1472,10 @@ __device__ __forceinline__ int skinny_b_swz(int row) {
   return (row & 7) | (((row >> 4) & 1) << 3);
 }
 
+// Row pitch of partial sums: N rounded up to the 4 columns the reduction reads
+// at a time.
+__host__ __device__ constexpr int64_t partial_pitch(int64_t N) { return (N + 3) & ~(int64_t)3; }
+
 struct SkinnyArgs {
   const int8_t *A;
   const int8_t *B;
@@ -1407,7 +1487,7 @@ struct SkinnyArgs {
   int tiles_n;     // ceil(N / NB)
   int k_split;     // K slices per column slab (workgroups along K)
   int k_chunk;     // rows per slice, a multiple of the stage rows x U
-  int32_t *ws;     // [batch][k_split][M][N] partials when k_split > 1
+  int32_t *ws;     // [batch][k_split][M][N] partials when k_split > 1 (ANY: rows of partial_pitch(N))
   uint64_t *fin;   // [batch][(M + 1) / 2][N] finishing words (FIN), zero between launches
   int fin_bits;    // FIN: width of each of the word's two sum fields
 };
@@ -1443,7 +1523,10 @@ constexpr int kFinSpanPerRow = 16256 + 16384;
 // read-modify-write of that one word, so the word's single modification order
 // alone decides which slice is last and what it sees: no fence, no flag in
 // other memory, no second kernel.
-template <int NB, int WAVES, int U, int MB, bool HAS_D, bool FIN = false>
+// ANY: N and K of at least 16 and operands at any address and pitch; the last
+// column block's chunk is read from the row's last 16 bytes and its columns
+// moved into place on the way to LDS, and A's last bytes likewise.
+template <int NB, int WAVES, int U, int MB, bool HAS_D, bool FIN = false, bool ANY = false>
 __global__ __launch_bounds__(64 * WAVES) void skinny_kernel(SkinnyArgs p) {
   constexpr int THREADS = 64 * WAVES;
   constexpr int NBLK = NB / 16;               // 16-column blocks = chunks per row
@@ -1484,6 +1567,7 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_kernel(SkinnyArgs p) {
 
   const int brow = tid / NBLK, bc = tid % NBLK;
   const int8_t *bsrc = Bb + min(n0 + bc * 16, N - 16);
+  const int b_drop = ANY ? min(max(n0 + bc * 16 - (N - 16), 0), 16) : 0;
   const int b_lds = brow * NB + ((bc ^ skinny_b_swz(brow)) << 4);
   // Loads for stages >= T (issued by the last U stages) re-read the slice's
   // last row, which is resident in L2, and are discarded.
@@ -1492,6 +1576,7 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_kernel(SkinnyArgs p) {
   // the L2-resident A slice and workspace.
   auto load_stage = [&](int s) -> v4i {
     const int krow = min(kbeg + s * R + brow, krow_last);
+    if constexpr (ANY) return ld_any_nt(bsrc + (int64_t)krow * p.ldb);
     return __builtin_nontemporal_load((const v4i *)(bsrc + (int64_t)krow * p.ldb));
   };
   v4i rb[U];
@@ -1505,7 +1590,11 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_kernel(SkinnyArgs p) {
       const int row = i / cpr, c = i - row * cpr;
       const int k = kbeg + c * 16;
       v4i v = v4i{0, 0, 0, 0};
-      if (row < M && k < K) v = *(const v4i *)(Ab + (int64_t)row * p.lda + k);
+      if constexpr (ANY) {
+        if (row < M) v = ld_row(Ab + (int64_t)row * p.lda, k, K);
+      } else if (row < M && k < K) {
+        v = *(const v4i *)(Ab + (int64_t)row * p.lda + k);
+      }
       st_lds_b128(As, row * a_stride + c * 16, v);
     }
   }
@@ -1524,6 +1613,7 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_kernel(SkinnyArgs p) {
     for (int u = 0; u < U; ++u) {
       const int s = t0 + u;
       int8_t *const Bs = Bs0 + (u & 1) * STAGE_BYTES;
+      if (ANY && b_drop) rb[u] = drop_bytes(rb[u], b_drop);
       st_lds_b128(Bs, b_lds, rb[u]);
       rb[u] = load_stage(s + U);
       lds_barrier();
@@ -1630,7 +1720,8 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_kernel(SkinnyArgs p) {
         if (g * 4 + 2 * h < M) finish(h, add(h));
     }
   } else {
-    int32_t *wsb = p.ws + ((int64_t)bidx * p.k_split + split) * M * N;
+    const int pitch = ANY ? partial_pitch(N) : N;
+    int32_t *wsb = p.ws + ((int64_t)bidx * p.k_split + split) * M * pitch;
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
@@ -1639,7 +1730,7 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_kernel(SkinnyArgs p) {
         // Non-temporal: the partials are read once, by the next kernel, and
         // kept out of L2 they need no writeback at the kernel boundary
         // (measured 15.4 -> 15.1 us per decode step at K = 4096, N = 14336).
-        if (row < M) __builtin_nontemporal_store(acc[mb][e], wsb + (int64_t)row * N + col);
+        if (row < M) __builtin_nontemporal_store(acc[mb][e], wsb + (int64_t)row * pitch + col);
       }
   }
 }
@@ -1647,7 +1738,7 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_kernel(SkinnyArgs p) {
 // C = D + sum over the K slices of the skinny partials. Launched on the same
 // stream right after skinny_kernel, so stream order makes the partials visible.
 struct ReduceArgs {
-  const int32_t *ws;   // [batch][k_split][M][N]
+  const int32_t *ws;   // [batch][k_split][M][partial_pitch(N)]
   const int32_t *D;
   int32_t *C;
   int64_t ldd, ldc, sd, sc;
@@ -1663,20 +1754,19 @@ constexpr int kReduceThreads = 64;
 
 template <bool HAS_D>
 __global__ __launch_bounds__(kReduceThreads) void skinny_reduce_kernel(ReduceArgs p) {
-  const int64_t i = (int64_t)blockIdx.x * kReduceThreads + threadIdx.x;   // over M*N/4 (N % 16 == 0)
-  const int64_t per = (int64_t)p.M * p.N / 4;
-  if (i >= per) return;
+  const int64_t i = (int64_t)blockIdx.x * kReduceThreads + threadIdx.x;   // over M * pitch / 4
+  const int64_t pitch = partial_pitch(p.N), slice = p.M * pitch;
+  if (i >= slice / 4) return;
   const int bidx = blockIdx.y;
   const int64_t e = i * 4;
-  const int row = (int)(e / p.N), col = (int)(e - (int64_t)row * p.N);
-  const int32_t *w = p.ws + (int64_t)bidx * p.k_split * p.M * p.N + e;
-  const int64_t slice = (int64_t)p.M * p.N;
+  const int row = (int)(e / pitch), col = (int)(e - row * pitch);
+  const int32_t *w = p.ws + (int64_t)bidx * p.k_split * slice + e;
   int32_t *c = p.C + bidx * p.sc + (int64_t)row * p.ldc + col;
   v4i s = v4i{0, 0, 0, 0};
   if constexpr (HAS_D) {
     const int32_t *d = p.D + bidx * p.sd + (int64_t)row * p.ldd + col;
 #pragma unroll
-    for (int t = 0; t < 4; ++t) s[t] = d[t];
+    for (int t = 0; t < 4; ++t) s[t] = col + t < p.N ? d[t] : 0;
   }
   // Up to 8 partials in flight at once: every load of a batch is issued
   // before the first add waits.
@@ -1692,7 +1782,8 @@ __global__ __launch_bounds__(kReduceThreads) void skinny_reduce_kernel(ReduceArg
       for (int t = 0; t < 4; ++t) s[t] = add_wrap(s[t], o[u][t]);
   }
 #pragma unroll
-  for (int t = 0; t < 4; ++t) c[t] = s[t];
+  for (int t = 0; t < 4; ++t)
+    if (col + t < p.N) c[t] = s[t];
 }
 
 // ---------------------------------------------------------------------------
@@ -2511,7 +2602,7 @@ Problem mfma_fold(const Problem &q) {
 // C = D + the k_split partial sums in ws, on `stream` after the kernel that
 // wrote them (stream order publishes the partials).
 int launch_reduce(const ReduceArgs &r, int64_t batch, hipStream_t stream) {
-  const int64_t per = (int64_t)r.M * r.N / 4;
+  const int64_t per = r.M * partial_pitch(r.N) / 4;
   if (per > 0x7fffffff || batch > 65535) return fail(VT_EUNSUPPORTED, "reduction grid too large");
   dim3 grid((unsigned)((per + kReduceThreads - 1) / kReduceThreads), (unsigned)batch);
   if (r.D) hipLaunchKernelGGL(skinny_reduce_kernel<true>, grid, dim3(kReduceThreads), 0, stream, r);
@@ -2736,6 +2827,7 @@ int launch_mfma_tiles(const Problem &r, hipStream_t stream, int num_cus) {
   const bool has_d = r.D != nullptr;
   dim3 grid((unsigned)blocks), block(256);
   a.batch_count = (int)r.batch;
+  a.k_last = a.K;
   if (!PACKED && BM == 256 && BN == 256 && persistent_fits(r)) {
     // Persistent: one workgroup per CU (the kernel's LDS allows no more).
     const int64_t g = blocks < num_cus ? blocks : num_cus;
@@ -2794,6 +2886,31 @@ int launch_mfma128(const Problem &q, Scratch &scr) {
   return launch_mfma<128, 128>(q, scr);
 }
 
+// Tiles over operands at any address and pitch (gemm_mfma_kernel EDGE 3), K
+// in ks slices of kc (the last one what is left) run as batches.
+template <int BM, int BN>
+int launch_any_tiles(const Problem &r, int ks, int64_t kc, hipStream_t stream, int num_cus) {
+  GemmArgs a;
+  a.A = r.A; a.B = r.B; a.D = r.D; a.C = r.C;
+  a.lda = r.lda; a.ldb = r.ldb; a.ldd = r.ldd; a.ldc = r.ldc;
+  a.sa = r.sa; a.sb = r.sb; a.sd = r.sd; a.sc = r.sc;
+  a.M = (int)r.M; a.N = (int)r.N;
+  a.K = (int)(ks > 1 ? kc : r.K);
+  a.k_last = (int)(ks > 1 ? r.K - (ks - 1) * kc : r.K);
+  a.tiles_m = (int)((r.M + BM - 1) / BM);
+  a.tiles_n = (int)((r.N + BN - 1) / BN);
+  a.group_m = 4;
+  a.batch_count = (int)(ks > 1 ? ks : r.batch);
+  const int64_t blocks = (int64_t)a.tiles_m * a.tiles_n * a.batch_count;
+  if (blocks > 0x7fffffff) return fail(VT_EUNSUPPORTED, "grid of %lld tiles too large", (long long)blocks);
+  const dim3 grid((unsigned)blocks), block(256);
+  const bool short_k = a.K <= 128, early_d = blocks <= num_cus;
+  if (r.D) launch_mfma_kernel<BM, BN, 3, true, false>(short_k, early_d, grid, block, stream, a);
+  else launch_mfma_kernel<BM, BN, 3, false, false>(short_k, early_d, grid, block, stream, a);
+  VT_HIP_CHECK(hipGetLastError());
+  return VT_OK;
+}
+
 // K slices of the skinny kernel: rows per slice (a multiple of the pipeline
 // length, shrunk until the A part fits in LDS), the split count that gives,
 // and the dynamic LDS bytes.
@@ -2820,11 +2937,11 @@ SkinnyGeom skinny_geometry(const Problem &q, int k_split) {
   return SkinnyGeom{chunk, lds, (int)((q.K + chunk - 1) / chunk)};
 }
 
-template <int NB, int WAVES, int U, int MB, bool FIN = false>
+template <int NB, int WAVES, int U, int MB, bool FIN, bool ANY>
 void launch_skinny_kernel(bool has_d, dim3 grid, dim3 block, size_t lds, hipStream_t s,
                           const SkinnyArgs &a) {
-  if (has_d) hipLaunchKernelGGL((skinny_kernel<NB, WAVES, U, MB, true, FIN>), grid, block, lds, s, a);
-  else hipLaunchKernelGGL((skinny_kernel<NB, WAVES, U, MB, false, FIN>), grid, block, lds, s, a);
+  if (has_d) hipLaunchKernelGGL((skinny_kernel<NB, WAVES, U, MB, true, FIN, ANY>), grid, block, lds, s, a);
+  else hipLaunchKernelGGL((skinny_kernel<NB, WAVES, U, MB, false, FIN, ANY>), grid, block, lds, s, a);
 }
 
 // Field width of the finishing word for k_split slices of chunk rows (the bit
@@ -2846,7 +2963,8 @@ bool skinny_finishes(int64_t M, int ks, int64_t chunk, const Scratch &scr) {
   return ks > 1 && M <= kSkinnyFinMaxM && !scr.fixed && skinny_fin_bits(ks, chunk) > 0;
 }
 
-template <int NB, int WAVES, int U>
+// ANY: operands at any address and pitch, N and K of at least 16.
+template <int NB, int WAVES, int U, bool ANY = false>
 int launch_skinny_cfg(const Problem &q, int k_split, Scratch &scr) {
   if (q.M > kSkinnyMaxM)
     return fail(VT_EUNSUPPORTED, "skinny variant needs M <= %d (M=%lld)", kSkinnyMaxM, (long long)q.M);
@@ -2875,7 +2993,7 @@ int launch_skinny_cfg(const Problem &q, int k_split, Scratch &scr) {
     a.fin_bits = skinny_fin_bits(ks, chunk);
   } else if (ks > 1) {
     void *w = nullptr;
-    const size_t pbytes = (size_t)q.batch * ks * q.M * q.N * sizeof(int32_t);
+    const size_t pbytes = (size_t)q.batch * ks * q.M * partial_pitch(q.N) * sizeof(int32_t);
     int rc = scr.take(kPartials, pbytes, &w);
     if (rc) return rc;
     a.ws = (int32_t *)w;
@@ -2886,14 +3004,14 @@ int launch_skinny_cfg(const Problem &q, int k_split, Scratch &scr) {
   // split or when it finishes the slices itself, else the reduction.
   const bool d_in = q.D && (ks == 1 || fin);
   if (fin) {
-    launch_skinny_kernel<NB, WAVES, U, 1, true>(d_in, grid, block, (size_t)lds, s, a);
+    launch_skinny_kernel<NB, WAVES, U, 1, true, ANY>(d_in, grid, block, (size_t)lds, s, a);
     VT_HIP_CHECK(hipGetLastError());
     return VT_OK;
   }
   switch (skinny_row_blocks(q.M)) {
-    case 1: launch_skinny_kernel<NB, WAVES, U, 1>(d_in, grid, block, (size_t)lds, s, a); break;
-    case 2: launch_skinny_kernel<NB, WAVES, U, 2>(d_in, grid, block, (size_t)lds, s, a); break;
-    default: launch_skinny_kernel<NB, WAVES, U, 4>(d_in, grid, block, (size_t)lds, s, a); break;
+    case 1: launch_skinny_kernel<NB, WAVES, U, 1, false, ANY>(d_in, grid, block, (size_t)lds, s, a); break;
+    case 2: launch_skinny_kernel<NB, WAVES, U, 2, false, ANY>(d_in, grid, block, (size_t)lds, s, a); break;
+    default: launch_skinny_kernel<NB, WAVES, U, 4, false, ANY>(d_in, grid, block, (size_t)lds, s, a); break;
   }
   VT_HIP_CHECK(hipGetLastError());
   if (ks > 1) {
@@ -3448,6 +3566,113 @@ int launch_vector(const Problem &q, int32_t variant, int32_t k_split, Scratch &s
   }
 }
 
+// ---------------------------------------------------------------------------
+// Operands at any address, pitch and size, read in place
+// ---------------------------------------------------------------------------
+
+enum DirectKind { kDirectNone, kDirectSkinny, kDirectTiles64, kDirectTiles128 };
+
+struct DirectPlan {
+  DirectKind kind = kDirectNone;
+  int ks = 1;             // K slices
+  int64_t kc = 0;         // K of every slice but the last (tiles)
+  int64_t scratch = 0;    // bytes of partial sums (tiles; the skinny kernel at most)
+};
+
+// K slices of whole 64-deep steps for a tile launch, the last one at least 16
+// deep (a shorter rest joins the slice before it).
+void direct_slices(const Problem &r, int ks, DirectPlan *d) {
+  d->kc = ((r.K + ks - 1) / ks + 63) / 64 * 64;
+  d->ks = (int)((r.K + d->kc - 1) / d->kc);
+  if (d->ks > 1 && r.K - (d->ks - 1) * d->kc < 16) --d->ks;
+  d->scratch = d->ks > 1 ? d->ks * r.M * partial_pitch(r.N) * 4 : 0;
+}
+
+// How a problem the vector kernels cannot read as it is runs without copies:
+// decode shapes on the skinny kernel, the rest on 64x64 tiles up to two a CU,
+// else 128x128 tiles; few tiles over a long K (4096, 128x128) or one that
+// saves 20 slices split it as the aligned tiles do. HIP graph per call, before
+// (copies, or the VALU kernel below 3 * 2^24 multiply-adds) and now: 100 x 203
+// x 333 8.3 -> 4.5 us, 1000 x 1001 x 999 + D 19.4 -> 8.7, 2000 x 2001 x 2003 43
+// -> 23, 5857 x 1373 x 435 39 -> 26, 999 x 257 x 9933 100 -> 17.5, 200 x 1001 x
+// 15001 142 -> 20, 16 x 14335 x 4095 43.5 -> 18, 48 x 4095 x 14337 54 -> 26, 8 x
+// 100 x 5001 105 -> 4.7. 64x64 against 128x128: 2487 x 344 x 899 (234 tiles of
+// 64x64) 8.8 and 12.0; 2000 x 2001 x 2003 (1024) 35 and 24.
+DirectPlan direct_plan(const Problem &q) {
+  DirectPlan d;
+  if (q.K < 16 || q.N < 16 || q.batch > 65535 || !mfma_addressable(q) || q.M >= (1ll << 30) ||
+      q.N >= (1ll << 30) || q.K >= (1ll << 30))
+    return d;
+  const Problem r = mfma_fold(q);
+  const double macs = (double)r.M * (double)r.N * (double)r.K * (double)r.batch;
+  // Short K over few outputs: the VALU kernel's one or two rounds of loads.
+  // Large products: the copies cost less than the persistent kernels save.
+  if ((r.K < 128 && macs < 16777216.0) || macs > 2e10) return d;
+  const int64_t t64 = (r.M + 63) / 64 * ((r.N + 63) / 64) * r.batch;
+  const int64_t t128 = (r.M + 127) / 128 * ((r.N + 127) / 128) * r.batch;
+  if (q.M <= 16 || (q.M <= kSkinnyMaxM && q.K >= 1024 && (q.N + 127) / 128 * q.batch < 256)) {
+    d.kind = kDirectSkinny;
+    const SkinnyGeom geo = skinny_geometry<kSkinnyNB, kSkinnyWaves, kSkinnyU>(q, 0);
+    d.ks = geo.ks;
+    d.scratch = geo.ks > 1 ? q.batch * geo.ks * q.M * partial_pitch(q.N) * 4 : 0;
+    return d;
+  }
+  const bool long_k = r.K >= 4096 && r.batch == 1;
+  d.kind = long_k || t64 > 512 ? kDirectTiles128 : kDirectTiles64;
+  const int64_t tiles = d.kind == kDirectTiles128 ? t128 : t64;
+  int ks = 1;
+  if (r.batch == 1) {
+    while (ks < 16 && 2 * ks * tiles <= kSplitCus && r.K / (2 * ks) >= 512) ks *= 2;
+    if (!long_k && (r.K - r.K / ks) / 64 < 20) ks = 1;
+  }
+  direct_slices(r, ks, &d);
+  return d;
+}
+
+// Runs a problem without copies where that is the faster way; *done says
+// whether it was launched. scratch_limit: bytes of scratch the call may take.
+int launch_direct(const Problem &q, int64_t scratch_limit, Scratch &scr, bool *done) {
+  DirectPlan d = direct_plan(q);
+  *done = false;
+  if (d.kind == kDirectNone) return VT_OK;
+  hipStream_t stream = (hipStream_t)scr.stream;
+  const Problem r = mfma_fold(q);
+  *done = true;
+  void *w = nullptr;
+  if (d.scratch > scratch_limit) {
+    d.kind = d.kind == kDirectSkinny ? kDirectTiles64 : d.kind;
+    direct_slices(r, 1, &d);
+  }
+  if (d.kind == kDirectSkinny) {
+    const int rc = launch_skinny_cfg<kSkinnyNB, kSkinnyWaves, kSkinnyU, true>(q, 0, scr);
+    if (rc == VT_OK || d.ks == 1) return rc;
+    // No workspace (none yet on a stream being captured, or no memory): the
+    // tiles need none.
+    (void)hipGetLastError();
+    g_err.clear();
+    d.kind = kDirectTiles64;
+    direct_slices(r, 1, &d);
+  } else if (d.scratch > 0 && scr.take(kPartials, (size_t)d.scratch, &w) != VT_OK) {
+    (void)hipGetLastError();
+    g_err.clear();
+    direct_slices(r, 1, &d);
+  }
+  Problem t = r;
+  if (d.ks > 1) {
+    t.sa = d.kc; t.sb = d.kc * r.ldb; t.D = nullptr; t.sd = 0; t.C = (int32_t *)w;
+    t.ldc = partial_pitch(r.N); t.sc = r.M * t.ldc;
+  }
+  const int cus = scr.st->num_cus;
+  const int rc = d.kind == kDirectTiles64 ? launch_any_tiles<64, 64>(t, d.ks, d.kc, stream, cus)
+                                          : launch_any_tiles<128, 128>(t, d.ks, d.kc, stream, cus);
+  if (rc || d.ks == 1) return rc;
+  ReduceArgs ra;
+  ra.ws = (const int32_t *)w; ra.D = r.D; ra.C = r.C;
+  ra.ldd = r.ldd; ra.ldc = r.ldc; ra.sd = 0; ra.sc = 0;
+  ra.M = (int)r.M; ra.N = (int)r.N; ra.k_split = d.ks;
+  return launch_reduce(ra, 1, stream);
+}
+
 // One validated vt_gemm_i8 problem and the kernel it runs.
 struct GemmCall {
   Problem q;
@@ -3530,6 +3755,13 @@ int prepare_gemm(const int8_t *A, const int8_t *B, const int32_t *D, int32_t *C,
 }
 
 int launch_gemm(const GemmCall &c, Scratch &scr) {
+  if (c.variant == VT_VARIANT_GENERIC || c.variant == VT_VARIANT_PADDED) {
+    // A fixed scratch buffer holds what vt_gemm_check reported for the call.
+    const int64_t limit = scr.fixed ? scratch_need(c.q, c.variant, c.k_split) : INT64_MAX;
+    bool done = false;
+    const int rc = launch_direct(c.q, limit, scr, &done);
+    if (rc || done) return rc;
+  }
   if (c.variant == VT_VARIANT_GENERIC) return launch_generic(c.q, (hipStream_t)scr.stream);
   if (c.variant == VT_VARIANT_PADDED) return launch_padded(c.q, scr);
   return launch_vector(c.q, c.variant, c.k_split, scr);
@@ -3546,6 +3778,14 @@ void set_kernel_attributes(DeviceState &st) {
       {(const void *)skinny_kernel<kSkinnyNB, kSkinnyWaves, kSkinnyU, 4, false>, kMaxSkinnyLds},
       {(const void *)skinny_kernel<kSkinnyNB, kSkinnyWaves, kSkinnyU, 1, true, true>, kMaxSkinnyLds},
       {(const void *)skinny_kernel<kSkinnyNB, kSkinnyWaves, kSkinnyU, 1, false, true>, kMaxSkinnyLds},
+      {(const void *)skinny_kernel<kSkinnyNB, kSkinnyWaves, kSkinnyU, 1, true, false, true>, kMaxSkinnyLds},
+      {(const void *)skinny_kernel<kSkinnyNB, kSkinnyWaves, kSkinnyU, 1, false, false, true>, kMaxSkinnyLds},
+      {(const void *)skinny_kernel<kSkinnyNB, kSkinnyWaves, kSkinnyU, 2, true, false, true>, kMaxSkinnyLds},
+      {(const void *)skinny_kernel<kSkinnyNB, kSkinnyWaves, kSkinnyU, 2, false, false, true>, kMaxSkinnyLds},
+      {(const void *)skinny_kernel<kSkinnyNB, kSkinnyWaves, kSkinnyU, 4, true, false, true>, kMaxSkinnyLds},
+      {(const void *)skinny_kernel<kSkinnyNB, kSkinnyWaves, kSkinnyU, 4, false, false, true>, kMaxSkinnyLds},
+      {(const void *)skinny_kernel<kSkinnyNB, kSkinnyWaves, kSkinnyU, 1, true, true, true>, kMaxSkinnyLds},
+      {(const void *)skinny_kernel<kSkinnyNB, kSkinnyWaves, kSkinnyU, 1, false, true, true>, kMaxSkinnyLds},
       {(const void *)replay_kernel, kMaxReplayLds + 256},
   };
   for (const auto &n : need) {

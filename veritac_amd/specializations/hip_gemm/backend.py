@@ -709,7 +709,8 @@ def modeled_counts(plan):
 def _padded_copy_bytes(plan, inner):
     """Bytes the padded variant moves besides its inner product: each copied
     operand read and its padded copy written, and, when C is copied out, C'
-    read back and C written (plus D)."""
+    read back and C written (plus D). The library reads the operands in place
+    where that is faster, so this is the most it moves."""
     m, n, k, b = plan["m"], plan["n"], plan["k"], plan["batch"]
     n_p, k_p = inner["n"], inner["k"]
     b_mats = 1 if plan["b_shared"] or b == 1 else b
