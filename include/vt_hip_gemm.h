@@ -108,8 +108,9 @@ extern "C" {
  * place (N, K >= 16 and rows the MFMA variants can address); for large
  * products VT_VARIANT_PADDED copies the operands the vector variants cannot
  * read, zero padded, to a workspace the library allocates once per (device,
- * stream) and grows as needed. vt_gemm_check reports the most it takes. For
- * aligned
+ * stream) and grows as needed, and writes C directly (without a workspace, as
+ * on a stream captured before it has one, it reads them in place).
+ * vt_gemm_check reports what copies of all three would take. For aligned
  * shapes VT_VARIANT_AUTO picks VT_VARIANT_SKINNY for M <= 16, and for
  * M <= 64 when K >= 512 and ceil(N / 128) * batch < 256 (the skinny kernel
  * runs 1, 2 or 4 row blocks of 16 over one stream of B), VT_VARIANT_GENERIC when K <= 64 and

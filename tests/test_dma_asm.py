@@ -225,3 +225,24 @@ def test_fence_check_catches_missing_nops():
     assert fence_violations(["v_accvgpr_write_b32 a0, v1"] + [other] * 3 + [mf]) != []
     assert fence_violations([mf] + [other] * 8 + ["v_accvgpr_read_b32 v0, a2"]) == []
     assert fence_violations([mf] + [other] * 2 + ["v_accvgpr_read_b32 v0, a2"]) != []
+
+
+@pytest.mark.parametrize("has_d", [0, 1])
+def test_ragged_dma16_kernel_keeps_the_same_discipline(asm, has_d):
+    """gemm_dma16_ragged_kernel<HAS_D> (rows of C and D of any length): the
+    DMA sequences, slice waits and MFMA fences of the edge kinds, no spills."""
+    name = "_ZN12_GLOBAL__N_124gemm_dma16_ragged_kernelILb%dEEEvNS_8GemmArgsE" % has_d
+    body = instructions(asm, name)
+    at = [i for i, l in enumerate(body) if re.search(r"\bm0\b", l)]
+    assert len(at) == (3 + 4) * 8
+    for i in at:
+        assert body[i].startswith("s_mov_b32 m0, s") and body[i + 1].startswith("s_nop 0")
+        assert body[i + 2].startswith("global_load_lds_dwordx4")
+    mfma = [i for i, l in enumerate(body) if l.startswith("v_mfma")]
+    assert len(mfma) == 4 * 64
+    loop = body[mfma[0]:mfma[-1] + 1]
+    assert not [l for l in loop if re.match(r"s_waitcnt .*vmcnt\(0\)", l)]
+    waits = [body[i - 1] for i in range(mfma[0], mfma[-1] + 8) if body[i] == "s_barrier"]
+    assert waits == ["s_waitcnt vmcnt(8)"] * 4
+    assert fence_violations(body) == []
+    assert not [l for l in body if l.startswith("scratch_")]

@@ -52,7 +52,9 @@
 //   generic_kernel  any shape, stride or alignment; one thread per output,
 //       int32 VALU. Used for tiny products, and where N or K is below 16.
 //   Operands off the 16-byte grid (odd N, K, pitches or addresses) are read in
-//       place by gemm_mfma_kernel<.., EDGE 3> and skinny_kernel<.., ANY>.
+//       place by gemm_mfma_kernel<.., EDGE 3> and skinny_kernel<.., ANY>, or
+//       for large products padded once and multiplied by
+//       gemm_dma16_ragged_kernel, which stores C at any alignment.
 //
 // Tails: rows of A past M and columns of B past N are read from clamped (valid)
 // addresses and their outputs are never stored; k past K reads A as zero, so
@@ -271,7 +273,8 @@ struct GemmArgs {
   int M, N, K;
   int tiles_m, tiles_n, group_m;
   int batch_count;   // batches (the persistent kernel walks all their tiles)
-  int k_last;        // EDGE 3: K of the last batch (K slices run as batches)
+  int k_last;        // gemm_mfma_kernel EDGE 3: K of the last batch (K slices run as batches)
+  int n_valid;       // gemm_dma16_ragged_kernel: columns of C and D
 };
 
 // EDGE: 0 full tiles; 1 M or N not a multiple of the tile (clamped source
@@ -1009,12 +1012,16 @@ __device__ __forceinline__ StripLanes strip_lanes(int lane, int strip_base, int6
 // One 16-row strip of store_tile16_lds: Cs / Ds point at the strip's first
 // row and the wave's first column. MASKED: store j of a lane writes only when
 // row_rel + 2 j >= 0 and col_ok (a moved-back tile leaves the rows and
-// columns it shares with its neighbour to the neighbour).
-template <int NI, bool HAS_D, bool MASKED = false>
+// columns it shares with its neighbour to the neighbour). RAGGED: rows of C
+// and D are 4-byte aligned and the lane's 4 columns end `valid` columns before
+// the matrix does (below 4: only that many are its own; D is then read from
+// the row's last 4 and moved into place, so nothing past a row is read).
+template <int NI, bool HAS_D, bool MASKED = false, bool RAGGED = false>
 __device__ __forceinline__ void store_strip16_lds(const v4i (&acc)[NI], int32_t *Cs,
                                                   const int32_t *Ds, int64_t ldc, int64_t ldd,
                                                   const StripLanes &sl, LDS_AS int8_t *lds,
-                                                  int row_rel = 0, bool col_ok = true) {
+                                                  int row_rel = 0, bool col_ok = true,
+                                                  int valid = 4) {
   static_assert(NI * 16 == 128, "two 512-byte rows per wave instruction");
 #pragma unroll
   for (int ni = 0; ni < NI; ++ni)
@@ -1026,9 +1033,20 @@ __device__ __forceinline__ void store_strip16_lds(const v4i (&acc)[NI], int32_t 
   for (int j = 0; j < 8; ++j) v[j] = *(LDS_AS v4i *)(lds + sl.rb[j >> 1] + j * 1024);
   if constexpr (HAS_D) {
     v4i d[8];
+    if constexpr (RAGGED) {
+      const int back = max(4 - valid, 0);
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      d[j] = *(const v4i *)((const int8_t *)(Ds + 2 * j * ldd) + sl.gofs_d);
+      for (int j = 0; j < 8; ++j)
+        d[j] = *(const v4i_any *)((const int8_t *)(Ds + 2 * j * ldd - back) + sl.gofs_d);
+      if (back) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) d[j] = drop_bytes(d[j], min(4 * back, 16));
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        d[j] = *(const v4i *)((const int8_t *)(Ds + 2 * j * ldd) + sl.gofs_d);
+    }
 #pragma unroll
     for (int j = 0; j < 8; ++j)
 #pragma unroll
@@ -1042,6 +1060,21 @@ __device__ __forceinline__ void store_strip16_lds(const v4i (&acc)[NI], int32_t 
       for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(v[j]));
     }
   }
+  if constexpr (RAGGED) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (col_ok && row_rel + 2 * j >= 0) {
+        int32_t *c = (int32_t *)((int8_t *)(Cs + 2 * j * ldc) + sl.gofs_c);
+        if (valid >= 4) {
+          __builtin_nontemporal_store(v[j], (v4i_any *)c);
+        } else {
+#pragma unroll
+          for (int t = 0; t < 3; ++t)
+            if (t < valid) c[t] = v[j][t];
+        }
+      }
+    return;
+  }
 #pragma unroll
   for (int j = 0; j < 8; ++j)
     if (!MASKED || (col_ok && row_rel + 2 * j >= 0))
@@ -1050,16 +1083,17 @@ __device__ __forceinline__ void store_strip16_lds(const v4i (&acc)[NI], int32_t 
 
 // row_rel0: the lane's row in the wave's first strip (2 j + lane / 32 for
 // store j) less the rows the tile leaves to its neighbour (MASKED).
-template <int MI, int NI, bool HAS_D, int FIRST = 0, bool MASKED = false>
+template <int MI, int NI, bool HAS_D, int FIRST = 0, bool MASKED = false, bool RAGGED = false>
 __device__ __forceinline__ void store_tile16_lds(const v4i (&acc)[MI][NI], int32_t *Cb,
                                                  const int32_t *Db, int64_t ldc, int64_t ldd,
                                                  const StripLanes &sl, LDS_AS int8_t *lds,
-                                                 int row_rel0 = 0, bool col_ok = true) {
+                                                 int row_rel0 = 0, bool col_ok = true,
+                                                 int valid = 4) {
 #pragma unroll
   for (int mi = FIRST; mi < MI; ++mi) {
-    store_strip16_lds<NI, HAS_D, MASKED>(acc[mi], Cb + mi * 16 * ldc,
+    store_strip16_lds<NI, HAS_D, MASKED, RAGGED>(acc[mi], Cb + mi * 16 * ldc,
                                          HAS_D ? Db + mi * 16 * ldd : nullptr, ldc, ldd, sl, lds,
-                                         row_rel0 + mi * 16, col_ok);
+                                         row_rel0 + mi * 16, col_ok, valid);
     __builtin_amdgcn_sched_barrier(0);
   }
 }
@@ -1137,8 +1171,12 @@ __device__ __forceinline__ void mfma16_in_place(v4i &acc, const v4i &a, const v4
 // step gs + 1; its reads were issued in step gs - 1 and consumed by step gs's
 // MFMAs. The 256x128 form (BN = 128) runs the same schedule over 32 slots,
 // with 6 DMAs per slice issued one every 4 slots.
-template <bool HAS_D, bool PACKED_B, bool EDGE = false, int BN = 256>
-__global__ __launch_bounds__(256, 1) void gemm_dma16_kernel(GemmArgs p) {
+// RAGGED (with EDGE; the 256x256 form, row-major B): rows of C and D have
+// n_valid <= N columns at any 4-byte aligned address (A and B are padded
+// copies there).
+template <bool HAS_D, bool PACKED_B, bool EDGE, int BN, bool RAGGED>
+__device__ __forceinline__ void dma16_tiles(const GemmArgs &p) {
+  static_assert(!RAGGED || (EDGE && BN == 256 && !PACKED_B), "ragged rows: 256x256 edge tiles, row-major B");
   // BN = 128 (the 256x128 form) gives each wave a 128x64 block and half the
   // B slice; the rest is shared.
   static_assert(BN == 256 || BN == 128, "256x256 or 256x128 tiles");
@@ -1427,11 +1465,12 @@ __global__ __launch_bounds__(256, 1) void gemm_dma16_kernel(GemmArgs p) {
     // Rows [m0, mn) and columns [n0, nn) of a moved-back tile are its
     // neighbour's to store (0 unless EDGE).
     if constexpr (BN == 256) {
-      store_tile16_lds<MI, NI, HAS_D, HAS_D || EDGE ? 0 : EARLY_STRIPS, EDGE>(
+      store_tile16_lds<MI, NI, HAS_D, HAS_D || EDGE ? 0 : EARLY_STRIPS, EDGE, RAGGED>(
           acc, c_tile,
           HAS_D ? p.D + bidx * p.sd + (int64_t)(m0 + wm * WTM) * p.ldd + n0 + wn * WTN : nullptr,
           p.ldc, p.ldd, sl, lds, wm * WTM + (lane >> 5) - (mn - m0),
-          wn * WTN + (lane & 31) * 4 >= nn - n0);
+          wn * WTN + (lane & 31) * 4 >= nn - n0,
+          RAGGED ? p.n_valid - (n0 + wn * WTN + (lane & 31) * 4) : 4);
     } else {
       const int32_t *d_tile =
           HAS_D ? p.D + bidx * p.sd + (int64_t)(m0 + wm * WTM) * p.ldd + n0 + wn * WTN : nullptr;
@@ -1451,6 +1490,16 @@ __global__ __launch_bounds__(256, 1) void gemm_dma16_kernel(GemmArgs p) {
     zero_acc();
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+template <bool HAS_D, bool PACKED_B, bool EDGE = false, int BN = 256>
+__global__ __launch_bounds__(256, 1) void gemm_dma16_kernel(GemmArgs p) {
+  dma16_tiles<HAS_D, PACKED_B, EDGE, BN, false>(p);
+}
+
+template <bool HAS_D>
+__global__ __launch_bounds__(256, 1) void gemm_dma16_ragged_kernel(GemmArgs p) {
+  dma16_tiles<HAS_D, false, true, 256, true>(p);
 }
 
 // ---------------------------------------------------------------------------
@@ -3491,6 +3540,26 @@ int64_t scratch_need(const Problem &q, int32_t variant, int32_t k_split) {
   return L.a_bytes + L.b_bytes + L.c_bytes + scratch_need(g, v, ks);
 }
 
+// Zero-padded copies of A (bA matrices) and B (bB) with K and N rounded up to
+// Kp and Np; a null destination is not copied.
+int launch_pad_copies(const Problem &q, int64_t Kp, int64_t Np, int8_t *Ap, int8_t *Bp, int64_t bA,
+                      int64_t bB, hipStream_t s) {
+  const PadArgs pa = {q.A, Ap, q.lda, bA > 1 ? q.sa : 0, q.M * Kp, q.M, q.K, q.M, Kp, bA};
+  const PadArgs pb = {q.B, Bp, q.ldb, bB > 1 ? q.sb : 0, Kp * Np, q.K, q.N, Kp, Np, bB};
+  // grid z = the operands copied; z = 0 takes the first of them
+  const int64_t blocks_a = Ap ? (q.M * (Kp / 16) + 255) / 256 : 0;
+  const int64_t blocks_b = Bp ? (Kp * (Np / 16) + 255) / 256 : 0;
+  const int64_t blocks = blocks_a > blocks_b ? blocks_a : blocks_b;
+  const int64_t ys = (Ap && bA > bB) || !Bp ? bA : bB;
+  if (blocks > 0x7fffffff) return fail(VT_EUNSUPPORTED, "padded copy grid too large");
+  if (blocks > 0) {
+    hipLaunchKernelGGL(pad_i8_kernel, dim3((unsigned)blocks, (unsigned)ys, Ap && Bp ? 2 : 1),
+                       dim3(256), 0, s, Ap ? pa : pb, pb);
+    VT_HIP_CHECK(hipGetLastError());
+  }
+  return VT_OK;
+}
+
 int launch_padded(const Problem &q, Scratch &scr) {
   if (!padded_fits(q))
     return fail(VT_EUNSUPPORTED, "padded path needs K > 0, M, N+15, K+15 < 2^30, batch <= 65535");
@@ -3506,19 +3575,8 @@ int launch_padded(const Problem &q, Scratch &scr) {
     if (rc) return rc;
     int8_t *Ap = (int8_t *)w, *Bp = Ap + a_bytes;
     int32_t *Cp = (int32_t *)(Bp + b_bytes);
-    const PadArgs pa = {q.A, Ap, q.lda, bA > 1 ? q.sa : 0, q.M * Kp, q.M, q.K, q.M, Kp, bA};
-    const PadArgs pb = {q.B, Bp, q.ldb, bB > 1 ? q.sb : 0, Kp * Np, q.K, q.N, Kp, Np, bB};
-    // grid z = the operands copied; z = 0 takes the first of them
-    const int64_t blocks_a = copy_a ? (q.M * (Kp / 16) + 255) / 256 : 0;
-    const int64_t blocks_b = copy_b ? (Kp * (Np / 16) + 255) / 256 : 0;
-    const int64_t blocks = blocks_a > blocks_b ? blocks_a : blocks_b;
-    const int64_t ys = (copy_a && bA > bB) || !copy_b ? bA : bB;
-    if (blocks > 0x7fffffff) return fail(VT_EUNSUPPORTED, "padded copy grid too large");
-    if (blocks > 0) {
-      hipLaunchKernelGGL(pad_i8_kernel, dim3((unsigned)blocks, (unsigned)ys, copy_a && copy_b ? 2 : 1),
-                         dim3(256), 0, s, copy_a ? pa : pb, pb);
-      VT_HIP_CHECK(hipGetLastError());
-    }
+    rc = launch_pad_copies(q, Kp, Np, copy_a ? Ap : nullptr, copy_b ? Bp : nullptr, bA, bB, s);
+    if (rc) return rc;
     g = padded_inner(q, L, Ap, Bp, Cp);
   } else {
     g = padded_inner(q, L, nullptr, nullptr, nullptr);
@@ -3588,6 +3646,73 @@ void direct_slices(const Problem &r, int ks, DirectPlan *d) {
   d->scratch = d->ks > 1 ? d->ks * r.M * partial_pitch(r.N) * 4 : 0;
 }
 
+// Whether a large problem the vector kernels cannot read as it is runs on the
+// persistent 256x256 kernel over padded copies of A and B (K rounded up to
+// 256, N to 16), which stores C (and adds D) in place at any alignment.
+// Estimates in ns: its slices (0.6 us each, 0.85 with every CU busy), the
+// copies at 4.5 TB/s, their launch and C at 5 TB/s, against the 128x128 tiles
+// that read the operands in place (a slice 0.2 us and 0.56 more per tile and
+// CU). HIP graph per call, both ways: 3000 x 3001 x 3003 75 us in place, 50
+// over copies; 4000 x 4001 x 4001 140 and 81; 8000 x 8001 x 2001 280 and 161;
+// 5857 x 2373 x 1435 63 and 46.
+struct LargeLayout {
+  int64_t Kp, Np, a_bytes, b_bytes;
+  bool copy_a, copy_b;
+};
+
+bool large_padded(const Problem &r, LargeLayout *L) {
+  if (r.M < 256 || r.N < 256 || r.K < 256 || r.ldc >= (1ll << 29) || (r.D && r.ldd >= (1ll << 29)) ||
+      r.batch > 65535)
+    return false;
+  auto round256 = [](int64_t v) { return (v + 255) / 256 * 256; };
+  L->Kp = round256(r.K);
+  L->Np = (r.N + 15) / 16 * 16;
+  L->copy_a = L->Kp != r.K || r.lda % 16 || r.sa % 16 || !aligned16(r.A);
+  L->copy_b = L->Kp != r.K || L->Np != r.N || r.ldb % 16 || r.sb % 16 || !aligned16(r.B);
+  const int64_t bA = r.batch > 1 && r.sa == 0 ? 1 : r.batch, bB = r.batch > 1 && r.sb == 0 ? 1 : r.batch;
+  L->a_bytes = L->copy_a ? round256(bA * r.M * L->Kp) : 0;
+  L->b_bytes = L->copy_b ? round256(bB * L->Kp * L->Np) : 0;
+  if (256 * L->Kp >= (1ll << 32) - 4096 || 64 * L->Np >= (1ll << 32) - 4096) return false;
+  const int64_t tiles = (r.M + 255) / 256 * ((r.N + 255) / 256) * r.batch;
+  if (tiles > 0x7fffffff) return false;
+  const double busy = (double)(tiles < kSplitCus ? tiles : kSplitCus) / kSplitCus;
+  const double rounds = (double)((tiles + kSplitCus - 1) / kSplitCus);
+  const double padded = rounds * (double)(L->Kp / 64) * (600.0 + 250.0 * busy) +
+                        2.0 * (double)(L->a_bytes + L->b_bytes) / 4500.0 + 6000.0 +
+                        4.0 * (double)r.M * (double)r.N * (double)r.batch / 5000.0;
+  const double per_cu = (double)((r.M + 127) / 128) * (double)((r.N + 127) / 128) * (double)r.batch / kSplitCus;
+  const double direct = (double)((r.K + 63) / 64) * (200.0 + 560.0 * (per_cu < 0.4 ? 0.4 : per_cu)) + 4000.0;
+  return padded < direct;
+}
+
+int launch_large_padded(const Problem &r, const LargeLayout &L, int8_t *w, hipStream_t s, int num_cus) {
+  int8_t *Ap = w, *Bp = w + L.a_bytes;
+  const int64_t bA = r.batch > 1 && r.sa == 0 ? 1 : r.batch, bB = r.batch > 1 && r.sb == 0 ? 1 : r.batch;
+  int rc = launch_pad_copies(r, L.Kp, L.Np, L.copy_a ? Ap : nullptr, L.copy_b ? Bp : nullptr, bA, bB, s);
+  if (rc) return rc;
+  GemmArgs a;
+  a.A = L.copy_a ? Ap : r.A;
+  a.lda = L.copy_a ? L.Kp : r.lda;
+  a.sa = L.copy_a ? (bA > 1 ? r.M * L.Kp : 0) : r.sa;
+  a.B = L.copy_b ? Bp : r.B;
+  a.ldb = L.copy_b ? L.Np : r.ldb;
+  a.sb = L.copy_b ? (bB > 1 ? L.Kp * L.Np : 0) : r.sb;
+  a.C = r.C; a.D = r.D; a.ldc = r.ldc; a.ldd = r.ldd; a.sc = r.sc; a.sd = r.sd;
+  a.M = (int)r.M; a.N = (int)L.Np; a.K = (int)L.Kp;
+  a.n_valid = (int)r.N;
+  a.k_last = a.K;
+  a.tiles_m = (a.M + 255) / 256;
+  a.tiles_n = (a.N + 255) / 256;
+  a.group_m = 4;
+  a.batch_count = (int)r.batch;
+  const int64_t blocks = (int64_t)a.tiles_m * a.tiles_n * r.batch;
+  const dim3 grid((unsigned)(blocks < num_cus ? blocks : num_cus));
+  if (r.D) hipLaunchKernelGGL(gemm_dma16_ragged_kernel<true>, grid, dim3(256), 0, s, a);
+  else hipLaunchKernelGGL(gemm_dma16_ragged_kernel<false>, grid, dim3(256), 0, s, a);
+  VT_HIP_CHECK(hipGetLastError());
+  return VT_OK;
+}
+
 // How a problem the vector kernels cannot read as it is runs without copies:
 // decode shapes on the skinny kernel, the rest on 64x64 tiles up to two a CU,
 // else 128x128 tiles; few tiles over a long K (4096, 128x128) or one that
@@ -3605,9 +3730,9 @@ DirectPlan direct_plan(const Problem &q) {
     return d;
   const Problem r = mfma_fold(q);
   const double macs = (double)r.M * (double)r.N * (double)r.K * (double)r.batch;
-  // Short K over few outputs: the VALU kernel's one or two rounds of loads.
-  // Large products: the copies cost less than the persistent kernels save.
-  if ((r.K < 128 && macs < 16777216.0) || macs > 2e10) return d;
+  // Short K over few outputs: the VALU kernel's few rounds of loads (64 x 60 x
+  // 64 2.6 us, 200 x 500 x 70 4.2; 200 x 200 x 128 4.6 against 3.4 on tiles).
+  if (r.K < 128 && macs < 16777216.0) return d;
   const int64_t t64 = (r.M + 63) / 64 * ((r.N + 63) / 64) * r.batch;
   const int64_t t128 = (r.M + 127) / 128 * ((r.N + 127) / 128) * r.batch;
   if (q.M <= 16 || (q.M <= kSkinnyMaxM && q.K >= 1024 && (q.N + 127) / 128 * q.batch < 256)) {
@@ -3639,6 +3764,14 @@ int launch_direct(const Problem &q, int64_t scratch_limit, Scratch &scr, bool *d
   const Problem r = mfma_fold(q);
   *done = true;
   void *w = nullptr;
+  LargeLayout L;
+  if (d.kind != kDirectSkinny && d.ks == 1 && large_padded(r, &L) && L.a_bytes + L.b_bytes <= scratch_limit) {
+    if (L.a_bytes + L.b_bytes == 0 ||
+        scr.take(kPadded, (size_t)(L.a_bytes + L.b_bytes), &w) == VT_OK)
+      return launch_large_padded(r, L, (int8_t *)w, stream, scr.st->num_cus);
+    (void)hipGetLastError();
+    g_err.clear();
+  }
   if (d.scratch > scratch_limit) {
     d.kind = d.kind == kDirectSkinny ? kDirectTiles64 : d.kind;
     direct_slices(r, 1, &d);
