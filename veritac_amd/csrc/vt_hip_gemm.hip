@@ -2318,6 +2318,15 @@ std::map<int, DeviceState> g_dev;
 void set_kernel_attributes(DeviceState &st);
 
 int current_device(int *dev_out, DeviceState **st_out) {
+  // The device this thread last found usable (its state is never freed).
+  static thread_local int last_dev = -1;
+  static thread_local DeviceState *last_st = nullptr;
+  int now = -1;
+  if (last_dev >= 0 && hipGetDevice(&now) == hipSuccess && now == last_dev) {
+    *dev_out = last_dev;
+    *st_out = last_st;
+    return VT_OK;
+  }
   int count = 0;
   if (hipGetDeviceCount(&count) != hipSuccess || count <= 0)
     return fail(VT_ENODEV, "no HIP device available");
@@ -2348,6 +2357,8 @@ int current_device(int *dev_out, DeviceState **st_out) {
   if (st.attr_err != hipSuccess)
     return fail(VT_EHIP, "hipFuncSetAttribute (dynamic LDS) failed on device %d: %s", dev,
                 hipGetErrorString(st.attr_err));
+  last_dev = dev;
+  last_st = &st;
   *dev_out = dev;
   *st_out = &st;
   return VT_OK;

@@ -32,6 +32,7 @@ from __future__ import annotations
 
 import hashlib
 import math
+import operator
 
 from ... import _lib
 from ..._lib import HipGemmError
@@ -924,9 +925,57 @@ def optimize(m, n, k, *, batch=1, b_shared=False, has_d=False, d_max_abs=0,
 # Execution
 # ---------------------------------------------------------------------------
 
+_torch_module = None
+
+
 def _torch():
-    import torch
-    return torch
+    global _torch_module
+    if _torch_module is None:
+        import torch
+        _torch_module = torch
+    return _torch_module
+
+
+_plan_values = operator.itemgetter("m", "n", "k", "batch", "dim", "b_shared", "has_d", "d_max_abs",
+                                   "variant", "k_split")
+_PLAN_TYPES = (int, int, int, int, int, bool, bool, int, str, int)
+_valid_plans = set()       # values of plans validate_plan has accepted
+_VALID_PLANS_MAX = 4096
+
+
+def _require_valid(plan):
+    """Raise HipGemmError unless validate_plan accepts the plan. Its verdict
+    depends on the plan's values alone, so accepted values (of exactly the
+    schema's types) are remembered: checking them again took a third of a
+    padded plan's call."""
+    values = None
+    if type(plan) is dict:
+        try:
+            values = _plan_values(plan)
+            if tuple(map(type, values)) != _PLAN_TYPES:
+                values = None
+            elif values in _valid_plans:
+                return
+        except KeyError:
+            pass
+    ok, reason = validate_plan(plan)
+    if not ok:
+        raise HipGemmError("invalid plan: " + reason)
+    if values is not None:
+        if len(_valid_plans) >= _VALID_PLANS_MAX:
+            _valid_plans.clear()
+        _valid_plans.add(values)
+
+
+def _current_stream(device):
+    """Raw handle of torch's current stream on a GPU (without the Stream object
+    and the device guard of the public call, 3 us of a 12 us call)."""
+    torch = _torch()
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is not None and device.index is not None:
+        return raw(device.index)
+    with torch.cuda.device(device):
+        return torch.cuda.current_stream(device).cuda_stream
 
 
 def _operand_shapes(plan):
@@ -943,7 +992,7 @@ def _check_tensor(name, t, shape, dtype, device):
         raise HipGemmError("%s must be a torch tensor" % name)
     if t.dtype != dtype:
         raise HipGemmError("%s must be %s (got %s)" % (name, dtype, t.dtype))
-    if tuple(t.shape) != tuple(shape):
+    if t.shape != shape:
         raise HipGemmError("%s has shape %s, plan needs %s" % (name, tuple(t.shape), tuple(shape)))
     if t.device != device:
         raise HipGemmError("%s is on %s, expected %s" % (name, t.device, device))
@@ -1010,8 +1059,7 @@ def pack_b(B, *, out=None, stream=None):
             raise HipGemmError("out.data must be a contiguous int8 tensor of %d bytes on %s"
                                % (batch * size, B.device))
     if stream is None:
-        with torch.cuda.device(B.device):
-            stream = torch.cuda.current_stream(B.device).cuda_stream
+        stream = _current_stream(B.device)
     elif out is None:
         _keep_for_stream(data, stream)
     _lib.pack_b_raw(B.data_ptr(), data.data_ptr(), k, n, B.stride(-2), batch,
@@ -1085,9 +1133,7 @@ def run(plan, A, B, D=None, *, out=None, stream=None, runner=None):
     orders the operands' producers before it, as with any raw stream; a C
     allocated here is recorded as used on that stream.
     """
-    ok, reason = validate_plan(plan)
-    if not ok:
-        raise HipGemmError("invalid plan: " + reason)
+    _require_valid(plan)
     torch = _torch()
     if not isinstance(A, torch.Tensor):
         raise HipGemmError("A must be a torch tensor")
@@ -1118,8 +1164,7 @@ def run(plan, A, B, D=None, *, out=None, stream=None, runner=None):
                                "no CPU path" % device)
         runner = native_runner
         if stream is None:
-            with torch.cuda.device(device):
-                stream = torch.cuda.current_stream(device).cuda_stream
+            stream = _current_stream(device)
         elif allocated:
             _keep_for_stream(out, stream)
     runner(plan, A, B, D, out, stream)
