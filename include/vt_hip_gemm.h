@@ -135,8 +135,11 @@ extern "C" {
  * the stream is being captured: a call that needs more workspace than its
  * stream has returns VT_EUNSUPPORTED during capture, so make the same calls
  * once on the stream before capturing (vt_gemm_check reports the bytes a
- * call takes from vt_gemm_i8_noalloc's array, which bounds what it takes
- * from a stream's workspaces). Graphs captured on one stream use that
+ * call takes from vt_gemm_i8_noalloc's array, which bounds what it needs
+ * from a stream's workspaces). Outside capture a call may also use workspaces
+ * it does not need where that is faster: K slices of the generic and packed
+ * paths, and padded copies (at most 256 MiB) for large products whose K is
+ * not a multiple of 64. Graphs captured on one stream use that
  * stream's workspaces: replay them in order on that stream (or with the same
  * ordering against it), never two at once. Overlapping launches on one
  * workspace race, and racing finishing words can stay nonzero and spoil the
@@ -400,8 +403,8 @@ int vt_pack_b_i8(const int8_t *B, int8_t *Bp, int64_t K, int64_t N, int64_t ldb,
  * k_split: workgroups along K for the groups of up to 64 rows (0 =
  * automatic: a split when even half-block groups are too few, or when narrow
  * groups over a long K would read A for longer than a split of two or four
- * over wider groups takes to sum (not needed: such a call runs unsplit when
- * its stream is captured before it has a workspace). The partial sums are
+ * over wider groups takes to sum (not while the stream is captured). The
+ * partial sums are
  * finished in the kernel up to 16 rows, through the finishing words described
  * under Workspace, or added by a second kernel);
  * the tile kernels choose their own.

@@ -114,10 +114,20 @@ def test_large_products_store_c_in_place(dev, case):
     check(dev, "padded", **case)
 
 
+# aligned rows with K off 64, where copies for the persistent kernel pay: whole
+# and ragged tiles, D, batches; the last one below the size stays on the tiles
+@pytest.mark.parametrize("case", [
+    dict(m=3000, n=3008, k=3024), dict(m=3072, n=3088, k=2832, ldc=3090), dict(m=2048, n=2064, k=4112),
+    dict(m=900, n=2000, k=2320, batch=4), dict(m=900, n=2000, k=2320, batch=4, shared=True),
+    dict(m=500, n=528, k=1040)])
+def test_large_aligned_products_with_k_off_64(dev, case):
+    check(dev, "auto", **case)
+
+
 def test_a_cold_capture_runs_without_a_workspace(dev):
     """The K slices' and copies' workspaces are not needed: a stream captured
     before it has any runs the same product without them."""
-    for m, n, k in ((300, 300, 3001), (16, 1001, 4095), (3000, 3001, 2050)):
+    for m, n, k in ((300, 300, 3001), (16, 1001, 4095), (3000, 3001, 2050), (3000, 3008, 3024), (9, 500, 5001)):
         say("cold capture", m, n, k)
         plan = hg.make_plan(m, n, k)
         A = torch.randint(-128, 128, (m, k), dtype=torch.int8, device=dev)

@@ -2407,6 +2407,7 @@ struct Scratch {
   void *stream = nullptr;
   int8_t *fixed = nullptr;   // device address of `scratch`, or null
   size_t used = 0;
+  bool copies_taken = false;   // the call holds padded copies in the kPadded workspace
 
   int take(ScratchKind kind, size_t bytes, void **out) {
     if (!fixed) return get_workspace(st, stream, kind, bytes, out);
@@ -2420,6 +2421,15 @@ struct Scratch {
     return VT_OK;
   }
 };
+
+// Whether a call may use a workspace it could do without. Not while its stream
+// is captured: a graph of calls that need no workspace may be replayed on any
+// stream, beside others captured on the same one.
+bool optional_workspace(const Scratch &scr) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  return !scr.fixed && hipStreamIsCapturing((hipStream_t)scr.stream, &cs) == hipSuccess &&
+         cs == hipStreamCaptureStatusNone;
+}
 
 bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
 
@@ -3304,8 +3314,9 @@ int launch_packed_rows(const Problem &q, int k_split, Scratch &scr, bool a_split
   a.kbt = (int)packed_kbt(q.K);
   const int cus = scr.st->num_cus;
   const PackedGeom base = packed_geometry(q.M, q.N, q.K, q.batch, false, cus);
-  const PackedGeom geo = k_split > 0 ? PackedGeom{base.hpw, k_split}
-                                     : packed_geometry(q.M, q.N, q.K, q.batch, a_split, cus);
+  PackedGeom geo = k_split > 0 ? PackedGeom{base.hpw, k_split}
+                               : packed_geometry(q.M, q.N, q.K, q.batch, a_split, cus);
+  if (k_split == 0 && geo.ks != base.ks && !optional_workspace(scr)) geo = base;
   a.hpw = geo.hpw;
   a.groups = (int)((2 * (q.N / 16) + a.hpw - 1) / a.hpw);
   a.kb_per_split = (a.kbt + geo.ks - 1) / geo.ks;
@@ -3323,8 +3334,8 @@ int launch_packed_rows(const Problem &q, int k_split, Scratch &scr, bool a_split
     const size_t bytes = fin ? (size_t)q.batch * ((q.M + 1) / 2) * q.N * sizeof(uint64_t)
                              : (size_t)q.batch * a.k_split * q.M * q.N * sizeof(int32_t);
     if (int rc = scr.take(fin ? kFinWords : kPartials, bytes, &w)) {
-      // A split only to read less of A is not needed: without a workspace
-      // (none yet on a stream being captured, or no memory) run unsplit.
+      // A split only to read less of A is not needed: with no memory for its
+      // workspace run unsplit.
       if (k_split > 0 || base.ks == geo.ks) return rc;
       (void)hipGetLastError();
       g_err.clear();
@@ -3584,6 +3595,7 @@ int launch_padded(const Problem &q, Scratch &scr) {
     void *w = nullptr;
     int rc = scr.take(kPadded, (size_t)(a_bytes + b_bytes + c_bytes), &w);
     if (rc) return rc;
+    scr.copies_taken = true;   // the inner product may not take that workspace again
     int8_t *Ap = (int8_t *)w, *Bp = Ap + a_bytes;
     int32_t *Cp = (int32_t *)(Bp + b_bytes);
     rc = launch_pad_copies(q, Kp, Np, copy_a ? Ap : nullptr, copy_b ? Bp : nullptr, bA, bB, s);
@@ -3624,8 +3636,15 @@ int launch_generic(const Problem &q, hipStream_t stream) {
 }
 
 
+int launch_large_aligned(const Problem &q, Scratch &scr, bool *done);
+
 // The vector variants (operands already checked by vector_ok).
 int launch_vector(const Problem &q, int32_t variant, int32_t k_split, Scratch &scr) {
+  if (variant != VT_VARIANT_SKINNY && q.K % 64) {
+    bool done = false;
+    const int rc = launch_large_aligned(q, scr, &done);
+    if (rc || done) return rc;
+  }
   switch (variant) {
     case VT_VARIANT_MFMA_256x256: return launch_mfma<256, 256>(q, scr);
     case VT_VARIANT_MFMA_128x128: return launch_mfma128(q, scr);
@@ -3657,21 +3676,25 @@ void direct_slices(const Problem &r, int ks, DirectPlan *d) {
   d->scratch = d->ks > 1 ? d->ks * r.M * partial_pitch(r.N) * 4 : 0;
 }
 
-// Whether a large problem the vector kernels cannot read as it is runs on the
-// persistent 256x256 kernel over padded copies of A and B (K rounded up to
-// 256, N to 16), which stores C (and adds D) in place at any alignment.
-// Estimates in ns: its slices (0.6 us each, 0.85 with every CU busy), the
-// copies at 4.5 TB/s, their launch and C at 5 TB/s, against the 128x128 tiles
-// that read the operands in place (a slice 0.2 us and 0.56 more per tile and
-// CU). HIP graph per call, both ways: 3000 x 3001 x 3003 75 us in place, 50
-// over copies; 4000 x 4001 x 4001 140 and 81; 8000 x 8001 x 2001 280 and 161;
-// 5857 x 2373 x 1435 63 and 46.
+// Whether a large problem the persistent kernels cannot read as it is runs on
+// gemm_dma16_ragged_kernel over padded copies of A and B (K rounded up to 256,
+// N to 16), which stores C (and adds D) in place at any alignment. `aligned`:
+// rows of 16-byte pieces, K off 64.
+// Estimates in ns: its slices (0.575 us each up to half the CUs, 0.84 with all
+// busy), the copies at 4.5 TB/s and their launch, and the last round's C at 5
+// TB/s, against the 128x128 tiles that read the operands in place, a slice of
+// which takes 0.2 us and 0.56 more per tile and CU (0.15 and 0.29 per whole
+// tile with aligned rows). HIP graph per call, in place against copies:
+// 3000 x 3001 x 3003 75 and 50 us; 4000 x 4001 x 4001 140 and 81; 8000 x 8001 x
+// 2001 280 and 161; 5857 x 2373 x 1435 63 and 46; aligned 3000 x 3008 x 3024 57
+// and 47, 8000 x 8000 x 2000 164 and 145, 8192 x 8192 x 8208 526 and 466, but
+// 2000 x 4096 x 2064 28 and 41, 4114 x 16208 x 880 + D 198 and 210.
 struct LargeLayout {
   int64_t Kp, Np, a_bytes, b_bytes;
   bool copy_a, copy_b;
 };
 
-bool large_padded(const Problem &r, LargeLayout *L) {
+bool large_padded(const Problem &r, bool aligned, LargeLayout *L) {
   if (r.M < 256 || r.N < 256 || r.K < 256 || r.ldc >= (1ll << 29) || (r.D && r.ldd >= (1ll << 29)) ||
       r.batch > 65535)
     return false;
@@ -3688,11 +3711,16 @@ bool large_padded(const Problem &r, LargeLayout *L) {
   if (tiles > 0x7fffffff) return false;
   const double busy = (double)(tiles < kSplitCus ? tiles : kSplitCus) / kSplitCus;
   const double rounds = (double)((tiles + kSplitCus - 1) / kSplitCus);
-  const double padded = rounds * (double)(L->Kp / 64) * (600.0 + 250.0 * busy) +
+  const double slice = 575.0 + (busy > 0.5 ? 530.0 * (busy - 0.5) : 0.0);
+  const double padded = rounds * (double)(L->Kp / 64) * slice +
                         2.0 * (double)(L->a_bytes + L->b_bytes) / 4500.0 + 6000.0 +
-                        4.0 * (double)r.M * (double)r.N * (double)r.batch / 5000.0;
-  const double per_cu = (double)((r.M + 127) / 128) * (double)((r.N + 127) / 128) * (double)r.batch / kSplitCus;
-  const double direct = (double)((r.K + 63) / 64) * (200.0 + 560.0 * (per_cu < 0.4 ? 0.4 : per_cu)) + 4000.0;
+                        4.0 * (double)r.M * (double)r.N * (double)r.batch / 5000.0 / rounds;
+  const int64_t t128 = (r.M + 127) / 128 * ((r.N + 127) / 128) * r.batch;
+  const double per_cu = (double)t128 / kSplitCus;
+  const double direct =
+      4000.0 + (double)((r.K + 63) / 64) *
+                   (aligned ? 150.0 + 290.0 * (double)((t128 + kSplitCus - 1) / kSplitCus)
+                            : 200.0 + 560.0 * (per_cu < 0.4 ? 0.4 : per_cu));
   return padded < direct;
 }
 
@@ -3765,6 +3793,28 @@ DirectPlan direct_plan(const Problem &q) {
   return d;
 }
 
+// An aligned problem with K off 64 (which keeps it off the persistent kernels)
+// over padded copies, where that is the faster way and there is a workspace for
+// them of at most kLargeCopyBytes; *done says whether it was launched.
+constexpr int64_t kLargeCopyBytes = 256ll << 20;
+
+int launch_large_aligned(const Problem &q, Scratch &scr, bool *done) {
+  const Problem r = mfma_fold(q);
+  LargeLayout L;
+  *done = false;
+  if (scr.copies_taken || !large_padded(r, true, &L) || L.a_bytes + L.b_bytes > kLargeCopyBytes ||
+      !optional_workspace(scr))
+    return VT_OK;
+  void *w = nullptr;
+  if (scr.take(kPadded, (size_t)(L.a_bytes + L.b_bytes), &w) != VT_OK) {
+    (void)hipGetLastError();
+    g_err.clear();
+    return VT_OK;
+  }
+  *done = true;
+  return launch_large_padded(r, L, (int8_t *)w, (hipStream_t)scr.stream, scr.st->num_cus);
+}
+
 // Runs a problem without copies where that is the faster way; *done says
 // whether it was launched. scratch_limit: bytes of scratch the call may take.
 int launch_direct(const Problem &q, int64_t scratch_limit, Scratch &scr, bool *done) {
@@ -3776,7 +3826,7 @@ int launch_direct(const Problem &q, int64_t scratch_limit, Scratch &scr, bool *d
   *done = true;
   void *w = nullptr;
   LargeLayout L;
-  if (d.kind != kDirectSkinny && d.ks == 1 && large_padded(r, &L) && L.a_bytes + L.b_bytes <= scratch_limit) {
+  if (d.kind != kDirectSkinny && d.ks == 1 && large_padded(r, false, &L) && L.a_bytes + L.b_bytes <= scratch_limit) {
     if (L.a_bytes + L.b_bytes == 0 ||
         scr.take(kPadded, (size_t)(L.a_bytes + L.b_bytes), &w) == VT_OK)
       return launch_large_padded(r, L, (int8_t *)w, stream, scr.st->num_cus);
@@ -3900,8 +3950,11 @@ int prepare_gemm(const int8_t *A, const int8_t *B, const int32_t *D, int32_t *C,
 
 int launch_gemm(const GemmCall &c, Scratch &scr) {
   if (c.variant == VT_VARIANT_GENERIC || c.variant == VT_VARIANT_PADDED) {
-    // A fixed scratch buffer holds what vt_gemm_check reported for the call.
-    const int64_t limit = scr.fixed ? scratch_need(c.q, c.variant, c.k_split) : INT64_MAX;
+    // A fixed scratch buffer holds what vt_gemm_check reported for the call;
+    // the generic variant reports none.
+    const int64_t limit = scr.fixed ? scratch_need(c.q, c.variant, c.k_split)
+                          : c.variant == VT_VARIANT_GENERIC && !optional_workspace(scr) ? 0
+                                                                                        : INT64_MAX;
     bool done = false;
     const int rc = launch_direct(c.q, limit, scr, &done);
     if (rc || done) return rc;

@@ -236,9 +236,8 @@ def packed_columns(plan, num_cus=NUM_CUS):
 def packed_split(plan):
     """(k_split, 64-row blocks per slice) the packed kernel launches.
 
-    Mirrors launch_packed_rows in csrc/vt_hip_gemm.hip (which runs unsplit
-    where a split that only saves reads of A finds no workspace, as on a
-    stream captured before its first such call).
+    Mirrors launch_packed_rows in csrc/vt_hip_gemm.hip (which leaves out a
+    split that only saves reads of A while the stream is being captured).
     """
     kbt = -(-plan["k"] // 64)
     per = -(-kbt // _packed_geometry(plan)[1])
