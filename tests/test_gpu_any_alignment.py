@@ -124,10 +124,18 @@ def test_large_aligned_products_with_k_off_64(dev, case):
     check(dev, "auto", **case)
 
 
+# few aligned tiles over a K that has no equal slices of whole 128-deep steps
+@pytest.mark.parametrize("m,n,k", [(84, 1040, 14832), (128, 512, 4112), (300, 512, 2064),
+                                   (256, 2048, 8208), (66, 1600, 3088), (130, 256, 4224)])
+def test_aligned_slices_of_unequal_depth(dev, m, n, k):
+    check(dev, "auto", m, n, k)
+
+
 def test_a_cold_capture_runs_without_a_workspace(dev):
     """The K slices' and copies' workspaces are not needed: a stream captured
     before it has any runs the same product without them."""
-    for m, n, k in ((300, 300, 3001), (16, 1001, 4095), (3000, 3001, 2050), (3000, 3008, 3024), (9, 500, 5001)):
+    for m, n, k in ((300, 300, 3001), (16, 1001, 4095), (3000, 3001, 2050), (3000, 3008, 3024), (9, 500, 5001),
+                    (84, 1040, 14832)):
         say("cold capture", m, n, k)
         plan = hg.make_plan(m, n, k)
         A = torch.randint(-128, 128, (m, k), dtype=torch.int8, device=dev)

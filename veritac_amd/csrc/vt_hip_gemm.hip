@@ -3637,12 +3637,18 @@ int launch_generic(const Problem &q, hipStream_t stream) {
 
 
 int launch_large_aligned(const Problem &q, Scratch &scr, bool *done);
+int launch_ragged_slices(const Problem &q, Scratch &scr, bool *done);
 
 // The vector variants (operands already checked by vector_ok).
 int launch_vector(const Problem &q, int32_t variant, int32_t k_split, Scratch &scr) {
   if (variant != VT_VARIANT_SKINNY && q.K % 64) {
     bool done = false;
     const int rc = launch_large_aligned(q, scr, &done);
+    if (rc || done) return rc;
+  }
+  if (variant == VT_VARIANT_MFMA_128x128 && q.K >= 1024) {
+    bool done = false;
+    const int rc = launch_ragged_slices(q, scr, &done);
     if (rc || done) return rc;
   }
   switch (variant) {
@@ -3793,6 +3799,23 @@ DirectPlan direct_plan(const Problem &q) {
   return d;
 }
 
+// The tiles of a direct plan, with the partial sums of its K slices in w.
+int launch_direct_tiles(const Problem &r, const DirectPlan &d, int32_t *w, hipStream_t stream, int num_cus) {
+  Problem t = r;
+  if (d.ks > 1) {
+    t.sa = d.kc; t.sb = d.kc * r.ldb; t.D = nullptr; t.sd = 0; t.C = w;
+    t.ldc = partial_pitch(r.N); t.sc = r.M * t.ldc;
+  }
+  const int rc = d.kind == kDirectTiles64 ? launch_any_tiles<64, 64>(t, d.ks, d.kc, stream, num_cus)
+                                          : launch_any_tiles<128, 128>(t, d.ks, d.kc, stream, num_cus);
+  if (rc || d.ks == 1) return rc;
+  ReduceArgs ra;
+  ra.ws = w; ra.D = r.D; ra.C = r.C;
+  ra.ldd = r.ldd; ra.ldc = r.ldc; ra.sd = 0; ra.sc = 0;
+  ra.M = (int)r.M; ra.N = (int)r.N; ra.k_split = d.ks;
+  return launch_reduce(ra, 1, stream);
+}
+
 // An aligned problem with K off 64 (which keeps it off the persistent kernels)
 // over padded copies, where that is the faster way and there is a workspace for
 // them of at most kLargeCopyBytes; *done says whether it was launched.
@@ -3851,20 +3874,31 @@ int launch_direct(const Problem &q, int64_t scratch_limit, Scratch &scr, bool *d
     g_err.clear();
     direct_slices(r, 1, &d);
   }
-  Problem t = r;
-  if (d.ks > 1) {
-    t.sa = d.kc; t.sb = d.kc * r.ldb; t.D = nullptr; t.sd = 0; t.C = (int32_t *)w;
-    t.ldc = partial_pitch(r.N); t.sc = r.M * t.ldc;
+  return launch_direct_tiles(r, d, (int32_t *)w, stream, scr.st->num_cus);
+}
+
+// Few aligned tiles over a long K that does not divide into the MFMA split's
+// equal slices of whole 128-deep steps: slices of whole 64-deep ones, the last
+// one shorter, when the stream's workspace may be used. Calls in a row, unsplit
+// (already with the K tail's loads in flight, 69 us) against sliced: 84 x 1040 x
+// 14832 14 us, 128 x 512 x 4112 32 -> 11, 200 x 1008 x 15008 128 -> 16, 512 x
+// 4096 x 9008 78 -> 34 (first figures: with the check at the load).
+int launch_ragged_slices(const Problem &q, Scratch &scr, bool *done) {
+  *done = false;
+  const Problem r = mfma_fold(q);
+  if (r.batch != 1 || mfma128_split(r) != 1) return VT_OK;
+  DirectPlan d = direct_plan(r);
+  if ((d.kind != kDirectTiles64 && d.kind != kDirectTiles128) || (d.ks < 4 && (d.ks < 2 || r.K < 8192)) ||
+      !optional_workspace(scr))
+    return VT_OK;
+  void *w = nullptr;
+  if (scr.take(kPartials, (size_t)d.scratch, &w) != VT_OK) {
+    (void)hipGetLastError();
+    g_err.clear();
+    return VT_OK;
   }
-  const int cus = scr.st->num_cus;
-  const int rc = d.kind == kDirectTiles64 ? launch_any_tiles<64, 64>(t, d.ks, d.kc, stream, cus)
-                                          : launch_any_tiles<128, 128>(t, d.ks, d.kc, stream, cus);
-  if (rc || d.ks == 1) return rc;
-  ReduceArgs ra;
-  ra.ws = (const int32_t *)w; ra.D = r.D; ra.C = r.C;
-  ra.ldd = r.ldd; ra.ldc = r.ldc; ra.sd = 0; ra.sc = 0;
-  ra.M = (int)r.M; ra.N = (int)r.N; ra.k_split = d.ks;
-  return launch_reduce(ra, 1, stream);
+  *done = true;
+  return launch_direct_tiles(r, d, (int32_t *)w, (hipStream_t)scr.stream, scr.st->num_cus);
 }
 
 // One validated vt_gemm_i8 problem and the kernel it runs.
