@@ -113,7 +113,7 @@ extern "C" {
  * vt_gemm_check reports what copies of all three would take. For aligned
  * shapes VT_VARIANT_AUTO picks VT_VARIANT_SKINNY for M <= 16, and for
  * M <= 64 when K >= 512 and ceil(N / 128) * batch < 256 (the skinny kernel
- * runs 1, 2 or 4 row blocks of 16 over one stream of B), VT_VARIANT_GENERIC when K <= 64 and
+ * runs 1 to 4 row blocks of 16 over one stream of B), VT_VARIANT_GENERIC when K <= 64 and
  * M * N * K * batch <= 2^20 (faster than any MFMA launch there), and an MFMA
  * variant otherwise. The MFMA variants
  * address each tile from a 64-bit base with 32-bit offsets inside it, so
@@ -396,7 +396,7 @@ int vt_pack_b_i8(const int8_t *B, int8_t *Bp, int64_t K, int64_t N, int64_t ldb,
  *     tiles the same way, K split into up to 16 slices (a second kernel adds
  *     them) when fewer than 64 tiles would run, as vt_gemm_i8 does;
  *   - up to 64 rows (or tiles whose offsets exceed 32 bits): groups of up to
- *     64 rows, each group streaming B once for its 1, 2 or 4 row blocks of
+ *     64 rows, each group streaming B once for its 1 to 4 row blocks of
  *     16. Columns go to workgroups in groups of 8-column half blocks: whole
  *     groups of four 16-column blocks when N gives 192 or more of them, else
  *     smaller groups, about one per CU.

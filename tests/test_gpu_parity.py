@@ -249,7 +249,7 @@ def test_batched_unshared_and_shared(dev):
 @pytest.mark.parametrize("m", [17, 24, 31, 32, 33, 48, 63, 64])
 @pytest.mark.parametrize("k_split", [0, 1, 3])
 def test_skinny_row_blocks(dev, m, k_split):
-    """17..64 rows run as 2 or 4 row blocks of 16 over the same B stream:
+    """17..64 rows run as 2 to 4 row blocks of 16 over the same B stream:
     rows past M are zero in the A slice and never stored; D added in place."""
     rng = np.random.default_rng(m * 10 + k_split)
     n, k = 1040, 4160

@@ -158,9 +158,9 @@ def packed_finishes(plan):
 
 
 def skinny_row_blocks(m):
-    """Row blocks of 16 the skinny kernel runs for m rows: 1, 2 or 4
+    """Row blocks of 16 the skinny kernel runs for m rows: 1 to 4
     (skinny_row_blocks in the HIP source)."""
-    return 1 if m <= 16 else 2 if m <= 32 else 4
+    return -(-m // 16)
 
 
 def skinny_a_stride(k_chunk):
