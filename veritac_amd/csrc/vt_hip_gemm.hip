@@ -1803,19 +1803,28 @@ constexpr int kReduceThreads = 64;
 
 template <bool HAS_D>
 __global__ __launch_bounds__(kReduceThreads) void skinny_reduce_kernel(ReduceArgs p) {
-  const int64_t i = (int64_t)blockIdx.x * kReduceThreads + threadIdx.x;   // over M * pitch / 4
+  // i over M * pitch / 4, below 2^31 (launch_reduce); pieces of 4 columns keep
+  // the division in 32 bits (36 x 8192 x 1024, whole
+  // call: 8.27 -> 7.99 us with that and one load and store a piece).
+  const uint32_t i = blockIdx.x * (uint32_t)kReduceThreads + threadIdx.x;
   const int64_t pitch = partial_pitch(p.N), slice = p.M * pitch;
   if (i >= slice / 4) return;
   const int bidx = blockIdx.y;
-  const int64_t e = i * 4;
-  const int row = (int)(e / pitch), col = (int)(e - row * pitch);
+  const int64_t e = (int64_t)i * 4;
+  const uint32_t pieces = (uint32_t)(pitch / 4);
+  const int row = (int)(i / pieces), col = (int)(i - (uint32_t)row * pieces) * 4;
+  const bool whole = col + 4 <= p.N;   // one access for the 4 columns (4-byte aligned)
   const int32_t *w = p.ws + (int64_t)bidx * p.k_split * slice + e;
   int32_t *c = p.C + bidx * p.sc + (int64_t)row * p.ldc + col;
   v4i s = v4i{0, 0, 0, 0};
   if constexpr (HAS_D) {
     const int32_t *d = p.D + bidx * p.sd + (int64_t)row * p.ldd + col;
+    if (whole) {
+      s = *(const v4i_any *)d;
+    } else {
 #pragma unroll
-    for (int t = 0; t < 4; ++t) s[t] = col + t < p.N ? d[t] : 0;
+      for (int t = 0; t < 3; ++t) s[t] = col + t < p.N ? d[t] : 0;
+    }
   }
   // Up to 8 partials in flight at once: every load of a batch is issued
   // before the first add waits.
@@ -1830,9 +1839,13 @@ __global__ __launch_bounds__(kReduceThreads) void skinny_reduce_kernel(ReduceArg
 #pragma unroll
       for (int t = 0; t < 4; ++t) s[t] = add_wrap(s[t], o[u][t]);
   }
+  if (whole) {
+    *(v4i_any *)c = s;
+  } else {
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
-    if (col + t < p.N) c[t] = s[t];
+    for (int t = 0; t < 3; ++t)
+      if (col + t < p.N) c[t] = s[t];
+  }
 }
 
 // ---------------------------------------------------------------------------
