@@ -120,3 +120,22 @@ def test_replay_repeated_calls_are_independent(dev, commands):
         B = rng.integers(-128, 128, p["k"] * p["n"]).tolist()
         assert rp.run_commands(s["commands"], p, A, B, device=dev)[0] == \
             gr.run_commands(s["commands"], p, A, B)[0]
+
+
+# The kernel takes 128 operations at a time: programs that end around one and
+# two of those, the product and its store on either side of the line.
+@pytest.mark.parametrize("count", [5, 127, 128, 129, 130, 131, 256, 257, 260])
+def test_operations_over_staging_lines(dev, count):
+    from veritac_amd.specializations.hip_gemm import schedules as sc
+    plan = sc.make_plan(16, 16, 16, "baseline")
+    commands = sc.gen_commands(plan)
+    at = next(i for i, c in enumerate(commands) if c["kind"] == "mvin")
+    base = len(rp.lower(commands, plan)[0])
+    commands[at:at] = [dict(commands[at]) for _ in range(count - base)]
+    assert len(rp.lower(commands, plan)[0]) == count
+    rng = np.random.default_rng(count)
+    A = rng.integers(-128, 128, (16, 16), dtype=np.int8)
+    B = rng.integers(-128, 128, (16, 16), dtype=np.int8)
+    say("replay operations", count)
+    C, _ = rp.run_commands(commands, plan, A.reshape(-1), B.reshape(-1))
+    assert np.array_equal(np.asarray(C).reshape(16, 16), go.gemm_i8(A, B))
