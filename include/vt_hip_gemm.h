@@ -143,7 +143,9 @@ extern "C" {
  * stream's workspaces: replay them in order on that stream (or with the same
  * ordering against it), never two at once. Overlapping launches on one
  * workspace race, and racing finishing words can stay nonzero and spoil the
- * later calls that use them.
+ * later calls that use them. Host threads may share a stream: a call that uses
+ * a workspace holds its stream's lock from then to its last launch, so no
+ * other thread's launch comes between its own.
  *
  * Sizes up to 2^40, leading dimensions up to 2^40, batch up to 2^31, batch
  * strides up to 2^56, and every operand's byte extent below 2^56. C may not
@@ -172,8 +174,9 @@ int vt_gemm_i8(const int8_t *A, const int8_t *B, const int32_t *D, int32_t *C,
  * reports the bytes) returns VT_EUNSUPPORTED before anything is launched.
  * Every call on a device shares that device's array and nothing in it needs
  * clearing between calls (each call writes all the scratch it reads), so
- * calls that overlap on one device -- on different streams, or from
- * different threads without ordering -- race: order them on one stream.
+ * calls on different streams of one device that are not ordered against each
+ * other race: order them on one stream (host threads may share it, as for
+ * vt_gemm_i8).
  */
 #define VT_NOALLOC_SCRATCH_BYTES (32 << 20)
 int vt_gemm_i8_noalloc(const int8_t *A, const int8_t *B, const int32_t *D,

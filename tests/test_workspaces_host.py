@@ -1,0 +1,119 @@
+"""The library's per-stream workspaces, on the CPU: vt_gemm_i8's host code runs
+against a HIP runtime that only logs (fake_hip.cpp), so what it launches and
+allocates, and in which order host threads do, can be checked without a GPU.
+Operand addresses are made up and never read."""
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+ROCM = "/opt/rocm"
+
+PRELUDE = """
+import ctypes, json, sys, threading
+fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+fake.fake_log.restype = ctypes.c_char_p
+fake.fake_capture.argtypes = [ctypes.c_void_p, ctypes.c_int]
+from veritac_amd import _lib
+_lib.load_library()
+STREAM = 1 << 20
+
+def gemm(m, n, k, variant="auto", stream=STREAM, batch=1, shared=True, where=0, call=_lib.gemm_raw):
+    base = (1 + where) << 43
+    multi = batch > 1
+    call(base, base + (1 << 40), None, base + (2 << 40), m, n, k, k, n, n, n, batch,
+         m * k if multi else 0, k * n if multi and not shared else 0, 0, m * n if multi else 0,
+         variant, 0, stream)
+
+def packed(m, n, k, batch=1, where=0, stream=STREAM, k_split=0):
+    base = (1 + where) << 43
+    multi = batch > 1
+    _lib.gemm_packed_raw(base, base + (1 << 40), None, base + (2 << 40), m, n, k, k, n, n, batch,
+                         m * k if multi else 0, n * (-(-k // 64) * 64) if multi else 0, 0,
+                         m * n if multi else 0, k_split, stream)
+
+def log():
+    return [line.split(" ", 3) for line in fake.fake_log().decode().splitlines()]
+
+def launches():
+    return [e for e in log() if e[1] == "launch"]
+
+def allocated():
+    return [int(e[2]) for e in log() if e[1] == "malloc"]
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    """run(code) -> what the code printed as JSON, in a process of its own."""
+    lib = str(tmp_path_factory.mktemp("fake") / "libfake_hip.so")
+    subprocess.run(["g++", "-O1", "-shared", "-fPIC", "-std=c++17", "-D__HIP_PLATFORM_AMD__",
+                    "-I", os.path.join(ROCM, "include"),
+                    os.path.join(ROOT, "tests", "fake_hip.cpp"), "-o", lib, "-pthread"], check=True)
+
+    def run(code):
+        proc = subprocess.run([sys.executable, "-c", PRELUDE + code, lib], cwd=ROOT,
+                              capture_output=True, text=True, timeout=120)
+        assert proc.returncode == 0, proc.stderr
+        return json.loads(proc.stdout)
+    return run
+
+
+# One call each that hands data from one launch to the next through a workspace.
+TWO_LAUNCHES = [
+    "gemm(84, 1040, 14832, where=w)",                      # K slices of unequal depth
+    "gemm(3000, 3008, 3024, where=w)",                     # copies for the persistent kernel
+    "gemm(3000, 3001, 3003, where=w)",                     # the same off the 16-byte grid
+    "gemm(70, 80, 4111, 'generic', where=w)",              # K slices in place
+    "gemm(40000, 8, 200, where=w)",                        # copies, a vector kernel, copy-out
+    "gemm(48, 4096, 14336, where=w)",                      # row-major decode
+    "gemm(128, 4096, 8192, where=w)",                      # equal K slices
+    "packed(48, 4096, 14336, where=w)",                    # packed decode, split to read less of A
+    "packed(48, 512, 8192, where=w)",                      # packed decode over few columns
+    "gemm(128, 4096, 8192, where=w, call=_lib.gemm_noalloc_raw)",   # the static array
+]
+
+
+@pytest.mark.parametrize("call", TWO_LAUNCHES)
+def test_a_call_keeps_its_workspace_until_its_last_launch(run, call):
+    """Two host threads on one stream: no launch of one comes between the
+    launches of the other's call, where it would overwrite what the first
+    kernel left for the second."""
+    got = run("""
+def calls(w):
+    for _ in range(6):
+        %s
+calls(0)                      # the stream's workspace, before the threads start
+per_call = len(launches()) // 6
+fake.fake_reset()
+fake.fake_pause(1500)
+ts = [threading.Thread(target=calls, args=(w,)) for w in (0, 1)]
+[t.start() for t in ts]; [t.join() for t in ts]
+print(json.dumps([per_call, launches()]))
+""" % call)
+    per_call, seen = got
+    assert per_call == (3 if "40000" in call else 2)
+    order = [e[0] for e in seen]
+    assert sorted(set(order)) == ["0", "1"] and len(order) == 12 * per_call
+    for i in range(0, len(order), per_call):
+        assert len(set(order[i:i + per_call])) == 1, [e[0] + " " + e[3][:40] for e in seen]
+
+
+def test_streams_do_not_wait_for_each_other(run):
+    """The lock is a stream's own: a thread in the middle of a call on one
+    stream does not hold up another stream's."""
+    order = run("""
+def calls(w):
+    for _ in range(4):
+        gemm(84, 1040, 14832, where=w, stream=STREAM + w)
+calls(0); calls(1)
+fake.fake_reset()
+fake.fake_pause(3000)
+ts = [threading.Thread(target=calls, args=(w,)) for w in (0, 1)]
+[t.start() for t in ts]; [t.join() for t in ts]
+print(json.dumps([e[0] for e in launches()]))
+""")
+    assert any(len(set(order[i:i + 2])) == 2 for i in range(0, len(order), 2))

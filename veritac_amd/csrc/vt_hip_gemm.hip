@@ -2326,17 +2326,27 @@ struct Workspace {
   size_t bytes = 0;
 };
 
+// What the library keeps for one stream of a device. `use` is held by a call
+// from its first workspace to its last launch (Scratch::take): host threads
+// sharing the stream (torch's default stream belongs to all of them) would
+// otherwise launch between the kernel that fills a workspace and the one that
+// reads it.
+struct StreamState {
+  std::mutex use;
+  Workspace ws[kScratchKinds];
+  // Workspaces superseded by larger ones. They are never freed: a HIP graph
+  // captured earlier may still hold their addresses.
+  std::vector<void *> retired;
+};
+
 struct DeviceState {
   bool probed = false;
   bool ok = false;
   int num_cus = 256;
   std::string arch;
   hipError_t attr_err = hipSuccess;   // dynamic-LDS limits, set once on this device
-  std::map<void *, Workspace> ws[kScratchKinds];   // per stream, per kind
-  // Workspaces superseded by larger ones. They are never freed: a HIP graph
-  // captured earlier may still hold their addresses, and a host thread may
-  // still be launching with one.
-  std::vector<void *> retired;
+  std::map<void *, StreamState> streams;   // nodes stay where they are
+  std::mutex scratch_use;                  // StreamState::use for `scratch`
   int8_t *scratch = nullptr;   // this device's address of the static scratch array
   hipError_t scratch_err = hipSuccess;
 };
@@ -2393,14 +2403,13 @@ int current_device(int *dev_out, DeviceState **st_out) {
   return VT_OK;
 }
 
-// The library's workspace of one kind on (device, stream). Calls on one
-// stream are ordered, so a stream's workspace is never used by two launches
-// in flight. It only grows, at least doubling, and is allocated outside
-// stream capture only: a call that needs more than the stream has while the
-// stream is being captured is refused (run it once before capturing).
-int get_workspace(DeviceState *st, void *stream, ScratchKind kind, size_t bytes, void **out) {
-  std::lock_guard<std::mutex> lk(g_mu);
-  Workspace &w = st->ws[kind][stream];
+// The library's workspace of one kind on a stream, whose `use` the caller
+// holds. Launches on one stream are ordered, so its workspace is never used by
+// two of them in flight. It only grows, at least doubling, and is allocated
+// outside stream capture only: a call that needs more than the stream has
+// while the stream is being captured is refused (run it once before capturing).
+int get_workspace(StreamState *ss, void *stream, ScratchKind kind, size_t bytes, void **out) {
+  Workspace &w = ss->ws[kind];
   if (w.bytes < bytes) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     VT_HIP_CHECK(hipStreamIsCapturing((hipStream_t)stream, &cs));
@@ -2417,7 +2426,7 @@ int get_workspace(DeviceState *st, void *stream, ScratchKind kind, size_t bytes,
     // leaves them zero. The clear is ordered before that launch on the same
     // stream; it is never captured, since growth under capture is refused above.
     if (kind == kFinWords) VT_HIP_CHECK(hipMemsetAsync(p, 0, nb, (hipStream_t)stream));
-    if (w.ptr) st->retired.push_back(w.ptr);
+    if (w.ptr) ss->retired.push_back(w.ptr);
     w.ptr = p;
     w.bytes = nb;
   }
@@ -2437,9 +2446,18 @@ struct Scratch {
   int8_t *fixed = nullptr;   // device address of `scratch`, or null
   size_t used = 0;
   bool copies_taken = false;   // the call holds padded copies in the kPadded workspace
+  StreamState *ss = nullptr;   // of `stream`, once a workspace was taken
+  std::unique_lock<std::mutex> use;   // held from the first take to the end of the call
 
   int take(ScratchKind kind, size_t bytes, void **out) {
-    if (!fixed) return get_workspace(st, stream, kind, bytes, out);
+    if (!use.owns_lock()) {
+      if (!fixed) {
+        std::lock_guard<std::mutex> lk(g_mu);
+        ss = &st->streams[stream];
+      }
+      use = std::unique_lock<std::mutex>(fixed ? st->scratch_use : ss->use);
+    }
+    if (!fixed) return get_workspace(ss, stream, kind, bytes, out);
     const size_t need = (bytes + 255) / 256 * 256;
     if (need > kScratchBytes - used)
       return fail(VT_EUNSUPPORTED,
