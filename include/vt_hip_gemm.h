@@ -138,8 +138,10 @@ extern "C" {
  * call takes from vt_gemm_i8_noalloc's array, which bounds what it needs
  * from a stream's workspaces). Outside capture a call may also use workspaces
  * it does not need where that is faster: K slices of the generic and packed
- * paths, and padded copies (at most 256 MiB) for large products whose K is
- * not a multiple of 64. Graphs captured on one stream use that
+ * paths, and padded copies for large products whose K is not a multiple of 64
+ * or that ask for the generic variant. Such a call never takes a stream's
+ * workspaces of one kind past 256 MiB, superseded ones included: it then runs
+ * without. Graphs captured on one stream use that
  * stream's workspaces: replay them in order on that stream (or with the same
  * ordering against it), never two at once. Overlapping launches on one
  * workspace race, and racing finishing words can stay nonzero and spoil the

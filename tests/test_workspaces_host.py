@@ -117,3 +117,36 @@ ts = [threading.Thread(target=calls, args=(w,)) for w in (0, 1)]
 print(json.dumps([e[0] for e in launches()]))
 """)
     assert any(len(set(order[i:i + 2])) == 2 for i in range(0, len(order), 2))
+
+
+def test_optional_workspaces_stay_within_their_bound(run):
+    """Calls that could run without a workspace leave a stream at most 256 MiB
+    of one kind, superseded workspaces included; past it they run without."""
+    got = run("""
+names = lambda: ["pad" if "pad_i8" in e[3] else "ragged" if "ragged" in e[3] else "other" for e in launches()]
+out = []
+for calls in ([(8192, 8192, 8208, "auto"), (8208, 8192, 8208, "auto"), (8192, 8192, 8208, "auto")],
+              [(3000, 3008, 3024, "auto"), (3000, 3008, 3280, "auto"), (8192, 8192, 8208, "auto"),
+               (8192, 8192, 9200, "auto")],
+              [(3000, 3001, 3003, "generic"), (8001, 8003, 17001, "generic")]):
+    fake.fake_reset()
+    STREAM += 1
+    for m, n, k, v in calls:
+        gemm(m, n, k, v, stream=STREAM)
+    out.append([allocated(), names()])
+print(json.dumps(out))
+""")
+    mib = 1 << 20
+    for sizes, _ in got:
+        assert sum(sizes) <= 256 * mib, sizes
+    # the second call needs more than is left and runs without copies; the third
+    # fits the first one's workspace
+    sizes, names = got[0]
+    assert len(sizes) == 1 and names.count("ragged") == 2 and names[:2] == ["pad", "ragged"]
+    assert names[-2:] == ["pad", "ragged"] and "other" in names[2:-2]
+    # growth doubles while there is room, and never past what is left
+    sizes, names = got[1]
+    assert len(sizes) == 3 and sizes[1] == 2 * sizes[0] and names.count("ragged") == 3
+    # the generic variant never needs copies: one of more than 256 MiB reads in place
+    sizes, names = got[2]
+    assert len(sizes) == 1 and names == ["pad", "ragged", "other"]

@@ -2334,6 +2334,7 @@ struct Workspace {
 struct StreamState {
   std::mutex use;
   Workspace ws[kScratchKinds];
+  size_t held[kScratchKinds] = {};   // bytes allocated per kind, superseded ones included
   // Workspaces superseded by larger ones. They are never freed: a HIP graph
   // captured earlier may still hold their addresses.
   std::vector<void *> retired;
@@ -2408,7 +2409,12 @@ int current_device(int *dev_out, DeviceState **st_out) {
 // two of them in flight. It only grows, at least doubling, and is allocated
 // outside stream capture only: a call that needs more than the stream has
 // while the stream is being captured is refused (run it once before capturing).
-int get_workspace(StreamState *ss, void *stream, ScratchKind kind, size_t bytes, void **out) {
+// `optional`: the call could do without; it is refused what would take the kind
+// past kOptionalBytes, superseded workspaces included.
+constexpr size_t kOptionalBytes = (size_t)256 << 20;
+
+int get_workspace(StreamState *ss, void *stream, ScratchKind kind, size_t bytes, bool optional,
+                  void **out) {
   Workspace &w = ss->ws[kind];
   if (w.bytes < bytes) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -2420,6 +2426,13 @@ int get_workspace(StreamState *ss, void *stream, ScratchKind kind, size_t bytes,
                   bytes, w.bytes);
     size_t nb = bytes > 2 * w.bytes ? bytes : 2 * w.bytes;
     if (nb < (1u << 20)) nb = 1u << 20;
+    if (optional) {
+      const size_t left = ss->held[kind] < kOptionalBytes ? kOptionalBytes - ss->held[kind] : 0;
+      if (bytes > left)
+        return fail(VT_EUNSUPPORTED, "an optional workspace of %zu bytes would hold more than %zu",
+                    bytes, kOptionalBytes);
+      if (nb > left) nb = left;
+    }
     void *p = nullptr;
     VT_HIP_CHECK(hipMalloc(&p, nb));
     // Finishing words read zero before their first launch, and every launch
@@ -2427,6 +2440,7 @@ int get_workspace(StreamState *ss, void *stream, ScratchKind kind, size_t bytes,
     // stream; it is never captured, since growth under capture is refused above.
     if (kind == kFinWords) VT_HIP_CHECK(hipMemsetAsync(p, 0, nb, (hipStream_t)stream));
     if (w.ptr) ss->retired.push_back(w.ptr);
+    ss->held[kind] += nb;
     w.ptr = p;
     w.bytes = nb;
   }
@@ -2449,7 +2463,7 @@ struct Scratch {
   StreamState *ss = nullptr;   // of `stream`, once a workspace was taken
   std::unique_lock<std::mutex> use;   // held from the first take to the end of the call
 
-  int take(ScratchKind kind, size_t bytes, void **out) {
+  int take(ScratchKind kind, size_t bytes, void **out, bool optional = false) {
     if (!use.owns_lock()) {
       if (!fixed) {
         std::lock_guard<std::mutex> lk(g_mu);
@@ -2457,7 +2471,7 @@ struct Scratch {
       }
       use = std::unique_lock<std::mutex>(fixed ? st->scratch_use : ss->use);
     }
-    if (!fixed) return get_workspace(ss, stream, kind, bytes, out);
+    if (!fixed) return get_workspace(ss, stream, kind, bytes, optional, out);
     const size_t need = (bytes + 255) / 256 * 256;
     if (need > kScratchBytes - used)
       return fail(VT_EUNSUPPORTED,
@@ -3381,10 +3395,11 @@ int launch_packed_rows(const Problem &q, int k_split, Scratch &scr, bool a_split
     void *w = nullptr;
     const size_t bytes = fin ? (size_t)q.batch * ((q.M + 1) / 2) * q.N * sizeof(uint64_t)
                              : (size_t)q.batch * a.k_split * q.M * q.N * sizeof(int32_t);
-    if (int rc = scr.take(fin ? kFinWords : kPartials, bytes, &w)) {
-      // A split only to read less of A is not needed: with no memory for its
-      // workspace run unsplit.
-      if (k_split > 0 || base.ks == geo.ks) return rc;
+    // A split only to read less of A is not needed: with no memory for its
+    // workspace run unsplit.
+    const bool optional = k_split == 0 && base.ks != geo.ks;
+    if (int rc = scr.take(fin ? kFinWords : kPartials, bytes, &w, optional)) {
+      if (!optional) return rc;
       (void)hipGetLastError();
       g_err.clear();
       return launch_packed_rows(q, 0, scr, false);
@@ -3866,18 +3881,15 @@ int launch_direct_tiles(const Problem &r, const DirectPlan &d, int32_t *w, hipSt
 
 // An aligned problem with K off 64 (which keeps it off the persistent kernels)
 // over padded copies, where that is the faster way and there is a workspace for
-// them of at most kLargeCopyBytes; *done says whether it was launched.
-constexpr int64_t kLargeCopyBytes = 256ll << 20;
-
+// them; *done says whether it was launched.
 int launch_large_aligned(const Problem &q, Scratch &scr, bool *done) {
   const Problem r = mfma_fold(q);
   LargeLayout L;
   *done = false;
-  if (scr.copies_taken || !large_padded(r, true, &L) || L.a_bytes + L.b_bytes > kLargeCopyBytes ||
-      !optional_workspace(scr))
+  if (scr.copies_taken || !large_padded(r, true, &L) || !optional_workspace(scr))
     return VT_OK;
   void *w = nullptr;
-  if (scr.take(kPadded, (size_t)(L.a_bytes + L.b_bytes), &w) != VT_OK) {
+  if (scr.take(kPadded, (size_t)(L.a_bytes + L.b_bytes), &w, true) != VT_OK) {
     (void)hipGetLastError();
     g_err.clear();
     return VT_OK;
@@ -3887,8 +3899,9 @@ int launch_large_aligned(const Problem &q, Scratch &scr, bool *done) {
 }
 
 // Runs a problem without copies where that is the faster way; *done says
-// whether it was launched. scratch_limit: bytes of scratch the call may take.
-int launch_direct(const Problem &q, int64_t scratch_limit, Scratch &scr, bool *done) {
+// whether it was launched. scratch_limit: bytes of scratch the call may take;
+// optional: as for get_workspace.
+int launch_direct(const Problem &q, int64_t scratch_limit, bool optional, Scratch &scr, bool *done) {
   DirectPlan d = direct_plan(q);
   *done = false;
   if (d.kind == kDirectNone) return VT_OK;
@@ -3899,7 +3912,7 @@ int launch_direct(const Problem &q, int64_t scratch_limit, Scratch &scr, bool *d
   LargeLayout L;
   if (d.kind != kDirectSkinny && d.ks == 1 && large_padded(r, false, &L) && L.a_bytes + L.b_bytes <= scratch_limit) {
     if (L.a_bytes + L.b_bytes == 0 ||
-        scr.take(kPadded, (size_t)(L.a_bytes + L.b_bytes), &w) == VT_OK)
+        scr.take(kPadded, (size_t)(L.a_bytes + L.b_bytes), &w, optional) == VT_OK)
       return launch_large_padded(r, L, (int8_t *)w, stream, scr.st->num_cus);
     (void)hipGetLastError();
     g_err.clear();
@@ -3917,7 +3930,7 @@ int launch_direct(const Problem &q, int64_t scratch_limit, Scratch &scr, bool *d
     g_err.clear();
     d.kind = kDirectTiles64;
     direct_slices(r, 1, &d);
-  } else if (d.scratch > 0 && scr.take(kPartials, (size_t)d.scratch, &w) != VT_OK) {
+  } else if (d.scratch > 0 && scr.take(kPartials, (size_t)d.scratch, &w, optional) != VT_OK) {
     (void)hipGetLastError();
     g_err.clear();
     direct_slices(r, 1, &d);
@@ -3940,7 +3953,7 @@ int launch_ragged_slices(const Problem &q, Scratch &scr, bool *done) {
       !optional_workspace(scr))
     return VT_OK;
   void *w = nullptr;
-  if (scr.take(kPartials, (size_t)d.scratch, &w) != VT_OK) {
+  if (scr.take(kPartials, (size_t)d.scratch, &w, true) != VT_OK) {
     (void)hipGetLastError();
     g_err.clear();
     return VT_OK;
@@ -4034,11 +4047,12 @@ int launch_gemm(const GemmCall &c, Scratch &scr) {
   if (c.variant == VT_VARIANT_GENERIC || c.variant == VT_VARIANT_PADDED) {
     // A fixed scratch buffer holds what vt_gemm_check reported for the call;
     // the generic variant reports none.
+    const bool optional = c.variant == VT_VARIANT_GENERIC;
     const int64_t limit = scr.fixed ? scratch_need(c.q, c.variant, c.k_split)
-                          : c.variant == VT_VARIANT_GENERIC && !optional_workspace(scr) ? 0
-                                                                                        : INT64_MAX;
+                          : !optional ? INT64_MAX
+                                      : optional_workspace(scr) ? (int64_t)kOptionalBytes : 0;
     bool done = false;
-    const int rc = launch_direct(c.q, limit, scr, &done);
+    const int rc = launch_direct(c.q, limit, optional, scr, &done);
     if (rc || done) return rc;
   }
   if (c.variant == VT_VARIANT_GENERIC) return launch_generic(c.q, (hipStream_t)scr.stream);
