@@ -64,3 +64,39 @@ def test_two_threads_on_one_stream(dev, m, n, k, variant):
     for _, _, want, outs in work:
         for i, out in enumerate(outs):
             assert torch.equal(out, want), i
+
+
+@pytest.mark.parametrize("m,n,k", [(84, 1040, 14832), (16, 4096, 8192)])
+def test_workspace_growth_while_another_thread_captures(dev, m, n, k):
+    """A call on a fresh stream allocates its workspace while another thread
+    captures its own stream; both results are right."""
+    print("growth beside a capture", m, n, k, flush=True)
+    plan, small = hg.make_plan(m, n, k), hg.make_plan(256, 256, 256)
+    A = torch.randint(-128, 128, (m, k), device=dev, dtype=torch.int8)
+    B = torch.randint(-128, 128, (k, n), device=dev, dtype=torch.int8)
+    a = torch.randint(-128, 128, (256, 256), device=dev, dtype=torch.int8)
+    out = torch.full((m, n), -2**31, dtype=torch.int32, device=dev)
+    c = torch.empty((256, 256), dtype=torch.int32, device=dev)
+    captured, other, failed = torch.cuda.Stream(), torch.cuda.Stream(), []
+    torch.cuda.synchronize()
+
+    def call():
+        try:
+            hg.run(plan, A, B, out=out, stream=other.cuda_stream)
+        except Exception as exc:
+            failed.append(exc)
+
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=captured):
+        hg.run(small, a, a, out=c)
+        t = threading.Thread(target=call)
+        t.start()
+        t.join()
+    assert not failed, failed
+    for _ in range(3):
+        c.fill_(-2**31)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(c, torch.matmul(a.double(), a.double()).to(torch.int32))
+    assert torch.equal(out, torch.matmul(A.double(), B.double()).to(torch.int32))

@@ -150,3 +150,25 @@ print(json.dumps(out))
     # the generic variant never needs copies: one of more than 256 MiB reads in place
     sizes, names = got[2]
     assert len(sizes) == 1 and names == ["pad", "ragged", "other"]
+
+
+def test_a_workspace_is_allocated_while_another_thread_captures(run):
+    """A thread capturing its own stream in global mode does not keep other
+    threads' calls from their workspaces, nor change how they run; the caller's
+    capture mode is as it was afterwards."""
+    got = run("""
+calls = [(84, 1040, 14832), (3000, 3008, 3024), (48, 4096, 14336), (16, 4096, 8192)]
+for other in (0, 1):
+    fake.fake_global_capture(other)
+    for c in calls:
+        STREAM += 1
+        gemm(*c, stream=STREAM)
+mode = ctypes.c_int(1)
+fake.hipThreadExchangeStreamCaptureMode(ctypes.byref(mode))
+kinds = [[e[1]] + (e[3:] if e[1] == "launch" else e[2:3]) for e in log()]
+print(json.dumps([mode.value, kinds]))
+""")
+    mode, kinds = got
+    assert mode == 0 and not [k for k in kinds if k[0] == "refused"]
+    half = len(kinds) // 2
+    assert kinds[:half] == kinds[half:] and [k[0] for k in kinds[:half]].count("malloc") == 4

@@ -2433,8 +2433,14 @@ int get_workspace(StreamState *ss, void *stream, ScratchKind kind, size_t bytes,
                     bytes, kOptionalBytes);
       if (nb > left) nb = left;
     }
+    // Another thread may be capturing a stream of its own, in the mode that
+    // refuses hipMalloc to every thread: this allocation is not part of it.
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    VT_HIP_CHECK(hipThreadExchangeStreamCaptureMode(&mode));
     void *p = nullptr;
-    VT_HIP_CHECK(hipMalloc(&p, nb));
+    const hipError_t err = hipMalloc(&p, nb);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    VT_HIP_CHECK(err);
     // Finishing words read zero before their first launch, and every launch
     // leaves them zero. The clear is ordered before that launch on the same
     // stream; it is never captured, since growth under capture is refused above.
