@@ -538,6 +538,27 @@ def test_packed_stages_and_splits(dev, m, n, k, hpw, ks):
     assert np.array_equal(gpu_gemm_packed(dev, A, B, D, in_place=True), go.gemm_i8(A, B, D))
 
 
+# The same split over batches: through the finishing words (up to 16 rows) and
+# a second kernel, two and four slices, the batches' partial sums apart.
+@pytest.mark.parametrize("m,n,k,batch,ks", [(14, 1024, 1616, 6, 2), (15, 384, 4896, 4, 4),
+                                            (62, 128, 4704, 12, 2), (61, 768, 3792, 2, 4)])
+def test_packed_splits_across_batches(dev, m, n, k, batch, ks):
+    plan = hg.make_plan(m, n, k, batch=batch, has_d=True, d_max_abs=1 << 20, variant=hg.PACKED_VARIANT)
+    assert hg.packed_split(plan)[0] == ks
+    say("packed split, batches", m, n, k, batch)
+    rng = np.random.default_rng(m + n + k)
+    A = rng.integers(-128, 128, (batch, m, k), dtype=np.int8)
+    B = rng.integers(-128, 128, (batch, k, n), dtype=np.int8)
+    D = rng.integers(-2**20, 2**20, (batch, m, n), dtype=np.int32)
+    Bp = hg.pack_b(to_dev(dev, B))
+    for _ in range(2):          # the second call finds the finishing words zero again
+        C = to_dev(dev, D)
+        hg.run(plan, to_dev(dev, A), Bp, C, out=C)
+        got = C.cpu().numpy()
+        for b in range(batch):
+            assert np.array_equal(got[b], go.gemm_i8(A[b], B[b], D[b])), b
+
+
 def test_packed_split_needs_no_workspace_under_capture(dev):
     """A split that only saves reads of A runs unsplit on a stream that is
     captured before it ever had a workspace, as such calls did before."""

@@ -109,6 +109,25 @@ def test_packed_plans_validate():
                for c in hg.optimize(16, 14336, 4096)["candidates"])
 
 
+# m, n, k, batch -> K slices that were timed fastest of 1, 2 and 4 (or within
+# 2 % of it), where the partial sums of every batch and the last round of
+# workgroups count: 64 x 1024 x 4096 in 8 batches takes 13.9 us unsplit and
+# 18.9 in four slices, 57 x 11296 x 10528 35.4 and 43.1
+A_SPLITS = {
+    (64, 1024, 4096, 8): 1, (64, 1536, 6144, 6): 1, (63, 672, 5840, 16): 1, (63, 912, 5376, 8): 1,
+    (57, 11296, 10528, 1): 1, (51, 6128, 8080, 1): 1, (11, 8896, 9008, 1): 1, (57, 1456, 13120, 6): 1,
+    (17, 4096, 14336, 1): 4, (48, 4096, 14336, 1): 4, (20, 3808, 12016, 1): 4, (64, 2048, 8192, 1): 4,
+    (16, 4096, 14336, 1): 4, (1, 4096, 14336, 1): 1, (48, 8192, 4096, 1): 1,
+}
+
+
+@pytest.mark.parametrize("shape", sorted(A_SPLITS))
+def test_split_to_read_less_of_a_pays_for_its_sums(shape):
+    m, n, k, batch = shape
+    plan = hg.make_plan(m, n, k, batch=batch, variant=hg.PACKED_VARIANT)
+    assert hg.packed_split(plan)[0] == A_SPLITS[shape]
+
+
 def test_packed_rows_in_whole_tiles_go_to_the_256_kernel():
     """Rows run on the 256x256 kernel when n % 256 == 0, k % 64 == 0 and there
     are at least 128 whole 256-row tiles: all of them, the last partial tile

@@ -4,10 +4,13 @@ allocates, and in which order host threads do, can be checked without a GPU.
 Operand addresses are made up and never read."""
 import json
 import os
+import random
 import subprocess
 import sys
 
 import pytest
+
+from veritac_amd.specializations.hip_gemm import backend as hg
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 ROCM = "/opt/rocm"
@@ -172,3 +175,27 @@ print(json.dumps([mode.value, kinds]))
     assert mode == 0 and not [k for k in kinds if k[0] == "refused"]
     half = len(kinds) // 2
     assert kinds[:half] == kinds[half:] and [k[0] for k in kinds[:half]].count("malloc") == 4
+
+
+def test_packed_grids_are_the_plan_mirror_s(run):
+    """Column groups and K slices the library launches for packed decode are
+    those backend.packed_columns and packed_split name, batches included."""
+    shapes = []
+    rng = random.Random(9)
+    while len(shapes) < 150:
+        m, n, k = rng.randint(1, 64), 16 * rng.randint(1, 800), 16 * rng.randint(1, 1000)
+        batch = 1 if rng.random() < 0.5 else rng.randint(2, 16)
+        if n * k * batch < 1 << 30:
+            shapes.append((m, n, k, batch))
+    got = run("""
+out = []
+for m, n, k, batch in %r:
+    fake.fake_reset()
+    packed(m, n, k, batch)
+    out.append(launches()[0])
+print(json.dumps(out))
+""" % (shapes,))
+    for (m, n, k, batch), first in zip(shapes, got):
+        plan = hg.make_plan(m, n, k, batch=batch, variant=hg.PACKED_VARIANT)
+        want = hg.packed_columns(plan)[1] * hg.packed_split(plan)[0] * batch
+        assert "packed_skinny" in first[3] and int(first[3].split(" ")[0]) == want, (m, n, k, batch)

@@ -3189,24 +3189,30 @@ int packed_hpw(int64_t N, int64_t batch, int ks, int num_cus) {
 }
 
 // Slices of K for M (<= 64) rows over so few columns that one workgroup per
-// CU takes narrow groups: every workgroup then reads its whole slice of A,
-// which costs 27 ns per KB (N = 4096, K = 14336, narrow groups unsplit: M = 1
-// 10.4 us, 16 16.8, 32 22.3, 48 29.3). Slices with wider groups read A/ks but
-// have to be summed: about 2 us through the finishing words, or 4 us and the
-// partial sums' traffic at 3 TB/s in a second kernel. The least of the three
-// estimates, in ns: at that N and K four slices for M = 16 (12.8 us), 32
-// (16.6) and 48 (20.0) and none for M = 1 (two slices 11.1); N = 2048,
-// K = 8192 four for M = 48 (16.4 -> 10.6); N = 8192, K = 4096 none (M = 48
-// 12.5 us, two slices 14.4).
-int packed_a_split(int64_t M, int64_t N, int64_t K) {
+// CU takes narrow groups: every workgroup then reads its whole slice of A.
+// Slices with wider groups read A/ks but have to be summed, and may leave the
+// last round of workgroups nearly empty. The least of three estimates in ns:
+// a round takes 315 per half block and 32 per row and 1000 of the slice's K,
+// the sum 2000 through the finishing words or 3500 and the partial sums at 1.5
+// TB/s in a second kernel. Fitted to 170 drawn shapes (M 1 to 64, up to 16
+// batches), each timed with 1, 2 and 4 slices: the choice takes 0.954 of the
+// unsplit time, the best of the three 0.950, and none loses 2 %. Calls in a
+// row, unsplit against the choice: N = 4096, K = 14336 M = 17 15.7 -> 12.6 us,
+// 48 28.5 -> 17.1; 57 x 11296 x 10528 35.4 (four slices, 2.8 rounds, 43.1);
+// 64 x 1024 x 4096 in 8 batches 13.9 (four slices 18.9). A captured call may
+// not take this split's workspace and runs unsplit (optional_workspace).
+int packed_a_split(int64_t M, int64_t N, int64_t K, int64_t batch, int num_cus) {
   int best = 1;
   int64_t least = 0;
   for (int ks = 1; ks <= 4; ks *= 2) {
     if (ks > 1 && packed_kbt(K) < (int64_t)ks * kPackedWaves) break;
     const int64_t chunk = (packed_kbt(K) + ks - 1) / ks * 64;
-    int64_t ns = 27 * M * K / ks / 1000;
+    const int hpw = packed_hpw(N, batch, ks, num_cus);
+    const int64_t wgs = (2 * (N / 16) + hpw - 1) / hpw * batch * ks;
+    int64_t ns = (wgs + num_cus - 1) / num_cus * chunk * (315 * hpw + 32 * M) / 1000;
     if (ks > 1)
-      ns += M <= kSkinnyFinMaxM && skinny_fin_bits(ks, chunk) > 0 ? 2000 : 4000 + 8 * M * N * ks / 3000;
+      ns += M <= kSkinnyFinMaxM && skinny_fin_bits(ks, chunk) > 0 ? 2000
+                                                                  : 3500 + 8 * M * N * ks * batch / 1500;
     if (ks == 1 || ns < least) {
       least = ns;
       best = ks;
@@ -3234,7 +3240,7 @@ PackedGeom packed_geometry(int64_t M, int64_t N, int64_t K, int64_t batch, bool 
     if (ks > 64) ks = 64;
     g.ks = (int)ks;
   } else if (a_split && g.hpw < 2 * kPackedNBW) {
-    g.ks = packed_a_split(M, N, K);
+    g.ks = packed_a_split(M, N, K, batch, num_cus);
     g.hpw = packed_hpw(N, batch, g.ks, num_cus);
   }
   return g;

@@ -189,17 +189,21 @@ def _packed_hpw(n, batch, ks, num_cus):
     return max(1, min(-(-2 * nbt * batch * ks // num_cus), 2 * PACKED_NBW))
 
 
-def _packed_a_split(m, n, k):
+def _packed_a_split(m, n, k, batch, num_cus):
     """packed_a_split in csrc/vt_hip_gemm.hip: K slices for m rows over narrow
-    column groups, by the least estimated cost of reading A and summing."""
+    column groups, by the least estimated time of the rounds of workgroups
+    (their columns of B and rows of A) and of the sum."""
     kbt, best, least = -(-k // 64), 1, None
     for ks in (1, 2, 4):
         if ks > 1 and kbt < ks * PACKED_WAVES:
             break
-        ns = 27 * m * k // ks // 1000
+        chunk = -(-kbt // ks) * 64
+        hpw = _packed_hpw(n, batch, ks, num_cus)
+        wgs = -(-2 * (n // 16) // hpw) * batch * ks
+        ns = -(-wgs // num_cus) * chunk * (315 * hpw + 32 * m) // 1000
         if ks > 1:
-            fin = m <= SKINNY_FIN_MAX_M and skinny_fin_bits(ks, -(-kbt // ks) * 64) > 0
-            ns += 2000 if fin else 4000 + 8 * m * n * ks // 3000
+            fin = m <= SKINNY_FIN_MAX_M and skinny_fin_bits(ks, chunk) > 0
+            ns += 2000 if fin else 3500 + 8 * m * n * ks * batch // 1500
         if least is None or ns < least:
             best, least = ks, ns
     return best
@@ -219,7 +223,7 @@ def _packed_geometry(plan, num_cus=NUM_CUS):
         return hpw, max(1, min(-(-224 // groups), -(-(-(-k // 64)) // PACKED_WAVES), 64))
     if hpw == 2 * PACKED_NBW:
         return hpw, 1
-    ks = _packed_a_split(m, n, k)
+    ks = _packed_a_split(m, n, k, batch, num_cus)
     return _packed_hpw(n, batch, ks, num_cus), ks
 
 
