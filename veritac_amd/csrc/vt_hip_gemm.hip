@@ -1932,10 +1932,10 @@ struct PackedArgs {
 // Wave w takes the 64-row blocks kb_beg + w, kb_beg + w + WAVES, ...;
 // per block it loads its MB A fragments (16 bytes per lane) and the NBW packed
 // B tiles, S blocks ahead of the MFMAs (non-temporal loads: B is streamed
-// once). Every load is unconditional: rows past M read row M - 1 (their
-// outputs are not stored), k past K reads the row's last 16 bytes (packed B is
-// zero there), and blocks past the wave's last one repeat it. A branch around
-// the loads made the compiler wait for all of them at every step.
+// once). No lane branches around a load: rows past M read row M - 1 (their
+// outputs are not stored) and k past K reads the row's last 16 bytes (packed B
+// is zero there). Such a branch made the compiler wait for all of the loads at
+// every step.
 // S: what bounds the kernel is the bytes in flight, NBW * S KB per wave. With
 // the two stages that four tiles need, one tile per wave left 16 KB in flight
 // per CU: M = 1, N = 4096, K = 14336 17.0 us, with four stages 10.4.
@@ -1970,12 +1970,16 @@ __global__ __launch_bounds__(64 * WAVES) void packed_skinny_kernel(PackedArgs p)
   const int live = nb_last - nb0 + 1;
   auto col_lo = [&](int n) { return (n == 0 && (h0 & 1)) ? 8 : 0; };
   auto col_hi = [&](int n) { return n >= live ? 0 : (n == live - 1 && (h1 & 1)) ? 8 : 16; };
-  int64_t b_off[NBW];
+  // Tile n's base is the wave's (scalar), its lanes' offsets 32 bits.
+  const bool dead_lo = (h0 & 1) && (lane & 15) < 8, dead_hi = (h1 & 1) && (lane & 15) >= 8;
+  const int8_t *b_tile[NBW];
+  uint32_t b_lane[NBW];
 #pragma unroll
   for (int n = 0; n < NBW; ++n) {
-    const int t = min(n, live - 1), c = lane & 15;
-    const bool dead = c < col_lo(t) || c >= col_hi(t);
-    b_off[n] = (int64_t)(nb0 + t) * p.kbt * 1024 + (dead ? lane ^ 8 : lane) * 16;
+    const bool dead = ((n == 0 || live == 1) && dead_lo) || (n >= live - 1 && dead_hi);
+    b_tile[n] = n == 0 ? Bb + (int64_t)nb0 * p.kbt * 1024
+                       : b_tile[n - 1] + (n < live ? (int64_t)p.kbt * 1024 : 0);
+    b_lane[n] = (uint32_t)(dead ? lane ^ 8 : lane) * 16;
   }
   v4i acc[MB][NBW];
 #pragma unroll
@@ -1990,7 +1994,7 @@ __global__ __launch_bounds__(64 * WAVES) void packed_skinny_kernel(PackedArgs p)
     const int kb = first + s * WAVES;
 #pragma unroll
     for (int n = 0; n < NBW; ++n)
-      bv[n] = __builtin_nontemporal_load((const v4i *)(Bb + b_off[n] + (int64_t)kb * 1024));
+      bv[n] = __builtin_nontemporal_load((const v4i *)(b_tile[n] + (int64_t)kb * 1024 + b_lane[n]));
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) av[mb] = *(const v4i *)(a_src[mb] + min(kb * 64 + acol, p.K - 16));
   };
@@ -2003,10 +2007,15 @@ __global__ __launch_bounds__(64 * WAVES) void packed_skinny_kernel(PackedArgs p)
   };
   // Whole rounds of S blocks have no branch around a load (it makes the
   // compiler wait for every load in flight); the last round loads only the
-  // blocks that are left.
-  if (steps > 0) {
+  // blocks that are left. Waves with fewer blocks than stages load each once:
+  // filling the other stages with the last block again, and 64-bit addresses
+  // per lane and tile, cost short calls up to a quarter (HIP graph per call
+  // with both and with neither: 64 x 8192 x 512 6.37 and 4.64 us, 59 x 2448 x
+  // 512 in 4 batches 6.05 and 5.37, 16 x 14336 x 512 3.34 and 3.04, 7 x 1600 x
+  // 608 in 11 batches 3.75 and 3.39).
+  if (steps >= S) {
 #pragma unroll
-    for (int s = 0; s < S; ++s) load(min(s, steps - 1), a[s], b[s]);
+    for (int s = 0; s < S; ++s) load(s, a[s], b[s]);
     int s0 = 0;
     for (; s0 + 2 * S <= steps; s0 += S) {
 #pragma unroll
@@ -2023,6 +2032,14 @@ __global__ __launch_bounds__(64 * WAVES) void packed_skinny_kernel(PackedArgs p)
 #pragma unroll
     for (int s = 0; s < S; ++s)
       if (s0 + s + S < steps) multiply(a[s], b[s]);
+  } else {
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+      if (s < steps) load(s, a[s], b[s]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+      if (s < steps) multiply(a[s], b[s]);
   }
 
   // 16x16 accumulator layout: element e of lane l is row 4*(l/16) + e,
