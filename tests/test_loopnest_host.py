@@ -502,3 +502,25 @@ def test_memory_bounds_are_counted_at_run_time():
     assert "if (++vt_iters > 777ULL) { atomicOr(vt_status, %d); return; }" \
         % ln.STATUS_ITERATIONS in src
     assert any("counted" in n for n in info["notes"])
+
+
+def test_tiled_nests_report_and_bound_what_their_threads_run():
+    """A nest on LDS tiles runs whole workgroups, each thread the steps of
+    several cells: the reported threads are those launched, a thread's steps of
+    all its cells stay within the cap (one row a thread at the least), and an
+    annotation the tiles replace is noted."""
+    decl = {b: {"dtype": "float64", "shape": (500, 500)} for b in "ABC"}
+    stmt = ln.matmul_stmt(500, 500, 500)
+    stmt["body"]["body"]["ann"] = "unrolled"
+
+    def rows(info):
+        return sum("vt_acc%d = *vt_out%d;" % (r, r) in info["source"] for r in range(8))
+    info = ln.emit_kernel(stmt, decl)
+    assert rows(info) > 1 and info["threads"] == info["grid"][0] * info["block"][0]
+    assert any("unrolled on i2" in n for n in info["notes"])
+    for cap in (500, 999, 1000, 1999, 2000):
+        capped = ln.emit_kernel(stmt, decl, max_iterations=cap)
+        assert rows(capped) == max(r for r in (1, 2, 4) if r * 500 <= cap), cap
+        assert capped["threads"] == capped["grid"][0] * capped["block"][0]
+    with pytest.raises(ln.LoopNestError, match="beyond the cap"):
+        ln.emit_kernel(stmt, decl, max_iterations=499)

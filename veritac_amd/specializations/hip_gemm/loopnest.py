@@ -62,7 +62,7 @@ integer division or modulo by zero yields 0; either event sets a bit in a status
 the call returns, and the offending store is skipped or read is 0.
 
 Bounded work. Each GPU thread runs at most MAX_THREAD_ITERATIONS iterations
-of sequential loops. Where interval arithmetic over the loop bounds gives an
+of sequential loops, those of every cell it owns counted. Where interval arithmetic over the loop bounds gives an
 upper bound on a thread's iterations, a nest above the cap is refused when
 it is emitted. Where it cannot (a bound that reads memory), every
 sequential loop counts its iterations, and a thread that reaches the cap
@@ -737,7 +737,7 @@ def _reads(e, out):
     return out
 
 
-def plan_tiled(stmt, mapped, buffers, layout):
+def plan_tiled(stmt, mapped, buffers, layout, max_iterations=MAX_THREAD_ITERATIONS):
     """How a reduction nest runs on LDS tiles, or None when it keeps the
     general lowering.
 
@@ -748,7 +748,8 @@ def plan_tiled(stmt, mapped, buffers, layout):
     guard), there is no integer division or modulo, and of the mapped loops
     the innermost, whose points become the lanes of a wave, has a read that
     changes with it and the steps but not with another one, the rows, so that
-    a workgroup reads it once for all its rows.
+    a workgroup reads it once for all its rows. A thread's rows times its
+    steps stay within max_iterations.
 
     Mapped iterations touch disjoint cells (threads_disjoint), so several may
     run in one thread, step by step; each cell meets its own steps in program
@@ -839,6 +840,8 @@ def plan_tiled(stmt, mapped, buffers, layout):
         return max(_SIZES[buffers[key[0]]["dtype"]], 1 if dot else 4)
 
     for per_wave in TILE_ROWS:
+        if per_wave > 1 and per_wave * steps > max_iterations:
+            continue
         groups = -(-row[2] // (per_wave * (BLOCK // WAVE)))
         workgroups = groups * chunks * _prod(m[2] for m in others)
         if workgroups >= TILE_WORKGROUPS:
@@ -1156,7 +1159,8 @@ def emit_kernel(stmt, buffers, name="loopnest", layout="dense",
     buffers: {name: {"dtype": one of DTYPES, "shape": (d0, ...)}} for every
     buffer the nest touches (shape is used by layout "dense" and for the
     parameter size checks). Returns a dict: source, kernel name, params (the
-    buffer names in parameter order), mapped loops, threads, grid, block and
+    buffer names in parameter order), mapped loops, threads (one per mapped
+    iteration, or whole workgroups of a nest on LDS tiles), grid, block and
     the suppression notes. `max_iterations` caps each thread's sequential
     loop iterations (at most MAX_THREAD_ITERATIONS).
     """
@@ -1202,11 +1206,15 @@ def emit_kernel(stmt, buffers, name="loopnest", layout="dense",
                                                DTYPES[buffers[b]["dtype"]], b) for b in params]
                     + ["int *__restrict__ vt_status"])
     em.lines.append('extern "C" __global__ __launch_bounds__(%d) void %s(%s) {' % (BLOCK, name, sig))
-    tiled = plan_tiled(stmt, mapped, buffers, layout)
+    tiled = plan_tiled(stmt, mapped, buffers, layout, max_iterations)
+    threads = total
     if tiled is not None:
         _Tiled(tiled, buffers, em.lines).emit()
         em.lines.append("}")
         blocks = tiled["workgroups"]
+        threads = blocks * BLOCK
+        notes += ["unrolled on %s: the LDS tiles' own unrolling runs it" % loop[1]
+                  for loop in seq_chain if loop[4] == "unrolled"]
     else:
         em.lines.append("  const long long vt_t = (long long)blockIdx.x * %d + threadIdx.x;" % BLOCK)
         em.lines.append("  if (vt_t >= %dLL) return;" % total)
@@ -1241,7 +1249,7 @@ def emit_kernel(stmt, buffers, name="loopnest", layout="dense",
     if blocks > 2**31 - 1:
         raise LoopNestError("%d mapped iterations exceed the launch limit" % total)
     return {"source": "\n".join(header + em.lines) + "\n", "kernel": name, "params": params,
-            "written": sorted(written), "mapped": [m[0] for m in mapped], "threads": total,
+            "written": sorted(written), "mapped": [m[0] for m in mapped], "threads": threads,
             "grid": (blocks, 1, 1), "block": (BLOCK, 1, 1), "notes": notes, "layout": layout}
 
 
