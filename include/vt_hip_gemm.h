@@ -211,6 +211,34 @@ int vt_gemm_check(int64_t M, int64_t N, int64_t K,
                   int32_t *variant_out, int32_t *k_split_out,
                   int64_t *scratch_bytes_out);
 
+/* The kernels a call runs (vt_gemm_route). */
+#define VT_ROUTE_NONE 0        /* nothing to compute                          */
+#define VT_ROUTE_VARIANT 1     /* the variant's own (vector variants)         */
+#define VT_ROUTE_VALU 2        /* one thread per output                       */
+#define VT_ROUTE_COPIES 3      /* A and B copied zero padded, a vector variant
+                                  over them, C copied out when N % 16         */
+#define VT_ROUTE_SKINNY 4      /* the decode kernel, operands read in place   */
+#define VT_ROUTE_TILES_64 5    /* 64x64 MFMA tiles, operands read in place    */
+#define VT_ROUTE_TILES_128 6   /* 128x128 MFMA tiles, operands read in place  */
+#define VT_ROUTE_PERSISTENT 7  /* the persistent 256x256 kernel over padded
+                                  copies of A and B, C written in place       */
+
+/*
+ * vt_gemm_route -- the kernels vt_gemm_i8 launches for a call vt_gemm_check
+ * accepts (same arguments and errors), its K slices (1 = unsplit, 0 = nothing
+ * to compute) and the workspace those kernels take, when at most scratch_limit
+ * bytes may be used: INT64_MAX for a stream with memory to spare, 0 for one
+ * that is captured before it has a workspace. Any output pointer may be NULL.
+ * No device call. No counterpart in the reference.
+ */
+int vt_gemm_route(int64_t M, int64_t N, int64_t K,
+                  int64_t lda, int64_t ldb, int64_t ldd, int64_t ldc,
+                  int64_t batch, int64_t stride_a, int64_t stride_b,
+                  int64_t stride_d, int64_t stride_c,
+                  int32_t has_d, int32_t variant, int32_t k_split,
+                  int64_t scratch_limit, int32_t *route_out,
+                  int32_t *k_slices_out, int64_t *scratch_bytes_out);
+
 /* vt_gemm_select flags. */
 #define VT_SELECT_ALIGNED 1   /* A and B 16-byte aligned (else: unaligned) */
 #define VT_SELECT_B_SHARED 2  /* batch > 1 shares one B (stride_b == 0)    */

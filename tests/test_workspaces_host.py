@@ -3,6 +3,7 @@ against a HIP runtime that only logs (fake_hip.cpp), so what it launches and
 allocates, and in which order host threads do, can be checked without a GPU.
 Operand addresses are made up and never read."""
 import json
+import math
 import os
 import random
 import subprocess
@@ -199,3 +200,36 @@ print(json.dumps(out))
         plan = hg.make_plan(m, n, k, batch=batch, variant=hg.PACKED_VARIANT)
         want = hg.packed_columns(plan)[1] * hg.packed_split(plan)[0] * batch
         assert "packed_skinny" in first[3] and int(first[3].split(" ")[0]) == want, (m, n, k, batch)
+
+
+@pytest.mark.parametrize("variant", ["auto", "generic", "padded", "mfma_128x128", "mfma_256x128",
+                                     "mfma_256x256", "skinny", hg.PACKED_VARIANT])
+def test_launched_workgroups_are_the_reported_ones(run, variant):
+    """required_resources counts the workgroups the library launches (copies
+    and sums of K slices aside), for plans on either side of the routes' rules."""
+    rng, calls, plans = random.Random(17), [], []
+    while len(calls) < 120:
+        m, n, k = (int(round(math.exp(rng.uniform(math.log(16), math.log(hi))))) for hi in (9000, 9000, 16000))
+        if variant not in ("auto", "generic", "padded") or rng.random() < 0.4:
+            n, k = n // 16 * 16, k // 16 * 16
+        m = min(m, 64) if variant == "skinny" else m
+        batch = 1 if rng.random() < 0.7 else rng.randint(2, 20)
+        shared = variant != hg.PACKED_VARIANT and rng.random() < 0.5
+        if m * n * batch < 2**29:
+            plans.append(hg.make_plan(m, n, k, batch=batch, b_shared=shared, variant=variant))
+            v, ks = plans[-1]["variant"], plans[-1]["k_split"]
+            calls.append((m, n, k, batch, shared, v, ks))
+    got = run("""
+out = []
+for m, n, k, batch, shared, v, ks in %r:
+    fake.fake_reset()
+    if v == "skinny_packed":
+        packed(m, n, k, batch)
+    else:
+        gemm(m, n, k, v, batch=batch, shared=shared)
+    out.append([e[3] for e in launches()])
+print(json.dumps(out))
+""" % (calls,))
+    for plan, names in zip(plans, got):
+        gemms = [e.split(" ", 1) for e in names if "pad_i8" not in e and "unpad" not in e and "reduce" not in e]
+        assert sum(int(g[0]) for g in gemms) == hg.required_resources(plan)[1], (plan, names)

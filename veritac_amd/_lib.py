@@ -37,7 +37,7 @@ VARIANT_IDS = {
 VARIANTS = tuple(VARIANT_IDS)
 
 # Every function include/vt_hip_gemm.h declares.
-EXPORTS = ("vt_gemm_i8", "vt_gemm_i8_noalloc", "vt_gemm_check", "vt_gemm_select", "vt_variant_info", "vt_variant_name",
+EXPORTS = ("vt_gemm_i8", "vt_gemm_i8_noalloc", "vt_gemm_check", "vt_gemm_route", "vt_gemm_select", "vt_variant_info", "vt_variant_name",
            "vt_last_error", "vt_sync", "vt_device_count", "vt_abi_version", "vt_replay_i8",
            "vt_device_query", "vt_packed_b_size", "vt_pack_b_i8", "vt_gemm_i8_packed",
            "vt_rtc_compile", "vt_rtc_code_size", "vt_rtc_launch", "vt_rtc_release")
@@ -100,6 +100,9 @@ def _declare(lib):
     lib.vt_gemm_check.argtypes = [i64] * 12 + [i32, i32, i32, pi32, pi32,
                                                 ctypes.POINTER(ctypes.c_int64)]
     lib.vt_gemm_check.restype = ctypes.c_int
+    lib.vt_gemm_route.argtypes = [i64] * 12 + [i32, i32, i32, i64, pi32, pi32,
+                                               ctypes.POINTER(ctypes.c_int64)]
+    lib.vt_gemm_route.restype = ctypes.c_int
     lib.vt_gemm_select.argtypes = [i64, i64, i64, i64, i64, i64, i32, pi32, pi32]
     lib.vt_gemm_select.restype = ctypes.c_int
     lib.vt_variant_info.argtypes = [i32, pi32, pi32, pi32, pi32, pi32]
@@ -206,6 +209,23 @@ def gemm_check(M, N, K, lda, ldb, ldd, ldc, batch=1, stride_a=0, stride_b=0, str
         return st, last_error(), None, None, None
     names = {i: nm for nm, i in VARIANT_IDS.items()}
     return st, "ok", names[v.value], ks.value, ws.value
+
+
+# VT_ROUTE_* by number: the kernels a call runs
+ROUTES = ("none", "variant", "valu", "copies", "skinny", "tiles_64", "tiles_128", "persistent")
+
+
+def gemm_route(M, N, K, lda, ldb, ldd, ldc, batch=1, stride_a=0, stride_b=0, stride_d=0,
+               stride_c=0, has_d=False, variant="auto", k_split=0, scratch_limit=2**63 - 1):
+    """vt_gemm_route: (one of ROUTES, K slices, workspace bytes); raises what
+    vt_gemm_i8 would refuse."""
+    lib = load_library()
+    vid = VARIANT_IDS[variant] if isinstance(variant, str) else int(variant)
+    r, ks, ws = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int64()
+    check(lib.vt_gemm_route(M, N, K, lda, ldb, ldd, ldc, batch, stride_a, stride_b, stride_d,
+                            stride_c, int(bool(has_d)), vid, k_split, scratch_limit,
+                            ctypes.byref(r), ctypes.byref(ks), ctypes.byref(ws)), "vt_gemm_route")
+    return ROUTES[r.value], ks.value, ws.value
 
 
 def variant_info(name):

@@ -3728,21 +3728,13 @@ int launch_generic(const Problem &q, hipStream_t stream) {
 }
 
 
-int launch_large_aligned(const Problem &q, Scratch &scr, bool *done);
-int launch_ragged_slices(const Problem &q, Scratch &scr, bool *done);
+int launch_other_routes(const Problem &q, int32_t variant, Scratch &scr, bool *done);
 
 // The vector variants (operands already checked by vector_ok).
 int launch_vector(const Problem &q, int32_t variant, int32_t k_split, Scratch &scr) {
-  if (variant != VT_VARIANT_SKINNY && q.K % 64) {
-    bool done = false;
-    const int rc = launch_large_aligned(q, scr, &done);
-    if (rc || done) return rc;
-  }
-  if (variant == VT_VARIANT_MFMA_128x128 && q.K >= 1024) {
-    bool done = false;
-    const int rc = launch_ragged_slices(q, scr, &done);
-    if (rc || done) return rc;
-  }
+  bool done = false;
+  const int rc = launch_other_routes(q, variant, scr, &done);
+  if (rc || done) return rc;
   switch (variant) {
     case VT_VARIANT_MFMA_256x256: return launch_mfma<256, 256>(q, scr);
     case VT_VARIANT_MFMA_128x128: return launch_mfma128(q, scr);
@@ -3908,87 +3900,125 @@ int launch_direct_tiles(const Problem &r, const DirectPlan &d, int32_t *w, hipSt
   return launch_reduce(ra, 1, stream);
 }
 
-// An aligned problem with K off 64 (which keeps it off the persistent kernels)
-// over padded copies, where that is the faster way and there is a workspace for
-// them; *done says whether it was launched.
-int launch_large_aligned(const Problem &q, Scratch &scr, bool *done) {
-  const Problem r = mfma_fold(q);
-  LargeLayout L;
-  *done = false;
-  if (scr.copies_taken || !large_padded(r, true, &L) || !optional_workspace(scr))
-    return VT_OK;
-  void *w = nullptr;
-  if (scr.take(kPadded, (size_t)(L.a_bytes + L.b_bytes), &w, true) != VT_OK) {
-    (void)hipGetLastError();
-    g_err.clear();
-    return VT_OK;
-  }
-  *done = true;
-  return launch_large_padded(r, L, (int8_t *)w, (hipStream_t)scr.stream, scr.st->num_cus);
+// The kernels of a call where they are not its variant's own (VT_ROUTE_*, else
+// VT_ROUTE_VARIANT), and the bytes of workspace they take.
+struct Route {
+  int32_t kind = VT_ROUTE_VARIANT;
+  int64_t scratch = 0;
+  DirectPlan d;      // VT_ROUTE_SKINNY and VT_ROUTE_TILES_*
+  LargeLayout L;     // VT_ROUTE_PERSISTENT
+};
+
+Route large_route(const LargeLayout &L) {
+  Route t;
+  t.kind = VT_ROUTE_PERSISTENT;
+  t.L = L;
+  t.scratch = L.a_bytes + L.b_bytes;
+  return t;
 }
 
-// Runs a problem without copies where that is the faster way; *done says
-// whether it was launched. scratch_limit: bytes of scratch the call may take;
-// optional: as for get_workspace.
-int launch_direct(const Problem &q, int64_t scratch_limit, bool optional, Scratch &scr, bool *done) {
+Route direct_route(const DirectPlan &d) {
+  Route t;
+  t.kind = d.kind == kDirectSkinny ? VT_ROUTE_SKINNY
+           : d.kind == kDirectTiles64 ? VT_ROUTE_TILES_64 : VT_ROUTE_TILES_128;
+  t.d = d;
+  t.scratch = d.scratch;
+  return t;
+}
+
+// The generic and padded variants: without their own kernels where that is the
+// faster way, in at most `limit` bytes of workspace.
+Route any_route(const Problem &q, int64_t limit) {
   DirectPlan d = direct_plan(q);
-  *done = false;
-  if (d.kind == kDirectNone) return VT_OK;
-  hipStream_t stream = (hipStream_t)scr.stream;
+  if (d.kind == kDirectNone) return Route();
   const Problem r = mfma_fold(q);
-  *done = true;
-  void *w = nullptr;
   LargeLayout L;
-  if (d.kind != kDirectSkinny && d.ks == 1 && large_padded(r, false, &L) && L.a_bytes + L.b_bytes <= scratch_limit) {
-    if (L.a_bytes + L.b_bytes == 0 ||
-        scr.take(kPadded, (size_t)(L.a_bytes + L.b_bytes), &w, optional) == VT_OK)
-      return launch_large_padded(r, L, (int8_t *)w, stream, scr.st->num_cus);
-    (void)hipGetLastError();
-    g_err.clear();
-  }
-  if (d.scratch > scratch_limit) {
+  if (d.kind != kDirectSkinny && d.ks == 1 && large_padded(r, false, &L) && L.a_bytes + L.b_bytes <= limit)
+    return large_route(L);
+  if (d.scratch > limit) {
     d.kind = d.kind == kDirectSkinny ? kDirectTiles64 : d.kind;
     direct_slices(r, 1, &d);
   }
-  if (d.kind == kDirectSkinny) {
-    const int rc = launch_skinny_cfg<kSkinnyNB, kSkinnyWaves, kSkinnyU, true>(q, 0, scr);
-    if (rc == VT_OK || d.ks == 1) return rc;
-    // No workspace (none yet on a stream being captured, or no memory): the
-    // tiles need none.
-    (void)hipGetLastError();
-    g_err.clear();
-    d.kind = kDirectTiles64;
-    direct_slices(r, 1, &d);
-  } else if (d.scratch > 0 && scr.take(kPartials, (size_t)d.scratch, &w, optional) != VT_OK) {
-    (void)hipGetLastError();
-    g_err.clear();
-    direct_slices(r, 1, &d);
-  }
-  return launch_direct_tiles(r, d, (int32_t *)w, stream, scr.st->num_cus);
+  return direct_route(d);
 }
 
-// Few aligned tiles over a long K that does not divide into the MFMA split's
-// equal slices of whole 128-deep steps: slices of whole 64-deep ones, the last
-// one shorter, when the stream's workspace may be used. Calls in a row, unsplit
-// (already with the K tail's loads in flight, 69 us) against sliced: 84 x 1040 x
-// 14832 14 us, 128 x 512 x 4112 32 -> 11, 200 x 1008 x 15008 128 -> 16, 512 x
-// 4096 x 9008 78 -> 34 (first figures: with the check at the load).
-int launch_ragged_slices(const Problem &q, Scratch &scr, bool *done) {
-  *done = false;
+// The vector variants, in at most `limit` bytes of a workspace they could do
+// without. K off 64 keeps a problem off the persistent kernels: padded copies
+// where they are the faster way (`copies`: the call may take them). Few tiles
+// over a long K that does not divide into the MFMA split's equal slices of
+// whole 128-deep steps: slices of whole 64-deep ones, the last one shorter.
+// Calls in a row, unsplit against sliced: 84 x 1040 x 14832 69 and 14 us, 128 x
+// 512 x 4112 32 and 11, 200 x 1008 x 15008 128 and 16, 512 x 4096 x 9008 78 and
+// 34 (the first with the K tail's loads in flight, the others before).
+Route vector_route(const Problem &q, int32_t variant, int64_t limit, bool copies) {
   const Problem r = mfma_fold(q);
-  if (r.batch != 1 || mfma128_split(r) != 1) return VT_OK;
-  DirectPlan d = direct_plan(r);
-  if ((d.kind != kDirectTiles64 && d.kind != kDirectTiles128) || (d.ks < 4 && (d.ks < 2 || r.K < 8192)) ||
-      !optional_workspace(scr))
-    return VT_OK;
-  void *w = nullptr;
-  if (scr.take(kPartials, (size_t)d.scratch, &w, true) != VT_OK) {
-    (void)hipGetLastError();
-    g_err.clear();
-    return VT_OK;
+  LargeLayout L;
+  if (copies && variant != VT_VARIANT_SKINNY && q.K % 64 && large_padded(r, true, &L) &&
+      L.a_bytes + L.b_bytes <= limit)
+    return large_route(L);
+  if (variant == VT_VARIANT_MFMA_128x128 && q.K >= 1024 && r.batch == 1 && mfma128_split(r) == 1) {
+    const DirectPlan d = direct_plan(r);
+    if ((d.kind == kDirectTiles64 || d.kind == kDirectTiles128) && d.scratch <= limit &&
+        (d.ks >= 4 || (d.ks >= 2 && r.K >= 8192)))
+      return direct_route(d);
   }
+  return Route();
+}
+
+// Launches a route other than the variant's own; *done is false when there was
+// no workspace for it. optional: as for get_workspace.
+int launch_route(const Problem &q, const Route &t, bool optional, Scratch &scr, bool *done) {
+  hipStream_t stream = (hipStream_t)scr.stream;
+  const int num_cus = scr.st->num_cus;
+  const Problem r = mfma_fold(q);
   *done = true;
-  return launch_direct_tiles(r, d, (int32_t *)w, (hipStream_t)scr.stream, scr.st->num_cus);
+  int rc = VT_OK;
+  void *w = nullptr;
+  if (t.kind == VT_ROUTE_SKINNY) {
+    rc = launch_skinny_cfg<kSkinnyNB, kSkinnyWaves, kSkinnyU, true>(q, 0, scr);
+    if (rc == VT_OK || t.scratch == 0) return rc;
+  } else {
+    if (t.scratch > 0)
+      rc = scr.take(t.kind == VT_ROUTE_PERSISTENT ? kPadded : kPartials, (size_t)t.scratch, &w, optional);
+    if (rc == VT_OK)
+      return t.kind == VT_ROUTE_PERSISTENT
+                 ? launch_large_padded(r, t.L, (int8_t *)w, stream, num_cus)
+                 : launch_direct_tiles(r, t.d, (int32_t *)w, stream, num_cus);
+  }
+  (void)hipGetLastError();
+  g_err.clear();
+  *done = false;
+  return VT_OK;
+}
+
+// Runs a call on the kernels its route names, unless they are its variant's
+// own; *done says whether it was launched. Without the workspace of one route
+// (none yet on a stream being captured, no memory, or too much held already)
+// the next one takes less.
+int launch_other_routes(const Problem &q, int32_t variant, Scratch &scr, bool *done) {
+  *done = false;
+  const bool any = variant == VT_VARIANT_GENERIC || variant == VT_VARIANT_PADDED;
+  const bool optional = variant != VT_VARIANT_PADDED;
+  // A fixed scratch buffer holds what vt_gemm_check reported for the call; the
+  // generic variant reports none.
+  int64_t limit = scr.fixed && any ? scratch_need(q, variant, 0)
+                  : !optional      ? INT64_MAX
+                                   : (int64_t)kOptionalBytes;
+  bool asked = scr.fixed && any;
+  for (;;) {
+    const Route t = any ? any_route(q, limit) : vector_route(q, variant, limit, !scr.copies_taken);
+    if (t.kind == VT_ROUTE_VARIANT) return VT_OK;
+    if (t.scratch > 0 && optional && !asked) {
+      asked = true;
+      if (!optional_workspace(scr)) {
+        limit = 0;
+        continue;
+      }
+    }
+    const int rc = launch_route(q, t, optional, scr, done);
+    if (rc || *done) return rc;
+    limit = t.scratch - 1;
+  }
 }
 
 // One validated vt_gemm_i8 problem and the kernel it runs.
@@ -4074,14 +4104,8 @@ int prepare_gemm(const int8_t *A, const int8_t *B, const int32_t *D, int32_t *C,
 
 int launch_gemm(const GemmCall &c, Scratch &scr) {
   if (c.variant == VT_VARIANT_GENERIC || c.variant == VT_VARIANT_PADDED) {
-    // A fixed scratch buffer holds what vt_gemm_check reported for the call;
-    // the generic variant reports none.
-    const bool optional = c.variant == VT_VARIANT_GENERIC;
-    const int64_t limit = scr.fixed ? scratch_need(c.q, c.variant, c.k_split)
-                          : !optional ? INT64_MAX
-                                      : optional_workspace(scr) ? (int64_t)kOptionalBytes : 0;
     bool done = false;
-    const int rc = launch_direct(c.q, limit, optional, scr, &done);
+    const int rc = launch_other_routes(c.q, c.variant, scr, &done);
     if (rc || done) return rc;
   }
   if (c.variant == VT_VARIANT_GENERIC) return launch_generic(c.q, (hipStream_t)scr.stream);
@@ -4347,6 +4371,45 @@ int vt_gemm_check(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int
   }
   if (k_split_out) *k_split_out = ks;
   if (scratch_bytes_out) *scratch_bytes_out = c.empty ? 0 : scratch_need(c.q, c.variant, c.k_split);
+  return VT_OK;
+}
+
+int vt_gemm_route(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldd,
+                  int64_t ldc, int64_t batch, int64_t stride_a, int64_t stride_b, int64_t stride_d,
+                  int64_t stride_c, int32_t has_d, int32_t variant, int32_t k_split,
+                  int64_t scratch_limit, int32_t *route_out, int32_t *k_slices_out,
+                  int64_t *scratch_bytes_out) {
+  g_err.clear();
+  GemmCall c;
+  int rc = prepare_gemm(nullptr, nullptr, nullptr, nullptr, has_d != 0, false, M, N, K, lda, ldb,
+                        ldd, ldc, batch, stride_a, stride_b, stride_d, stride_c, variant, k_split,
+                        "vt_gemm_route", &c);
+  if (rc) return rc;
+  if (scratch_limit < 0) return fail(VT_EINVAL, "negative scratch limit");
+  int32_t kind = VT_ROUTE_NONE, slices = 0;
+  int64_t scratch = 0;
+  if (!c.empty) {
+    const bool any = c.variant == VT_VARIANT_GENERIC || c.variant == VT_VARIANT_PADDED;
+    if (c.variant != VT_VARIANT_PADDED && scratch_limit > (int64_t)kOptionalBytes)
+      scratch_limit = (int64_t)kOptionalBytes;
+    const Route t = any ? any_route(c.q, scratch_limit) : vector_route(c.q, c.variant, scratch_limit, true);
+    kind = t.kind;
+    slices = 1;
+    scratch = t.scratch;
+    if (kind == VT_ROUTE_SKINNY || kind == VT_ROUTE_TILES_64 || kind == VT_ROUTE_TILES_128) {
+      slices = t.d.ks;
+    } else if (kind == VT_ROUTE_VARIANT) {
+      scratch = scratch_need(c.q, c.variant, c.k_split);
+      if (c.variant == VT_VARIANT_GENERIC) kind = VT_ROUTE_VALU;
+      else if (c.variant == VT_VARIANT_PADDED) kind = VT_ROUTE_COPIES;
+      else if (c.variant == VT_VARIANT_SKINNY)
+        slices = skinny_geometry<kSkinnyNB, kSkinnyWaves, kSkinnyU>(c.q, c.k_split).ks;
+      else slices = mfma_split_for(c.q, c.variant);
+    }
+  }
+  if (route_out) *route_out = kind;
+  if (k_slices_out) *k_slices_out = slices;
+  if (scratch_bytes_out) *scratch_bytes_out = scratch;
   return VT_OK;
 }
 

@@ -254,6 +254,123 @@ def _folded(plan):
     return (m * b, 1) if plan["b_shared"] and b > 1 else (m, b)
 
 
+# ---------------------------------------------------------------------------
+# Routes: the kernels a row-major plan runs where they are not its variant's
+# ---------------------------------------------------------------------------
+
+OPTIONAL_BYTES = 256 << 20    # kOptionalBytes in the HIP source
+ROUTE_TILES = {"tiles_64": 64, "tiles_128": 128, "persistent": 256}
+
+
+def _large_padded(m, n, k, b, b_mats, aligned):
+    """(padded n, padded k, bytes of the copies) of a folded problem that runs
+    on the persistent kernel over padded copies, else None (large_padded in
+    the HIP source, contiguous operands)."""
+    if min(m, n, k) < 256 or n >= 2**29 or b > 65535:
+        return None
+    k_p, n_p = -(-k // 256) * 256, -(-n // 16) * 16
+    a_bytes = -(-b * m * k_p // 256) * 256 if k_p != k else 0
+    b_bytes = -(-b_mats * k_p * n_p // 256) * 256 if k_p != k or n_p != n else 0
+    if 256 * k_p >= 2**32 - 4096 or 64 * n_p >= 2**32 - 4096:
+        return None
+    tiles = -(-m // 256) * -(-n // 256) * b
+    if tiles > 2**31 - 1:
+        return None
+    busy, rounds = min(tiles, NUM_CUS) / NUM_CUS, float(-(-tiles // NUM_CUS))
+    one = 575.0 + (530.0 * (busy - 0.5) if busy > 0.5 else 0.0)
+    padded = (rounds * (k_p // 64) * one + 2.0 * (a_bytes + b_bytes) / 4500.0 + 6000.0
+              + 4.0 * m * n * b / 5000.0 / rounds)
+    t128 = -(-m // 128) * -(-n // 128) * b
+    direct = 4000.0 + -(-k // 64) * (150.0 + 290.0 * -(-t128 // NUM_CUS) if aligned
+                                     else 200.0 + 560.0 * max(t128 / NUM_CUS, 0.4))
+    return (n_p, k_p, a_bytes + b_bytes) if padded < direct else None
+
+
+def _direct_route(plan, limit):
+    """(route, K slices, workspace bytes) of a problem read in place, or None
+    (direct_plan in the HIP source, contiguous operands)."""
+    m, n, k, batch = plan["m"], plan["n"], plan["k"], plan["batch"]
+    if (k < 16 or n < 16 or batch > 65535 or 256 * k >= 2**32 - 4096 or 64 * n >= 2**32 - 4096
+            or max(m, n, k) >= 2**30):
+        return None
+    fm, fb = _folded(plan)
+    if k < 128 and fm * n * k * fb < 1 << 24:
+        return None
+    pitch = -(-n // 4) * 4
+    t64, t128 = (-(-fm // t) * -(-n // t) * fb for t in (64, 128))
+    if m <= 16 or (m <= SKINNY_MAX_M and k >= 1024 and -(-n // 128) * batch < NUM_CUS):
+        ks = skinny_split(dict(plan, k_split=0))[0]
+        scratch = batch * ks * m * pitch * 4 if ks > 1 else 0
+        return ("skinny", ks, scratch) if scratch <= limit else ("tiles_64", 1, 0)
+    long_k = k >= 4096 and fb == 1
+    route = "tiles_128" if long_k or t64 > 512 else "tiles_64"
+    tiles, ks = t128 if route == "tiles_128" else t64, 1
+    if fb == 1:
+        while ks < 16 and 2 * ks * tiles <= NUM_CUS and k // (2 * ks) >= 512:
+            ks *= 2
+        if not long_k and (k - k // ks) // 64 < 20:
+            ks = 1
+    kc = -(-(-(-k // ks)) // 64) * 64       # whole 64-deep steps, the last slice at least 16 deep
+    ks = -(-k // kc)
+    if ks > 1 and k - (ks - 1) * kc < 16:
+        ks -= 1
+    scratch = ks * fm * pitch * 4 if ks > 1 else 0
+    return (route, ks, scratch) if scratch <= limit else (route, 1, 0)
+
+
+def gemm_route(plan, limit=2**63 - 1):
+    """(route, K slices, workspace bytes) of the kernels vt_gemm_i8 launches for
+    a row-major plan on contiguous operands: one of _lib.ROUTES, with at most
+    `limit` bytes of workspace (vt_gemm_route in the HIP source, which gives
+    "variant", "valu" and "copies" their own slices and bytes; 1 and 0 here)."""
+    m, n, k, batch, variant = plan["m"], plan["n"], plan["k"], plan["batch"], plan["variant"]
+    if variant != "padded":
+        limit = min(limit, OPTIONAL_BYTES)
+    fm, fb = _folded(plan)
+    b_mats = 1 if fb == 1 or plan["b_shared"] else fb
+    if variant in ("generic", "padded"):
+        own = ("valu" if variant == "generic" else "copies", 1, 0)
+        route = _direct_route(plan, 2**63 - 1)
+        if route is None:
+            return own
+        if route[0] != "skinny" and route[1] == 1:
+            large = _large_padded(fm, n, k, fb, b_mats, False)
+            if large is not None and large[2] <= limit:
+                return "persistent", 1, large[2]
+        return _direct_route(plan, limit)
+    if variant.startswith("mfma"):
+        if k % 64:
+            large = _large_padded(fm, n, k, fb, b_mats, True)
+            if large is not None and large[2] <= limit:
+                return "persistent", 1, large[2]
+        if (variant == "mfma_128x128" and k >= 1024 and fb == 1
+                and mfma_k_split(dict(plan, routed=True)) == 1):
+            route = _direct_route(dict(plan, m=fm, batch=1), 2**63 - 1)
+            if (route is not None and route[0] != "skinny" and route[2] <= limit
+                    and (route[1] >= 4 or (route[1] >= 2 and k >= 8192))):
+                return route
+    return "variant", 1, 0
+
+
+def launched_plan(plan):
+    """The plan whose kernels a row-major plan's call runs on a stream with
+    workspaces (outside capture): the plan itself, or one with `routed` set and
+    the tiles (`tile`), K slices (`slices`), operands read in place
+    (`in_place`) or bytes of padded copies (`copied`) of its route."""
+    if plan.get("routed") or plan.get("packed_b") or plan["variant"] == PACKED_VARIANT:
+        return plan
+    route, ks, scratch = gemm_route(plan)
+    if route == "skinny":
+        return dict(plan, variant="skinny", k_split=0, routed=True, in_place=True)
+    if route == "persistent":
+        return dict(plan, n=-(-plan["n"] // 16) * 16, k=-(-plan["k"] // 256) * 256, k_split=0,
+                    variant="mfma_256x256", routed=True, tile=256, slices=1, copied=scratch)
+    if route in ROUTE_TILES:
+        return dict(plan, variant="mfma_128x128", k_split=0, routed=True, in_place=True,
+                    tile=ROUTE_TILES[route], slices=ks)
+    return plan
+
+
 def _k_split_for_tiles(m, n, k, b, tm, tn):
     """mfma_k_split<tm, tn> in the HIP source, on a folded problem: a k of at
     least 1024 over at most 64 tiles is cut into up to 16 slices of whole
@@ -282,6 +399,8 @@ def mfma_k_split(plan):
     variant = plan["variant"]
     if not variant.startswith("mfma"):
         return 1
+    if "slices" in plan:
+        return plan["slices"]
     tm, tn = mfma_tile_shape(plan)
     m, b = _folded(plan)
     return _k_split_for_tiles(m, plan["n"], plan["k"], b, tm, tn)
@@ -327,10 +446,13 @@ def _mfma_parts(plan):
     """(the whole rows or columns on the persistent 256x256 kernel, the rest
     on 128x128 tiles) as two plans, or None when neither mfma_split_rows nor
     mfma_split_cols splits the plan."""
+    if "tile" in plan:
+        return None
     rows = mfma_split_rows(plan)
     cols = 0 if rows else mfma_split_cols(plan)
     if not rows and not cols:
         return None
+    plan = dict(plan, routed=True)
     if plan["b_shared"] and plan["batch"] > 1:
         plan = dict(plan, m=plan["m"] * plan["batch"], batch=1)
     if rows:
@@ -450,6 +572,8 @@ def mfma_quarter_tiles(plan):
 
 def mfma_tile_shape(plan):
     """(rows, columns) of the output tiles an MFMA plan's kernel runs."""
+    if "tile" in plan:
+        return plan["tile"], plan["tile"]
     tm, tn = TILES[plan["variant"]][:2]
     if mfma_quarter_tiles(plan):
         return 64, 64
@@ -489,8 +613,11 @@ def required_resources(plan):
     The analogue of backend.py:97-104 (scratchpad / accumulator rows) for a
     gfx950 launch: LDS is the on-chip buffer a workgroup needs, workgroups
     the grid size. The persistent 256x256 kernel launches one workgroup per
-    CU (at most) whatever the tile count, and so does its 256x128 form.
+    CU (at most) whatever the tile count, and so does its 256x128 form. A plan
+    whose call runs other kernels than its variant's own (gemm_route) counts
+    those, as on a stream with workspaces.
     """
+    plan = launched_plan(plan)
     variant = plan["variant"]
     tm, tn, _, _, lds = TILES[variant]
     m, n, batch = plan["m"], plan["n"], plan["batch"]
@@ -648,6 +775,10 @@ def validate_plan(plan):
 _MODEL_MFMA_EFF = {"mfma_256x256": 0.70, "mfma_256x128": 0.60, "mfma_128x128": 0.45,
                    "skinny": 0.25, "skinny_packed": 0.25, "generic": 0.002}
 
+# Share of that left when operands off the 16-byte grid are read in place (a
+# slice of 128x128 tiles takes 0.56 us per CU against 0.29 of aligned ones).
+_MODEL_IN_PLACE = 0.5
+
 
 def algorithmic_bytes(plan):
     """A once + B once (shared B counted once) + C written + D read."""
@@ -667,8 +798,12 @@ def modeled_counts(plan):
     lds, wgs = required_resources(plan)
     ops = 2 * b * m * n * k
     alg = algorithmic_bytes(plan)
+    run = launched_plan(plan)
     parts = _mfma_parts(plan) if variant.startswith("mfma") else None
-    if parts is not None:
+    if run is not plan:
+        # padded copies: read once, written once
+        l2_bytes = modeled_counts(run)["bytes_l2_modeled"] + 2 * run.get("copied", 0)
+    elif parts is not None:
         l2_bytes = sum(modeled_counts(p)["bytes_l2_modeled"] for p in parts)
     elif variant.startswith("mfma"):
         m_eff, b_eff = (m * b, 1) if (plan["b_shared"] and b > 1) else (m, b)
@@ -713,8 +848,7 @@ def modeled_counts(plan):
 def _padded_copy_bytes(plan, inner):
     """Bytes the padded variant moves besides its inner product: each copied
     operand read and its padded copy written, and, when C is copied out, C'
-    read back and C written (plus D). The library reads the operands in place
-    where that is faster, so this is the most it moves."""
+    read back and C written (plus D)."""
     m, n, k, b = plan["m"], plan["n"], plan["k"], plan["batch"]
     n_p, k_p = inner["n"], inner["k"]
     b_mats = 1 if plan["b_shared"] or b == 1 else b
@@ -744,6 +878,11 @@ def modeled_objective(plan, counts):
     """
     m, n, k, b = plan["m"], plan["n"], plan["k"], plan["batch"]
     variant = plan["variant"]
+    run = launched_plan(plan)
+    if run is not plan:
+        t, wgs = modeled_objective(run, modeled_counts(run))
+        copied = run.get("copied", 0)
+        return t + (2 * copied / PEAK_HBM_BYTES + _LAUNCH_S if copied else 0.0), wgs
     if variant == "padded":
         # the inner product's objective, plus the copies at the HBM rate and
         # their launches (one for the operands, one for the copy-out)
@@ -780,6 +919,8 @@ def modeled_objective(plan, counts):
     waves = -(-units // NUM_CUS)
     fill = units / (waves * NUM_CUS) if units else 1.0
     eff = _MODEL_MFMA_EFF[variant] * (fill if variant.startswith("mfma") else 1.0)
+    if plan.get("in_place"):
+        eff *= _MODEL_IN_PLACE
     t_compute = padded_ops / (PEAK_INT8_OPS * eff)
     t_memory = counts["bytes_algorithmic"] / (PEAK_HBM_BYTES * min(1.0, wgs / NUM_CUS))
     t = max(t_compute, t_memory)
@@ -860,7 +1001,14 @@ def native_check(plan):
         return False, ("vt_gemm_check would run %r for a %r plan (fail-closed)"
                        % (variant, plan["variant"]))
     how = ""
-    parts = _mfma_parts(dict(plan, variant=variant))
+    run = launched_plan(dict(plan, variant=variant))
+    if run["variant"] == "skinny" and run.get("in_place"):
+        how = "; operands in place on the decode kernel"
+    elif run.get("in_place"):
+        how = "; operands in place on %dx%d tiles, K in %d" % (run["tile"], run["tile"], run["slices"])
+    elif "copied" in run:
+        how = "; on the persistent 256x256 kernel over %d bytes of padded copies" % run["copied"]
+    parts = _mfma_parts(run) if run["variant"].startswith("mfma") else None
     if parts is not None and parts[0]["n"] == parts[1]["n"]:
         how = "; %d rows on the persistent 256x256 kernel, %d on 128x128 tiles" % (
             parts[0]["m"], parts[1]["m"])
@@ -920,7 +1068,10 @@ def optimize(m, n, k, *, batch=1, b_shared=False, has_d=False, d_max_abs=0,
         correct = [c for c in eligible if c["measured_correct"]]
         winner = min(correct, key=lambda c: c["measured_ms"])["plan"] if correct else None
     else:
-        winner = min(eligible, key=lambda c: c["objective"])["plan"] if eligible else None
+        # off the 16-byte grid the generic and padded variants run the same
+        # kernels; padded keeps its workspace under capture
+        winner = min(eligible, key=lambda c: (c["objective"], c["plan"]["variant"] == "generic")
+                     )["plan"] if eligible else None
     return {"candidates": candidates, "winner": winner}
 
 
