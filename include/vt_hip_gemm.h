@@ -109,7 +109,8 @@ extern "C" {
  * products VT_VARIANT_PADDED copies the operands the vector variants cannot
  * read, zero padded, to a workspace the library allocates once per (device,
  * stream) and grows as needed, and writes C directly (without a workspace, as
- * on a stream captured before it has one, it reads them in place).
+ * on a stream captured before it has one, it reads them in place, or runs one
+ * thread per output where N or K is below 16).
  * vt_gemm_check reports what copies of all three would take. For aligned
  * shapes VT_VARIANT_AUTO picks VT_VARIANT_SKINNY for M <= 16, and for
  * M <= 64 when K >= 512 and ceil(N / 128) * batch < 256 (the skinny kernel

@@ -202,6 +202,25 @@ print(json.dumps(out))
         assert "packed_skinny" in first[3] and int(first[3].split(" ")[0]) == want, (m, n, k, batch)
 
 
+def test_captured_copies_do_not_depend_on_what_larger_calls_took(run):
+    """A stream warmed up with a larger padded call, which reads its operands
+    in place and takes no workspace, captures calls that would copy theirs:
+    they run one thread per output."""
+    got = run("""
+gemm(2000, 2001, 2003)
+fake.fake_capture(STREAM, 1)
+fake.fake_reset()
+gemm(40000, 8, 200)
+gemm(4000, 5000, 9, "padded")
+fake.fake_capture(STREAM, 0)
+gemm(40000, 8, 200)
+print(json.dumps([[e[3] for e in launches()], allocated()]))
+""")
+    names, sizes = got
+    assert "generic_kernel" in names[0] and "generic_kernel" in names[1]
+    assert ["pad_i8" in names[2], "unpad" in names[-1], len(sizes)] == [True, True, 1]
+
+
 @pytest.mark.parametrize("variant", ["auto", "generic", "padded", "mfma_128x128", "mfma_256x128",
                                      "mfma_256x256", "skinny", hg.PACKED_VARIANT])
 def test_launched_workgroups_are_the_reported_ones(run, variant):

@@ -3686,6 +3686,12 @@ int launch_padded(const Problem &q, Scratch &scr) {
   if (a_bytes + b_bytes + c_bytes > 0) {
     void *w = nullptr;
     int rc = scr.take(kPadded, (size_t)(a_bytes + b_bytes + c_bytes), &w);
+    if (rc == VT_EUNSUPPORTED && !scr.fixed) {
+      // The stream is captured and has no workspace of that size: larger calls
+      // that read their operands in place never gave it one.
+      g_err.clear();
+      return launch_generic(q, s);
+    }
     if (rc) return rc;
     scr.copies_taken = true;   // the inner product may not take that workspace again
     int8_t *Ap = (int8_t *)w, *Bp = Ap + a_bytes;
