@@ -36,26 +36,33 @@ def wrapped(x):
 
 
 def check(dev, variant, m, n, k, batch=1, shared=False, a_off=0, lda=None, b_off=0, ldb=None,
-          ldc=None, with_d=True):
+          ldc=None, shared_a=False, gap_a=0, route=None):
     """C = A.B and, in place, C = D + A.B through vt_gemm_i8 on flat buffers at
-    the given byte offsets and pitches; row padding and the guard stay."""
-    say(variant, m, n, k, batch, shared, a_off, lda, b_off, ldb, ldc)
+    the given byte offsets, pitches and gap between A's batches; row padding and
+    the guard stay. route: the kernels the call is to run (_lib.ROUTES)."""
+    say(variant, m, n, k, batch, shared, a_off, lda, b_off, ldb, ldc, shared_a, gap_a)
     lda, ldb, ldc = lda or k, ldb or n, ldc or n
+    strides = (0, 0, 0, 0)
+    if batch > 1:
+        strides = (0 if shared_a else m * lda + gap_a, 0 if shared else k * ldb, m * ldc, m * ldc)
+    if route is not None:
+        got = _lib.gemm_route(m, n, k, lda, ldb, ldc, ldc, batch, *strides, has_d=True, variant=variant)
+        assert got[0] == route, got
     g = torch.Generator(device=dev)
     g.manual_seed(m * 7 + n * 3 + k)
     bs = 1 if shared else batch
-    Af = torch.randint(-128, 128, (a_off + batch * m * lda,), generator=g, device=dev, dtype=torch.int8)
+    As = 1 if shared_a else batch
+    Af = torch.randint(-128, 128, (a_off + As * (m * lda + gap_a),), generator=g, device=dev, dtype=torch.int8)
     Bf = torch.randint(-128, 128, (b_off + bs * k * ldb,), generator=g, device=dev, dtype=torch.int8)
-    A = Af[a_off:].view(batch, m, lda)[:, :, :k]
+    A = Af[a_off:].view(As, m * lda + gap_a)[:, :m * lda].reshape(As, m, lda)[:, :, :k]
     B = Bf[b_off:].view(bs, k, ldb)[:, :, :n]
     AB = torch.matmul(A.double(), B.double())
     D = torch.randint(-2**31, 2**31, (batch * m * ldc + 64,), generator=g, device=dev, dtype=torch.int32)
-    for d in ([None, D] if with_d else [None]):
+    for d in (None, D):
         C = D.clone() if d is not None else torch.full_like(D, -2**31)
         before = C.clone()
         _lib.gemm_raw(Af.data_ptr() + a_off, Bf.data_ptr() + b_off, C.data_ptr() if d is not None else None,
-                      C.data_ptr(), m, n, k, lda, ldb, ldc, ldc, batch, m * lda if batch > 1 else 0,
-                      k * ldb if bs > 1 else 0, m * ldc if batch > 1 else 0, m * ldc if batch > 1 else 0,
+                      C.data_ptr(), m, n, k, lda, ldb, ldc, ldc, batch, *strides,
                       variant, 0, torch.cuda.current_stream().cuda_stream)
         torch.cuda.synchronize()
         got, old = C[:batch * m * ldc].view(batch, m, ldc), before[:batch * m * ldc].view(batch, m, ldc)
@@ -72,18 +79,19 @@ TILES = [(17, 16, 128), (65, 17, 129), (64, 63, 191), (100, 31, 143), (129, 65, 
 @pytest.mark.parametrize("m,n,k", TILES)
 @pytest.mark.parametrize("variant", ["generic", "padded"])
 def test_tiles_in_place(dev, variant, m, n, k):
-    check(dev, variant, m, n, k)
+    check(dev, variant, m, n, k, route="tiles_64")
 
 
-@pytest.mark.parametrize("m,n,k", [(1300, 1301, 129), (1700, 1001, 700), (1600, 1599, 70)])
+@pytest.mark.parametrize("m,n,k", [(1500, 1601, 129), (1700, 1301, 700), (1600, 1599, 70)])
 def test_tiles_of_128(dev, m, n, k):
-    check(dev, "padded", m, n, k)
+    check(dev, "padded", m, n, k, route="tiles_128")
 
 
 @pytest.mark.parametrize("m,n,k", [(70, 333, 4111), (200, 1001, 15001), (999, 257, 9933), (129, 40, 4609),
                                    (300, 300, 3001)])
 def test_k_slices(dev, m, n, k):
-    check(dev, "padded", m, n, k)
+    assert _lib.gemm_route(m, n, k, k, n, n, n, variant="padded")[1] > 1
+    check(dev, "padded", m, n, k, route="tiles_128" if k >= 4096 else "tiles_64")
 
 
 # decode: column blocks of 16 and slabs of 256 with a short end, K tails, slices
@@ -91,7 +99,7 @@ def test_k_slices(dev, m, n, k):
                                    (33, 259, 1025), (64, 1001, 2047), (2, 100, 20001), (1, 16, 16384 + 1)])
 @pytest.mark.parametrize("variant", ["generic", "padded"])
 def test_decode_in_place(dev, variant, m, n, k):
-    check(dev, variant, m, n, k)
+    check(dev, variant, m, n, k, route="skinny")
 
 
 @pytest.mark.parametrize("case", [
@@ -111,23 +119,54 @@ def test_addresses_pitches_and_batches(dev, case):
     dict(m=3000, n=3003, k=2047, ldc=3010), dict(m=700, n=1999, k=2100, batch=5, shared=True),
     dict(m=700, n=1999, k=2100, batch=6)])
 def test_large_products_store_c_in_place(dev, case):
-    check(dev, "padded", **case)
+    check(dev, "padded", route="persistent", **case)
 
 
 # aligned rows with K off 64, where copies for the persistent kernel pay: whole
-# and ragged tiles, D, batches; the last one below the size stays on the tiles
+# and ragged tiles, D, C at its own pitch, batches of both operands, of A or of
+# B alone (B shared without the fold: A's batches lie apart); then sizes the
+# estimate leaves on the tiles
 @pytest.mark.parametrize("case", [
-    dict(m=3000, n=3008, k=3024), dict(m=3072, n=3088, k=2832, ldc=3090), dict(m=2048, n=2064, k=4112),
-    dict(m=900, n=2000, k=2320, batch=4), dict(m=900, n=2000, k=2320, batch=4, shared=True),
-    dict(m=500, n=528, k=1040)])
+    dict(m=3000, n=3008, k=3024), dict(m=2816, n=3072, k=3088, ldc=3074), dict(m=3328, n=2560, k=2192),
+    dict(m=1574, n=2448, k=2768, batch=2), dict(m=421, n=2320, k=2128, batch=7, shared=True, gap_a=16),
+    dict(m=1546, n=672, k=2272, batch=7, shared_a=True)])
 def test_large_aligned_products_with_k_off_64(dev, case):
-    check(dev, "auto", **case)
+    check(dev, "auto", route="persistent", **case)
+
+
+@pytest.mark.parametrize("case", [
+    dict(m=3072, n=3088, k=2832, ldc=3090), dict(m=2048, n=2064, k=4112), dict(m=500, n=528, k=1040),
+    dict(m=900, n=2000, k=2320, batch=4), dict(m=900, n=2000, k=2320, batch=4, shared=True)])
+def test_aligned_products_with_k_off_64_on_tiles(dev, case):
+    check(dev, "auto", route="variant", **case)
+
+
+# N or K below 16: copies of A and B (one of them where the other is aligned),
+# a vector kernel, C copied out where N % 16; auto takes it from 3 * 2^24
+# multiply-adds on
+@pytest.mark.parametrize("case", [
+    dict(m=40000, n=8, k=200), dict(m=9000, n=15, k=500, lda=503, ldb=17, ldc=18, a_off=3, b_off=1),
+    dict(m=9000, n=15, k=512), dict(m=6000, n=11, k=300, batch=3), dict(m=6000, n=11, k=300, batch=3, shared=True),
+    dict(m=30, n=7, k=16 * 1024 + 5, batch=16), dict(m=2000, n=3000, k=15), dict(m=3000, n=2000, k=12, ldc=2003),
+    dict(m=1500, n=2001, k=9, batch=2, shared=True)])
+def test_copies_where_n_or_k_is_below_16(dev, case):
+    check(dev, "auto", route="copies", **case)
+
+
+# one thread per output: the same sizes below that, tiny aligned products
+@pytest.mark.parametrize("case", [
+    dict(m=100, n=15, k=300), dict(m=3, n=9, k=1000, batch=3, ldc=10), dict(m=77, n=130, k=13, a_off=1),
+    dict(m=64, n=64, k=64), dict(m=50, n=100, k=127)])
+def test_one_thread_per_output(dev, case):
+    check(dev, "generic", route="valu", **case)
 
 
 # few aligned tiles over a K that has no equal slices of whole 128-deep steps
 @pytest.mark.parametrize("m,n,k", [(84, 1040, 14832), (128, 512, 4112), (300, 512, 2064),
                                    (256, 2048, 8208), (66, 1600, 3088), (130, 256, 4224)])
 def test_aligned_slices_of_unequal_depth(dev, m, n, k):
+    route, ks, _ = _lib.gemm_route(m, n, k, k, n, n, n)
+    assert route in ("tiles_64", "tiles_128") and ks >= 4
     check(dev, "auto", m, n, k)
 
 
@@ -135,7 +174,7 @@ def test_a_cold_capture_runs_without_a_workspace(dev):
     """The K slices' and copies' workspaces are not needed: a stream captured
     before it has any runs the same product without them."""
     for m, n, k in ((300, 300, 3001), (16, 1001, 4095), (3000, 3001, 2050), (3000, 3008, 3024), (9, 500, 5001),
-                    (84, 1040, 14832)):
+                    (84, 1040, 14832), (4000, 15, 1000), (4000, 5000, 9)):
         say("cold capture", m, n, k)
         plan = hg.make_plan(m, n, k)
         A = torch.randint(-128, 128, (m, k), dtype=torch.int8, device=dev)

@@ -461,20 +461,20 @@ def test_decode_kernel_padded_strides(dev):
 
 PADDED_SHAPES = [(1000, 1000, 1000, 1), (1001, 999, 1003, 1), (16, 14335, 4095, 1),
                  (1, 4097, 4095, 1), (300, 500, 1000, 3), (5, 7, 9, 1),
-                 # N % 16 == 0: the product writes C and adds D itself
+                 # N % 16 == 0
                  (500, 2000, 1500, 1), (200, 512, 777, 3), (7, 4096, 1001, 1),
-                 # K % 16 == 0: A is read in place, only B is copied
+                 # K % 16 == 0: A is aligned
                  (300, 1001, 1024, 1), (16, 14335, 4096, 1), (100, 333, 512, 2),
-                 # aligned: nothing is copied
+                 # aligned
                  (256, 256, 256, 1), (64, 512, 512, 2)]
 
 
 @pytest.mark.parametrize("shape", PADDED_SHAPES)
 def test_padded_variant(dev, shape):
-    """K and N not multiples of 16: zero-padded copies of the operands that
-    need them through the MFMA or skinny kernel, then C (plus D, also in
-    place) copied out or, when N % 16 == 0, written by the product; compared
-    with the C oracle and with the VALU kernel."""
+    """K and N not multiples of 16: the operands read in place by the MFMA or
+    skinny kernels, or (tiny products here; N or K below 16 in
+    test_gpu_any_alignment.py) zero-padded copies, the product and C copied
+    out; compared with the C oracle and with the generic variant."""
     m, n, k, batch = shape
     rng = np.random.default_rng(m + n + k + batch)
     A = rng.integers(-128, 128, (batch, m, k) if batch > 1 else (m, k), dtype=np.int8)
@@ -502,7 +502,8 @@ def test_padded_variant(dev, shape):
 
 def test_padded_variant_unaligned_pointers_and_pitches(dev):
     """A at an odd address with an odd pitch, B with a pitch that is not a
-    multiple of 16, per-batch B: the copies read any layout."""
+    multiple of 16, per-batch B: any layout is read in place (the copies' own
+    test is test_copies_where_n_or_k_is_below_16)."""
     batch, m, n, k = 2, 300, 250, 777
     lda, ldb = k + 3, n + 5
     rng = np.random.default_rng(9)
@@ -523,9 +524,9 @@ def test_padded_variant_unaligned_pointers_and_pitches(dev):
 @pytest.mark.parametrize("case", ["a_offset", "b_pitch", "b_stride"])
 def test_padded_variant_copies_only_misaligned_operands(dev, case):
     """K and N multiples of 16 with one operand the vector kernels cannot read
-    (A at an odd address, B with an odd pitch or batch stride): only that
-    operand is copied and the product writes C itself, here with D in place
-    and C at a pitch that is not a multiple of 16."""
+    (A at an odd address, B with an odd pitch or batch stride): read in place,
+    here with D in place and C at a pitch that is not a multiple of 16 (too
+    small for copies)."""
     batch, m, n, k = 2, 200, 320, 512
     a_off = 1 if case == "a_offset" else 0
     ldb = n + 5 if case == "b_pitch" else n
@@ -540,7 +541,7 @@ def test_padded_variant_copies_only_misaligned_operands(dev, case):
     Abuf[a_off:a_off + A.size] = torch.from_numpy(A.reshape(-1)).to(dev)
     Bt = torch.from_numpy(Bflat).to(dev)
     C = torch.from_numpy(D.copy()).to(dev)
-    say("padded copies", case)
+    say("padded in place", case)
     _lib.gemm_raw(Abuf.data_ptr() + a_off, Bt.data_ptr(), C.data_ptr(), C.data_ptr(), m, n, k,
                   k, ldb, ldc, ldc, batch, m * k, sb, m * ldc, m * ldc, "padded", 0, None)
     _lib.sync(None)

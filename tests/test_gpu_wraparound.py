@@ -8,7 +8,7 @@ product that carries the sum across (the wrap happens where D is added), and
 a K past 131071, where the products alone leave int32 (the wrap happens in
 the MFMA accumulators, or in the K-split reduction). Each case reaches the
 kernel named beside it (variant and K split checked on the host by
-vt_gemm_check) and compares with the oracle's exact sum wrapped to int32
+vt_gemm_check, the generic variant's kernels by vt_gemm_route) and compares with the oracle's exact sum wrapped to int32
 (needs a gfx950 GPU)."""
 import numpy as np
 import pytest
@@ -39,9 +39,16 @@ def near_limits(rng, shape):
     return np.where(top, INT32_MAX - off, INT32_MIN + off).astype(np.int32)
 
 
+# (m, n) of the generic cases below -> the kernels they run (vt_gemm_route)
+GENERIC_ROUTES = {(64, 64): "tiles_64", (16, 64): "skinny", (64, 15): "valu", (16, 16): "skinny",
+                  (16, 15): "valu", (80, 48): "tiles_128"}
+
+
 def run_raw(dev, A, B, D, variant, k_split, want_split, in_place=False):
     m, k = A.shape
     n = B.shape[1]
+    if variant == "generic":
+        assert _lib.gemm_route(m, n, k, k, n, n, n, has_d=True, variant=variant)[0] == GENERIC_ROUTES[m, n]
     st = _lib.gemm_check(m, n, k, k, n, n, n, has_d=True, variant=variant, k_split=k_split)
     assert st[0] == _lib.VT_OK and st[3] == want_split, st
     At, Bt = torch.from_numpy(A).to(dev), torch.from_numpy(B).to(dev)
@@ -55,7 +62,9 @@ def run_raw(dev, A, B, D, variant, k_split, want_split, in_place=False):
 
 # (variant, k_split asked, M, N, K, K split that runs): the kernel each reaches
 D_CASES = [
-    ("generic", 0, 64, 64, 256, 0),             # generic_kernel (VALU)
+    ("generic", 0, 64, 64, 256, 0),             # gemm_mfma_kernel<64,64>, operands in place
+    ("generic", 0, 16, 64, 256, 0),             # skinny_kernel, operands in place
+    ("generic", 0, 64, 15, 256, 0),             # generic_kernel (VALU)
     ("mfma_128x128", 0, 256, 256, 512, 0),      # gemm_mfma_kernel<128,128>
     ("mfma_256x128", 0, 256, 256, 512, 0),      # gemm_mfma_kernel<256,128>
     ("mfma_256x256", 0, 2304, 2048, 1024, 0),   # gemm_dma16_kernel (72 tiles, no split)
@@ -88,7 +97,9 @@ def test_partial_sum_near_int32_limits_wraps(dev, variant, k_split, m, n, k, spl
 
 
 @pytest.mark.parametrize("variant,m,n,split", [
-    ("generic", 16, 16, 0),                 # VALU sum wraps
+    ("generic", 16, 16, 0),                 # decode kernel, operands in place; the reduction wraps
+    ("generic", 16, 15, 0),                 # VALU sum wraps
+    ("generic", 80, 48, 0),                 # 128x128 tiles in place; the reduction wraps
     ("skinny", 16, 256, 64),                # partials in range; the reduction wraps
     ("mfma_128x128", 256, 256, 16),         # K split; the reduction wraps
     ("mfma_256x256", 2304, 4096, 0)])       # gemm_dma16_kernel (144 tiles, K unsplit): the
