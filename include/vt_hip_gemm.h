@@ -263,7 +263,9 @@ int vt_gemm_select(int64_t M, int64_t N, int64_t K, int64_t batch,
  * persistent 256x256 kernels, one workgroup per CU, take 160 KiB (K % 256 == 0
  * with 16-byte C and D rows) or 128 KiB, and so does the persistent form of
  * 256x128 (160 KiB; M >= 256, N >= 128, K % 256 == 0, 16-byte C and D rows). The
- * skinny figure excludes the A slice, which depends on K and the split.
+ * skinny figure excludes the A slice, which depends on K and the split. The
+ * generic figures are those of its VALU kernel, the padded ones the padding
+ * granularity: vt_gemm_route names what such a call runs.
  */
 int vt_variant_info(int32_t variant, int32_t *tile_m, int32_t *tile_n,
                     int32_t *tile_k, int32_t *threads, int32_t *lds_bytes);

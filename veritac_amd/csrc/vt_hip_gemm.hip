@@ -278,9 +278,9 @@ struct GemmArgs {
 };
 
 // EDGE: 0 full tiles; 1 M or N not a multiple of the tile (clamped source
-// rows and columns, masked stores); 2 also K not a multiple of 128 (each load
-// checks the K tail). The K checks sit in the k loop, so a ragged M or N
-// alone does not pay for them; 3 any M, any N and K of at least 16, operands at
+// rows and columns, masked stores); 2 also K not a multiple of 128 (the last
+// slice's loads move back inside the row, and A past K is zeroed on the way to
+// LDS: checks in the k loop that a ragged M or N alone does not pay for); 3 any M, any N and K of at least 16, operands at
 // any address and pitch (16-byte loads need no alignment): a row's last bytes
 // are read from its last 16, moved into place, and zero past it.
 //
@@ -2308,7 +2308,7 @@ const VariantInfo kVariants[VT_VARIANT_COUNT] = {
     {"skinny", 16, 256, 64, 1024, 2 * 16 * 1024},
     {"generic", 4, 64, 1, 256, 0},
     {"mfma_256x128", 256, 128, 64, 256, 3 * (256 * 64 + 64 * 128)},
-    {"padded", 16, 16, 16, 256, 0},   // padding granularity; the inner kernel decides the rest
+    {"padded", 16, 16, 16, 256, 0},   // padding granularity; vt_gemm_route names the kernels
 };
 
 // Default skinny configuration: 256-column slabs (full 128-byte lines of B
@@ -3185,8 +3185,8 @@ int launch_skinny(const Problem &q, int k_split, Scratch &scr) {
 }
 
 // Packed-B decode configuration: 4 column blocks (64 columns) per workgroup,
-// 8 waves, 2 row blocks of loads ahead. For N = 14336 that is 224 workgroups
-// streaming 256 KiB each.
+// 8 waves, 2 to 4 row blocks of loads ahead (packed_stages). For N = 14336 that
+// is 224 workgroups streaming 256 KiB each.
 constexpr int kPackedNBW = 4, kPackedWaves = 8;
 
 int64_t packed_kbt(int64_t K) { return (K + 63) / 64; }
@@ -3780,11 +3780,14 @@ void direct_slices(const Problem &r, int ks, DirectPlan *d) {
 // busy), the copies at 4.5 TB/s and their launch, and the last round's C at 5
 // TB/s, against the 128x128 tiles that read the operands in place, a slice of
 // which takes 0.2 us and 0.56 more per tile and CU (0.15 and 0.29 per whole
-// tile with aligned rows). HIP graph per call, in place against copies:
-// 3000 x 3001 x 3003 75 and 50 us; 4000 x 4001 x 4001 140 and 81; 8000 x 8001 x
-// 2001 280 and 161; 5857 x 2373 x 1435 63 and 46; aligned 3000 x 3008 x 3024 57
-// and 47, 8000 x 8000 x 2000 164 and 145, 8192 x 8192 x 8208 526 and 466, but
-// 2000 x 4096 x 2064 28 and 41, 4114 x 16208 x 880 + D 198 and 210.
+// tile with aligned rows). In place (captured before the stream has a
+// workspace) against copies, in us: 3000 x 3001 x 3003 75 and 50; 4000 x 4001 x
+// 4001 130 and 78; 8000 x 8001 x 2001 273 and 155; 5857 x 2373 x 1435 63 and
+// 46. Aligned, on the tiles (as captured calls stay) against copies (calls in a
+// row): 3000 x 3008 x 3024 53 and 46, 8000 x 8000 x 2000 163 and 142, 8192 x
+// 8192 x 8208 526 and 454; where the tiles are kept, copies took longer when
+// the rule was made: 2000 x 4096 x 2064 28 and 41, 4114 x 16208 x 880 + D 198
+// and 210.
 struct LargeLayout {
   int64_t Kp, Np, a_bytes, b_bytes;
   bool copy_a, copy_b;
@@ -3851,12 +3854,15 @@ int launch_large_padded(const Problem &r, const LargeLayout &L, int8_t *w, hipSt
 // How a problem the vector kernels cannot read as it is runs without copies:
 // decode shapes on the skinny kernel, the rest on 64x64 tiles up to two a CU,
 // else 128x128 tiles; few tiles over a long K (4096, 128x128) or one that
-// saves 20 slices split it as the aligned tiles do. HIP graph per call, before
-// (copies, or the VALU kernel below 3 * 2^24 multiply-adds) and now: 100 x 203
-// x 333 8.3 -> 4.5 us, 1000 x 1001 x 999 + D 19.4 -> 8.7, 2000 x 2001 x 2003 43
-// -> 23, 5857 x 1373 x 435 39 -> 26, 999 x 257 x 9933 100 -> 17.5, 200 x 1001 x
-// 15001 142 -> 20, 16 x 14335 x 4095 43.5 -> 18, 48 x 4095 x 14337 54 -> 26, 8 x
-// 100 x 5001 105 -> 4.7. 64x64 against 128x128: 2487 x 344 x 899 (234 tiles of
+// saves 20 slices split it as the aligned tiles do. Calls in a row, over
+// copies or on the VALU kernel (below 3 * 2^24 multiply-adds) and this way:
+// 1000 x 1001 x 999 + D 18.8 -> 8.0 us, 2000 x 2001 x 2003 41.7 -> 21.9, 5857 x
+// 1373 x 435 36.6 -> 23.6, 999 x 257 x 9933 99 -> 16.7, 200 x 1001 x 15001 142
+// -> 18.5, 16 x 14335 x 4095 38.9 -> 16.6, 48 x 4095 x 14337 48.1 -> 22.9, 8 x
+// 100 x 5001 80 -> 7.3; HIP graph per call 100 x 203 x 333 8.4 -> 4.5. Without
+// a workspace (captured on a stream that has none; the generic variant always
+// when captured) nothing is split: 999 x 257 x 9933 68, 200 x 1001 x 15001 100,
+// 16 x 14335 x 4095 19.6, 48 x 4095 x 14337 60, 8 x 100 x 5001 20.6. 64x64 against 128x128: 2487 x 344 x 899 (234 tiles of
 // 64x64) 8.8 and 12.0; 2000 x 2001 x 2003 (1024) 35 and 24.
 DirectPlan direct_plan(const Problem &q) {
   DirectPlan d;
@@ -3953,9 +3959,9 @@ Route any_route(const Problem &q, int64_t limit) {
 // where they are the faster way (`copies`: the call may take them). Few tiles
 // over a long K that does not divide into the MFMA split's equal slices of
 // whole 128-deep steps: slices of whole 64-deep ones, the last one shorter.
-// Calls in a row, unsplit against sliced: 84 x 1040 x 14832 69 and 14 us, 128 x
-// 512 x 4112 32 and 11, 200 x 1008 x 15008 128 and 16, 512 x 4096 x 9008 78 and
-// 34 (the first with the K tail's loads in flight, the others before).
+// Unsplit (HIP graph per call; captured calls stay that way) against sliced
+// (calls in a row), in us: 84 x 1040 x 14832 68 and 13, 128 x 512 x 4112 21 and
+// 11, 200 x 1008 x 15008 73 and 17, 512 x 4096 x 9008 45 and 33.
 Route vector_route(const Problem &q, int32_t variant, int64_t limit, bool copies) {
   const Problem r = mfma_fold(q);
   LargeLayout L;
