@@ -379,7 +379,8 @@ def test_persistent_multi_tile_walks(dev, shape):
 # K of at most 128: one pair of k steps, the SHORT instantiation (both slices
 # fetched in one round trip), on edge and whole tiles, with and without D
 SHORT_K_SHAPES = [(64, 64, 64), (128, 128, 128), (200, 304, 16), (256, 256, 80),
-                  (384, 512, 128), (130, 144, 48), (512, 256, 64)]
+                  (384, 512, 128), (130, 144, 48), (512, 256, 64),
+                  (413, 192, 32), (90, 48, 112), (65, 208, 96)]
 
 
 @pytest.mark.parametrize("variant", ["mfma_128x128", "mfma_256x128", "mfma_256x256"])

@@ -280,7 +280,7 @@ struct GemmArgs {
 // EDGE: 0 full tiles; 1 M or N not a multiple of the tile (clamped source
 // rows and columns, masked stores); 2 also K not a multiple of 128 (the last
 // slice's loads move back inside the row, and A past K is zeroed on the way to
-// LDS: checks in the k loop that a ragged M or N alone does not pay for); 3 any M, any N and K of at least 16, operands at
+// LDS, or at the load with SHORT: checks in the k loop that a ragged M or N alone does not pay for); 3 any M, any N and K of at least 16, operands at
 // any address and pitch (16-byte loads need no alignment): a row's last bytes
 // are read from its last 16, moved into place, and zero past it.
 //
@@ -392,7 +392,11 @@ __global__ __launch_bounds__(256, 1) void gemm_mfma_kernel(GemmArgs p) {
   // they are never computed. No load has a branch around it and no loaded
   // value is used before store_slice, two steps later: the K tail's check at
   // the load made the compiler wait for it there (64x64 tiles, 1000 x 1008 x
-  // 1008 + D: 9.5 -> 7.3 us).
+  // 1008 + D: 9.5 -> 7.3 us). SHORT waits for all of its loads at once, and
+  // checks at the load: lanes of A past K load nothing and all rows of B past K
+  // are one (HIP graph per call, this way and the other: 413 x 192 x 32 2.76 and
+  // 2.91 us, 256 x 256 x 96 + D 3.27 and 3.40, 574 x 3392 x 64 3.85 and 4.01).
+  constexpr bool CHECK_LOADS = EDGE == 2 && SHORT;
   auto load_slice = [&](int kt, v4i *ra, v4i *rb) {
     const int k0 = min(kt, KT - 1) * BK;
     const int8_t *abase = Ab + k0 - LEFT;
@@ -401,19 +405,25 @@ __global__ __launch_bounds__(256, 1) void gemm_mfma_kernel(GemmArgs p) {
 #pragma unroll
     for (int i = 0; i < CA; ++i) {
       if constexpr (EDGE == 3) ra[i] = ld_any(abase + (tail ? a_tail[i] : a_goff[i]));
-      else if constexpr (EDGE == 2) ra[i] = *(const v4i *)(abase + (tail ? a_tail[i] : a_goff[i]));
+      else if constexpr (CHECK_LOADS) {
+        ra[i] = v4i{0, 0, 0, 0};
+        if (kt * BK + a_k[i] < K) ra[i] = *(const v4i *)(abase + a_goff[i]);
+      } else if constexpr (EDGE == 2) ra[i] = *(const v4i *)(abase + (tail ? a_tail[i] : a_goff[i]));
       else ra[i] = *(const v4i *)(abase + a_goff[i]);
     }
 #pragma unroll
     for (int i = 0; i < CB; ++i) {
       if constexpr (EDGE == 3) rb[i] = ld_any(bbase + (tail ? b_tail[i] : b_goff[i]));
-      else if constexpr (EDGE == 2) rb[i] = *(const v4i *)(bbase + (tail ? b_tail[i] : b_goff[i]));
+      else if constexpr (CHECK_LOADS && !PACKED_B) {
+        const int row = tid / BCH + (256 / BCH) * i;
+        rb[i] = *(const v4i *)(Bb + (int64_t)(min(kt * BK + row, K - 1) - row) * p.ldb + b_goff[i]);
+      } else if constexpr (EDGE == 2) rb[i] = *(const v4i *)(bbase + (tail ? b_tail[i] : b_goff[i]));
       else rb[i] = *(const v4i *)(bbase + b_goff[i]);
     }
   };
   // Slice kt's registers -> LDS buffer buf.
   auto store_slice = [&](int buf, int kt, v4i *ra, v4i *rb) {
-    if (EDGE >= 2 && (kt + 1) * BK > K) {
+    if (EDGE >= 2 && !CHECK_LOADS && (kt + 1) * BK > K) {
 #pragma unroll
       for (int i = 0; i < CA; ++i) {
         const int past = kt * BK + a_k[i] - (K - 16);   // bytes of the chunk past K
@@ -517,8 +527,7 @@ __global__ __launch_bounds__(256, 1) void gemm_mfma_kernel(GemmArgs p) {
   // SHORT (K <= 128, one pair of steps; the host picks it): slices 0 and 1
   // are both in flight before the first wait and nothing more is fetched,
   // so the k loop costs one global round trip instead of three. Longer K
-  // keeps the general schedule below (the slices it fetches past the end
-  // re-read the last one and are never computed).
+  // keeps the general schedule below.
   v4i ra0[CA], rb0[CB], ra1[CA], rb1[CB];
   if constexpr (SHORT) {
     load_slice(0, ra0, rb0);
