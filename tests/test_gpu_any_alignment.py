@@ -122,6 +122,16 @@ def test_large_products_store_c_in_place(dev, case):
     check(dev, "padded", route="persistent", **case)
 
 
+# the same with K below the kernel's 256 (zeros from K on): C off 64-byte rows
+# and large enough that storing it is what takes the time
+@pytest.mark.parametrize("case", [
+    dict(m=3400, n=3401, k=17), dict(m=3300, n=3313, k=130), dict(m=257, n=43009, k=48),
+    dict(m=40001, n=300, k=64), dict(m=3072, n=3585, k=255), dict(m=700, n=2001, k=90, batch=10),
+    dict(m=700, n=2001, k=90, batch=10, shared=True), dict(m=3500, n=3392, k=100, ldc=3401)])
+def test_large_products_of_a_short_k(dev, case):
+    check(dev, "padded", route="persistent", **case)
+
+
 # aligned rows with K off 64, where copies for the persistent kernel pay: whole
 # and ragged tiles, D, C at its own pitch, batches of both operands, of A or of
 # B alone (B shared without the fold: A's batches lie apart); then sizes the

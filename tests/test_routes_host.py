@@ -68,6 +68,12 @@ def test_the_plan_mirror_names_the_library_s_routes(variant):
     ((1700, 1001, 700), {}, ("tiles_64", 1)),
     ((2000, 2001, 2003), {}, ("tiles_128", 1)),
     ((3000, 3001, 3003), {}, ("persistent", 1)),
+    # short K: by C's bytes, and only where its rows are off 64 bytes
+    ((12675, 8829, 87), {}, ("persistent", 1)),
+    ((3436, 11135, 178), {}, ("persistent", 1)),
+    ((11661, 6839, 26), {}, ("persistent", 1)),
+    ((3325, 1267, 66), {}, ("tiles_128", 1)),
+    ((8558, 4560, 327), {}, ("tiles_128", 1)),
     ((40000, 8, 200), {}, ("copies", 1)),
     ((4000, 5000, 9), {}, ("copies", 1)),
     ((16, 15, 139264), dict(variant="generic"), ("valu", 1)),

@@ -242,10 +242,11 @@ def test_launched_workgroups_are_the_reported_ones(run, variant):
 out = []
 for m, n, k, batch, shared, v, ks in %r:
     fake.fake_reset()
+    STREAM += 1        # a stream with all of its workspaces' bounds left
     if v == "skinny_packed":
-        packed(m, n, k, batch)
+        packed(m, n, k, batch, stream=STREAM)
     else:
-        gemm(m, n, k, v, batch=batch, shared=shared)
+        gemm(m, n, k, v, batch=batch, shared=shared, stream=STREAM)
     out.append([e[3] for e in launches()])
 print(json.dumps(out))
 """ % (calls,))

@@ -68,6 +68,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <string>
@@ -3796,14 +3797,18 @@ void direct_slices(const Problem &r, int ks, DirectPlan *d) {
 // row): 3000 x 3008 x 3024 53 and 46, 8000 x 8000 x 2000 163 and 142, 8192 x
 // 8192 x 8208 526 and 454; where the tiles are kept, copies took longer when
 // the rule was made: 2000 x 4096 x 2064 28 and 41, 4114 x 16208 x 880 + D 198
-// and 210.
+// and 210. Rows of C off 64 bytes bound a short K: the tiles store 4 bytes a
+// lane at 1.3 TB/s, the persistent kernel 16 bytes of whole rows at 3 TB/s
+// (1.2 and 2 with D to read) after its copies. Calls in a row, in place against
+// copies: 12675 x 8829 x 87 357 and 152, 3436 x 11135 x 178 124 and 67, 1246 x
+// 12947 x 133 + D 53 and 32, but 3325 x 1267 x 66 8.5 and 19.5.
 struct LargeLayout {
   int64_t Kp, Np, a_bytes, b_bytes;
   bool copy_a, copy_b;
 };
 
 bool large_padded(const Problem &r, bool aligned, LargeLayout *L) {
-  if (r.M < 256 || r.N < 256 || r.K < 256 || r.ldc >= (1ll << 29) || (r.D && r.ldd >= (1ll << 29)) ||
+  if (r.M < 256 || r.N < 256 || r.K < (aligned ? 256 : 16) || r.ldc >= (1ll << 29) || (r.D && r.ldd >= (1ll << 29)) ||
       r.batch > 65535)
     return false;
   auto round256 = [](int64_t v) { return (v + 255) / 256 * 256; };
@@ -3820,15 +3825,20 @@ bool large_padded(const Problem &r, bool aligned, LargeLayout *L) {
   const double busy = (double)(tiles < kSplitCus ? tiles : kSplitCus) / kSplitCus;
   const double rounds = (double)((tiles + kSplitCus - 1) / kSplitCus);
   const double slice = 575.0 + (busy > 0.5 ? 530.0 * (busy - 0.5) : 0.0);
-  const double padded = rounds * (double)(L->Kp / 64) * slice +
+  double padded = rounds * (double)(L->Kp / 64) * slice +
                         2.0 * (double)(L->a_bytes + L->b_bytes) / 4500.0 + 6000.0 +
                         4.0 * (double)r.M * (double)r.N * (double)r.batch / 5000.0 / rounds;
   const int64_t t128 = (r.M + 127) / 128 * ((r.N + 127) / 128) * r.batch;
   const double per_cu = (double)t128 / kSplitCus;
-  const double direct =
+  double direct =
       4000.0 + (double)((r.K + 63) / 64) *
                    (aligned ? 150.0 + 290.0 * (double)((t128 + kSplitCus - 1) / kSplitCus)
                             : 200.0 + 560.0 * (per_cu < 0.4 ? 0.4 : per_cu));
+  if (!aligned && r.ldc % 16) {
+    const double c = 4.0 * (double)r.M * (double)r.N * (double)r.batch;
+    padded = std::max(padded, 14000.0 + c / (r.D ? 2000.0 : 3000.0));
+    direct = std::max(direct, c / (r.D ? 1200.0 : 1300.0));
+  }
   return padded < direct;
 }
 

@@ -262,11 +262,11 @@ OPTIONAL_BYTES = 256 << 20    # kOptionalBytes in the HIP source
 ROUTE_TILES = {"tiles_64": 64, "tiles_128": 128, "persistent": 256}
 
 
-def _large_padded(m, n, k, b, b_mats, aligned):
+def _large_padded(m, n, k, b, b_mats, has_d, aligned):
     """(padded n, padded k, bytes of the copies) of a folded problem that runs
     on the persistent kernel over padded copies, else None (large_padded in
     the HIP source, contiguous operands)."""
-    if min(m, n, k) < 256 or n >= 2**29 or b > 65535:
+    if min(m, n) < 256 or k < (256 if aligned else 16) or n >= 2**29 or b > 65535:
         return None
     k_p, n_p = -(-k // 256) * 256, -(-n // 16) * 16
     a_bytes = -(-b * m * k_p // 256) * 256 if k_p != k else 0
@@ -283,6 +283,10 @@ def _large_padded(m, n, k, b, b_mats, aligned):
     t128 = -(-m // 128) * -(-n // 128) * b
     direct = 4000.0 + -(-k // 64) * (150.0 + 290.0 * -(-t128 // NUM_CUS) if aligned
                                      else 200.0 + 560.0 * max(t128 / NUM_CUS, 0.4))
+    if not aligned and n % 16:
+        c = 4.0 * m * n * b
+        padded = max(padded, 14000.0 + c / (2000.0 if has_d else 3000.0))
+        direct = max(direct, c / (1200.0 if has_d else 1300.0))
     return (n_p, k_p, a_bytes + b_bytes) if padded < direct else None
 
 
@@ -334,13 +338,13 @@ def gemm_route(plan, limit=2**63 - 1):
         if route is None:
             return own
         if route[0] != "skinny" and route[1] == 1:
-            large = _large_padded(fm, n, k, fb, b_mats, False)
+            large = _large_padded(fm, n, k, fb, b_mats, plan["has_d"], False)
             if large is not None and large[2] <= limit:
                 return "persistent", 1, large[2]
         return _direct_route(plan, limit)
     if variant.startswith("mfma"):
         if k % 64:
-            large = _large_padded(fm, n, k, fb, b_mats, True)
+            large = _large_padded(fm, n, k, fb, b_mats, plan["has_d"], True)
             if large is not None and large[2] <= limit:
                 return "persistent", 1, large[2]
         if (variant == "mfma_128x128" and k >= 1024 and fb == 1
