@@ -504,6 +504,17 @@ def test_memory_bounds_are_counted_at_run_time():
     assert any("counted" in n for n in info["notes"])
 
 
+@pytest.mark.parametrize("m,n,k,tiled", [
+    (64, 64, 33, True), (64, 63, 33, False), (64, 64, 32, False), (100, 90, 32, False), (100, 90, 40, True),
+    (1000, 1000, 2, False), (1000, 1000, 12, False), (1000, 1000, 13, True), (1000, 1000, 32, True),
+    (500, 500, 500, True)])
+def test_short_sums_keep_one_thread_per_cell(m, n, k, tiled):
+    """Up to 32 steps the compiler unrolls the one-thread-per-cell loop, which
+    LDS tiles only beat on large nests."""
+    decl = {b: {"dtype": "float32", "shape": s} for b, s in zip("ABC", ((m, k), (k, n), (m, n)))}
+    assert ("vt_tile" in ln.emit_kernel(ln.matmul_stmt(m, k, n), decl)["source"]) == tiled
+
+
 def test_tiled_nests_report_and_bound_what_their_threads_run():
     """A nest on LDS tiles runs whole workgroups, each thread the steps of
     several cells: the reported threads are those launched, a thread's steps of
