@@ -290,7 +290,7 @@ def _large_padded(m, n, k, b, b_mats, has_d, aligned):
     return (n_p, k_p, a_bytes + b_bytes) if padded < direct else None
 
 
-def _direct_route(plan, limit):
+def _direct_route(plan):
     """(route, K slices, workspace bytes) of a problem read in place, or None
     (direct_plan in the HIP source, contiguous operands)."""
     m, n, k, batch = plan["m"], plan["n"], plan["k"], plan["batch"]
@@ -304,8 +304,7 @@ def _direct_route(plan, limit):
     t64, t128 = (-(-fm // t) * -(-n // t) * fb for t in (64, 128))
     if m <= 16 or (m <= SKINNY_MAX_M and k >= 1024 and -(-n // 128) * batch < NUM_CUS):
         ks = skinny_split(dict(plan, k_split=0))[0]
-        scratch = batch * ks * m * pitch * 4 if ks > 1 else 0
-        return ("skinny", ks, scratch) if scratch <= limit else ("tiles_64", 1, 0)
+        return "skinny", ks, batch * ks * m * pitch * 4 if ks > 1 else 0
     long_k = k >= 4096 and fb == 1
     route = "tiles_128" if long_k or t64 > 512 else "tiles_64"
     tiles, ks = t128 if route == "tiles_128" else t64, 1
@@ -318,8 +317,7 @@ def _direct_route(plan, limit):
     ks = -(-k // kc)
     if ks > 1 and k - (ks - 1) * kc < 16:
         ks -= 1
-    scratch = ks * fm * pitch * 4 if ks > 1 else 0
-    return (route, ks, scratch) if scratch <= limit else (route, 1, 0)
+    return route, ks, ks * fm * pitch * 4 if ks > 1 else 0
 
 
 def gemm_route(plan, limit=2**63 - 1):
@@ -334,14 +332,16 @@ def gemm_route(plan, limit=2**63 - 1):
     b_mats = 1 if fb == 1 or plan["b_shared"] else fb
     if variant in ("generic", "padded"):
         own = ("valu" if variant == "generic" else "copies", 1, 0)
-        route = _direct_route(plan, 2**63 - 1)
+        route = _direct_route(plan)
         if route is None:
             return own
         if route[0] != "skinny" and route[1] == 1:
             large = _large_padded(fm, n, k, fb, b_mats, plan["has_d"], False)
             if large is not None and large[2] <= limit:
                 return "persistent", 1, large[2]
-        return _direct_route(plan, limit)
+        if route[2] <= limit:
+            return route
+        return "tiles_64" if route[0] == "skinny" else route[0], 1, 0
     if variant.startswith("mfma"):
         if k % 64:
             large = _large_padded(fm, n, k, fb, b_mats, plan["has_d"], True)
@@ -349,7 +349,7 @@ def gemm_route(plan, limit=2**63 - 1):
                 return "persistent", 1, large[2]
         if (variant == "mfma_128x128" and k >= 1024 and fb == 1
                 and mfma_k_split(dict(plan, routed=True)) == 1):
-            route = _direct_route(dict(plan, m=fm, batch=1), 2**63 - 1)
+            route = _direct_route(dict(plan, m=fm, batch=1))
             if (route is not None and route[0] != "skinny" and route[2] <= limit
                     and (route[1] >= 4 or (route[1] >= 2 and k >= 8192))):
                 return route
@@ -361,7 +361,9 @@ def launched_plan(plan):
     workspaces (outside capture): the plan itself, or one with `routed` set and
     the tiles (`tile`), K slices (`slices`), operands read in place
     (`in_place`) or bytes of padded copies (`copied`) of its route."""
-    if plan.get("routed") or plan.get("packed_b") or plan["variant"] == PACKED_VARIANT:
+    variant = plan["variant"]
+    if (plan.get("routed") or plan.get("packed_b") or variant in ("skinny", PACKED_VARIANT)
+            or (plan["k"] % 64 == 0 and variant in ("mfma_256x256", "mfma_256x128"))):
         return plan
     route, ks, scratch = gemm_route(plan)
     if route == "skinny":
@@ -691,7 +693,8 @@ def make_plan(m, n, k, *, batch=1, b_shared=False, has_d=False, d_max_abs=0,
             "b_shared": bool(b_shared), "has_d": bool(has_d), "d_max_abs": d_max_abs,
             "variant": variant, "k_split": k_split}
     if variant == "auto":
-        ok, reason = validate_plan(dict(plan, variant="generic"))
+        # sizes and bounds only: any variant's kernels will do
+        ok, reason = validate_plan(dict(plan, variant="generic", routed=True))
         if not ok:
             raise HipGemmError("cannot plan: " + reason)
         vec = n % DIM == 0 and k % DIM == 0
